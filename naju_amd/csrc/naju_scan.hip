@@ -2787,14 +2787,14 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
       if ((int64_t)l.n_tiles * l.nseg > 0x7fffffff) return fail(NAJU_ERR_UNSUPPORTED, "problem too large");
       hipError_t e = hipSuccess;
       if (l.nseg > 1) {
-        e = mc_fwd_launch(a, true, x_dtype, gate_dtype, y_dt, st);
+        e = mc_map_launch(a, false, x_dtype, gate_dtype, st);
         if (e == hipSuccess) {
           const int64_t n = (int64_t)a.batch * a.D * a.N;
           hipLaunchKernelGGL(gn_seg_carry_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, 1);
           e = hipGetLastError();
         }
       }
-      if (e == hipSuccess) e = mc_fwd_launch(a, false, x_dtype, gate_dtype, y_dt, st);
+      if (e == hipSuccess) e = mc_fwd_launch(a, x_dtype, gate_dtype, y_dt, st);
       if (e != hipSuccess) return fail(NAJU_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
       return NAJU_OK;
     }
@@ -3059,24 +3059,24 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
         r.ckpt = (float*)(ws + l.off_dense);
         r.Kc = (int)((T + kMcQ - 1) / kMcQ);
         r.seg_sc = ck_rows / kMcQ;
-        r.nseg = r.Kc_src + 1;  // the map launch runs segments 0 .. nseg - 2
+        r.nseg = r.Kc_src;
         r.n_dtiles = (int)((D + kMcDT - 1) / kMcDT);
         r.n_tiles = (int)(batch * r.n_dtiles);
         if ((int64_t)r.n_tiles * r.Kc_src > 0x7fffffff) return fail(NAJU_ERR_UNSUPPORTED, "problem too large");
-        e = mc_fwd_launch(r, true, x_dtype, gate_dtype, x_dtype, st);
+        e = mc_fwd_launch(r, x_dtype, gate_dtype, x_dtype, st);
         a.ckpt = r.ckpt;
       }
       a.ck_rows = kMcQ;
       a.Kc = (int)((T + kMcQ - 1) / kMcQ);
       if (e == hipSuccess && l.nseg > 1) {
-        e = mc_bwd_launch(a, true, x_dtype, gate_dtype, du_dt, dg_dt, st);
+        e = mc_map_launch(a, true, x_dtype, gate_dtype, st);
         if (e == hipSuccess) {
           const int64_t n = (int64_t)a.batch * a.D * a.N;
           hipLaunchKernelGGL(gn_seg_carry_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, -1);
           e = hipGetLastError();
         }
       }
-      if (e == hipSuccess) e = mc_bwd_launch(a, false, x_dtype, gate_dtype, du_dt, dg_dt, st);
+      if (e == hipSuccess) e = mc_bwd_launch(a, x_dtype, gate_dtype, du_dt, dg_dt, st);
       if (e != hipSuccess) return fail(NAJU_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
       goto fold;
     }

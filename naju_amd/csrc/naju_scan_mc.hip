@@ -28,103 +28,12 @@
 // value s: the state chain needs no data movement between lanes.
 #include <hip/hip_runtime.h>
 
+#include "mc_ops.h"
 #include "naju_scan.h"
 #include "scan_internal.h"
 
 namespace naju_detail {
 namespace {
-
-typedef float f4_t __attribute__((ext_vector_type(4)));
-
-// D += A B for one 16x16x4 float32 tile: lane l supplies A[l%16][l/16] and
-// B[l/16][l%16] and holds D[4(l/16) + r][l%16] in value r.
-__device__ __forceinline__ f4_t mma(float a, float b, f4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// Four values that are exact in the 2-byte stream type TT (B and C as
-// staged: converted from TT, zero rows included) packed as TT pairs.
-template <typename TT>
-__device__ __forceinline__ void pack4(const float (&x)[4], uint32_t (&w)[2]) {
-  if constexpr (__is_same(TT, bf16_t)) {
-    // the upper halves of the float bits (exact: the low halves are zero)
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      w[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, x[2 * k + 1]), __builtin_bit_cast(uint32_t, x[2 * k]),
-                                   0x07060302u);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-      const h2 h = {(_Float16)x[2 * k], (_Float16)x[2 * k + 1]};
-      w[k] = __builtin_bit_cast(uint32_t, h);
-    }
-  }
-}
-
-// D += A B with K = 32 on the 16-bit matrix-core path, for operands exact in
-// TT (bf16 or f16): lane l supplies A[l%16][k] and B[k][l%16] for its eight
-// k of the product, a0 and b0 (then a1 and b1) packed by pack4 from the same
-// four k each, so that any assignment of the lane's values to k pairs A and
-// B alike. The products are exact in float32 and only the accumulation
-// rounds, as on the float32 path, at one instruction in place of eight.
-template <typename TT>
-__device__ __forceinline__ f4_t mma_k32(const uint32_t (&a0)[2], const uint32_t (&a1)[2], const uint32_t (&b0)[2],
-                                        const uint32_t (&b1)[2], f4_t c) {
-  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-  const u4 av = {a0[0], a0[1], a1[0], a1[1]}, bv = {b0[0], b0[1], b1[0], b1[1]};
-  if constexpr (__is_same(TT, bf16_t)) {
-    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, av), __builtin_bit_cast(v8, bv), c, 0, 0,
-                                                   0);
-  } else {
-    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, av), __builtin_bit_cast(v8, bv), c, 0, 0, 0);
-  }
-}
-
-// x[k] = hi + mid + lo exactly, in three bf16 parts packed in pairs like
-// pack4: hi keeps the top 8 significant bits of x (truncated), mid the next
-// 8 of the remainder and lo the at most 8 left, so each part is exact in
-// bf16 and each difference exact in float32. (x = +-inf or nan gives nan
-// parts; the states and adjoints split here are finite for finite inputs.)
-__device__ __forceinline__ void split4_bf16(const float (&x)[4], uint32_t (&h)[2], uint32_t (&md)[2],
-                                            uint32_t (&lo)[2]) {
-  uint32_t hb[4], mb[4], lb[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    // x as rounded: the subtraction below must not be fused with the
-    // product that formed x (the parts would then sum to the unrounded
-    // product, differently wherever the compiler chose to fuse)
-    float xk = x[k];
-    asm volatile("" : "+v"(xk));
-    hb[k] = __builtin_bit_cast(uint32_t, xk) & 0xffff0000u;
-    const float r = xk - __builtin_bit_cast(float, hb[k]);
-    mb[k] = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
-    lb[k] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, mb[k]));
-  }
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    h[k] = __builtin_amdgcn_perm(hb[2 * k + 1], hb[2 * k], 0x07060302u);
-    md[k] = __builtin_amdgcn_perm(mb[2 * k + 1], mb[2 * k], 0x07060302u);
-    lo[k] = __builtin_amdgcn_perm(lb[2 * k + 1], lb[2 * k], 0x07060302u);
-  }
-}
-
-// D += A B over the lane's four k (the k-steps of four 16x16x4 float32
-// products) with A exact in bf16 (a: packed by pack4) and B float32 given by
-// its split4_bf16 parts: hi and mid in one K = 32 product, lo (with zeros)
-// in a second. Each product is exact; the result matches the float32 path
-// up to the accumulation's rounding, at two instructions in place of four.
-// (The K = 16 form, v_mfma_f32_16x16x16_bf16, took the lo part at first and
-// gave run-to-run different results in this position on gfx950 with the
-// compiler's default scheduling; the K = 32 form is used throughout.)
-__device__ __forceinline__ f4_t mma_x3(const uint32_t (&a)[2], const uint32_t (&h)[2], const uint32_t (&md)[2],
-                                       const uint32_t (&lo)[2], f4_t c) {
-  c = mma_k32<bf16_t>(a, a, h, md, c);
-  const uint32_t z[2] = {0u, 0u};
-  return mma_k32<bf16_t>(a, z, lo, z, c);
-}
 
 constexpr int Q = kMcQ;    // rows per sub-block
 constexpr int TP = Q + 4;  // pitch of the per-wave [channel][row] tiles
@@ -221,11 +130,11 @@ __device__ __forceinline__ void ld4r_at(const TT* __restrict__ p, const uint32_t
 //   Bt [n][p(t)]  (B transposed, time rows permuted p(4s + g) = 4g + s, so
 //                  the four rows 4s + g (s = 0..3) a lane feeds to the state
 //                  update are one 16-byte read).
-template <int NP, bool MAP>
+template <int NP, bool RECOMP>
 struct McBC {
   static constexpr int P = NP + 4;
-  float Bn[2][MAP ? 1 : kMcQ][MAP ? 4 : P];
-  float C[2][MAP ? 1 : kMcQ][MAP ? 4 : P];
+  float Bn[2][RECOMP ? 1 : kMcQ][RECOMP ? 4 : P];
+  float C[2][RECOMP ? 1 : kMcQ][RECOMP ? 4 : P];
   float Bt[2][NP][TP];
 };
 
@@ -234,7 +143,7 @@ struct McBC {
 // become the neutral step when the gates are formed), and the workgroup's B
 // (and C) groups of four entries: thread tid < 4 NP takes row (4 tid) / NP,
 // entries n0 .. n0+3 with n0 = (4 tid) % NP.
-template <int NP, bool MAP, typename TU, typename TG, typename TB>
+template <int NP, bool RECOMP, typename TU, typename TG, typename TB>
 struct McIn {
   Raw4<TG> f, i;
   Raw4<TU> u;
@@ -269,13 +178,13 @@ struct McIn {
       const uint32_t ro = (uint32_t)((row < rows ? row : rows - 1) * a.ldbc);
       if (N == NP) {
         ld4r<TB>((const TB*)a.Bm + bb, ro + n0, b);
-        if constexpr (!MAP) ld4r<TB>((const TB*)a.Cm + bb, ro + n0, c);
+        if constexpr (!RECOMP) ld4r<TB>((const TB*)a.Cm + bb, ro + n0, c);
       } else {
         uint32_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = ro + (uint32_t)(n0 + e < N ? n0 + e : N - 1);
         ld4r_at<TB>((const TB*)a.Bm + bb, o, b);
-        if constexpr (!MAP) ld4r_at<TB>((const TB*)a.Cm + bb, o, c);
+        if constexpr (!RECOMP) ld4r_at<TB>((const TB*)a.Cm + bb, o, c);
       }
     }
   }
@@ -297,7 +206,7 @@ struct McIn {
   // B (and C) into LDS buffer buf; zeros past T and past N. (Each 16 lanes
   // read one 64-entry row of B and C, coalesced; the backward's staging takes
   // another lane map, which the forward measured slower with.)
-  __device__ __forceinline__ void stage(McBC<NP, MAP>& sh, int buf, const ScanArgs& a, int64_t t0, int tid) const {
+  __device__ __forceinline__ void stage(McBC<NP, RECOMP>& sh, int buf, const ScanArgs& a, int64_t t0, int tid) const {
     if (tid < 4 * NP) {
       const int row = (4 * tid) / NP, n0 = (4 * tid) % NP;
       const bool rok = t0 + row < a.T;
@@ -306,10 +215,10 @@ struct McIn {
       for (int e = 0; e < 4; ++e) {
         const bool ok = rok && n0 + e < a.N;
         vb[e] = ok ? b.get(e) : 0.f;
-        if constexpr (!MAP) vc[e] = ok ? c.get(e) : 0.f;
+        if constexpr (!RECOMP) vc[e] = ok ? c.get(e) : 0.f;
         sh.Bt[buf][n0 + e][4 * (row & 3) + (row >> 2)] = vb[e];
       }
-      if constexpr (!MAP) {
+      if constexpr (!RECOMP) {
         *(float4*)&sh.Bn[buf][row][n0] = make_float4(vb[0], vb[1], vb[2], vb[3]);
         *(float4*)&sh.C[buf][row][n0] = make_float4(vc[0], vc[1], vc[2], vc[3]);
       }
@@ -352,17 +261,15 @@ __device__ __forceinline__ void store_state64(float* ckw, const f4_t (&X)[MT], f
 // One workgroup per (batch row, kMcDT channels, time segment); the segment's
 // sub-blocks are walked in order, the inputs of sub-block sb + 1 loaded while
 // sb is computed and staged at its end, B and C double-buffered
-// in LDS (one barrier per sub-block). MAP: the segment's map from a zero
-// state (decay per channel into segF, state into segZ) for the carry pass
-// over the segments, or with a.recomp the states entering the segment's
-// sub-blocks, from its checkpoint (one segment per checkpoint interval),
-// into a.ckpt; otherwise y, the checkpoint and hT from the entering state
-// (h0, or seg0 when T is split into segments).
-template <int NP, bool MAP, typename TU, typename TG, typename TB>
+// in LDS (one barrier per sub-block). RECOMP: the states entering the
+// segment's sub-blocks, from its checkpoint (one segment per checkpoint
+// interval), into a.ckpt; otherwise y, the checkpoint and hT from the
+// entering state (h0, or seg0 when T is split into segments).
+template <int NP, bool RECOMP, typename TU, typename TG, typename TB>
 __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) void mc_fwd_kernel(const ScanArgs a, int y_dt) {
   constexpr int MT = NP / 16;  // 16-entry tiles of the state index
-  using In = McIn<NP, MAP, TU, TG, TB>;
-  __shared__ __align__(16) McBC<NP, MAP> sh;
+  using In = McIn<NP, RECOMP, TU, TG, TB>;
+  __shared__ __align__(16) McBC<NP, RECOMP> sh;
   // per wave: f (later G for the exact path, then y) and w = i u as [channel][row]
   __shared__ __align__(16) float s_t[kMcW][2][16][TP];
 
@@ -388,9 +295,9 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
   // state entries n = 16m + 4g + r of channel d
   f4_t X[MT];
   {
-    const float* xin = MAP ? (a.recomp ? a.ck_src + ((int64_t)b * a.Kc_src + seg) * D * N : nullptr)
-                           : (a.nseg > 1 ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * N
-                                         : (a.h0 ? a.h0 + (int64_t)b * D * N : nullptr));
+    const float* xin = RECOMP ? a.ck_src + ((int64_t)b * a.Kc_src + seg) * D * N
+                              : (a.nseg > 1 ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * N
+                                            : (a.h0 ? a.h0 + (int64_t)b * D * N : nullptr));
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -402,7 +309,6 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
 #pragma unroll
     for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(X[m]));
   }
-  float Fseg = 1.f;
   // load role: row rho, channels cq .. cq+3 of the wave's 16
   const int rho = lane >> 2, cq = (lane & 3) * 4;
   // channels of the load role inside [0, D) (0..4), formed once: past D a
@@ -411,7 +317,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
   // D of the load role's channels (the D u term of y is added there)
   float Dvc[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) Dvc[e] = (!MAP && dw + cq + e < D) ? a.Dsk[dw + cq + e] : 0.f;
+  for (int e = 0; e < 4; ++e) Dvc[e] = (!RECOMP && dw + cq + e < D) ? a.Dsk[dw + cq + e] : 0.f;
   asm volatile("" : "+v"(Dvc[0]), "+v"(Dvc[1]), "+v"(Dvc[2]), "+v"(Dvc[3]));
 
   // inputs of sub-blocks sb (cur) and sb + 1 (nxt), loaded one sub-block
@@ -459,7 +365,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
     // (the product B_(arow) C_(arow)^T transposed; k-step (q, r') takes
     // n = 16q + 4k + r')
     f4_t Gp = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (!MAP && sizeof(TB) == 2 && NP >= 32) {
+    if constexpr (!RECOMP && sizeof(TB) == 2 && NP >= 32) {
       // B and C exact in TB: two 16-entry groups of n per K = 32 product
 #pragma unroll
       for (int q = 0; q < NP / 16; q += 2) {
@@ -473,7 +379,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
         }
         Gp = mma_k32<TB>(pb[0], pb[1], pc[0], pc[1], Gp);
       }
-    } else if constexpr (!MAP) {
+    } else if constexpr (!RECOMP) {
 #pragma unroll
       for (int q = 0; q < NP / 16; ++q) {
         const float4 c4 = *(const float4*)&sh.C[buf][arow][16 * q + 4 * g];
@@ -501,7 +407,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
     float pf[4], pe[4];
     const float Pall = own_decays(fa, g, pf, pe);
 
-    if constexpr (!MAP) {
+    if constexpr (!RECOMP) {
       // intra-sub-block part of y for the own rows t = 4r + g,
       // S[t] = sum_{s<=t} P[t,s] G[t][s] w_s.
       float S[4];
@@ -618,12 +524,11 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
         }
       }
     } else {
-      Fseg *= Pall;
-      if (NP == 64 && N == 64 && a.recomp && dw + 16 <= D) {
+      if (NP == 64 && N == 64 && dw + 16 <= D) {
         // the state entering sb, as the scan's checkpoint holds it (the
         // wave's gate tiles are free: f and w are in registers)
         store_state64(a.ckpt + (((int64_t)b * a.Kc + sb) * D + dw) * N, X, &s_t[wv][0][0][0], j, g, lane_l);
-      } else if (a.recomp && dok) {
+      } else if (dok) {
         // the state entering sb, as the scan's checkpoint holds it
         float* ck = a.ckpt + (((int64_t)b * a.Kc + sb) * D + d) * N;
 #pragma unroll
@@ -666,24 +571,12 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
         X[m] = mma(bt.w, wp[3], X[m]);
       }
     }
-    // the map's B of sb + 1 into the other buffer, as late as possible so
+    // the recompute's B of sb + 1 into the other buffer, as late as possible so
     // that its loads have the whole sub-block to land
-    if (MAP && sb + 1 < sb1) nxt.stage(sh, buf ^ 1, a, t0 + Q, tid);
+    if (RECOMP && sb + 1 < sb1) nxt.stage(sh, buf ^ 1, a, t0 + Q, tid);
     cur = nxt;
   }
-  if (!dok) return;
-  if (MAP) {
-    if (a.recomp) return;
-    const int64_t o = ((int64_t)b * a.nseg + seg) * D + d;
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = 16 * m + 4 * g + r;
-        if (n < N) a.segZ[o * N + n] = X[m][r];
-      }
-    if (g == 0) a.segF[o] = Fseg;
-  } else if (a.hT && seg == a.nseg - 1) {
+  if (!RECOMP && dok && a.hT && seg == a.nseg - 1) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -727,19 +620,19 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
 // (5 KB) and a pool of seven [16][TP] tiles (8.75 KB) that holds G, G^T,
 // gathers, the rectangle sums' partials, (dy Pf) / (w Pe), H / H^T and
 // finally the wave's dB / dC, which the workgroup adds in wave order.
-template <int NP, bool MAP>
+template <int NP>
 struct McBwdLds {
   static constexpr int P = NP + 4;
   static constexpr int POOL = 9 * 16 * TP;  // floats of a wave's pool
-  float Bn[MAP ? 1 : kMcQ][MAP ? 4 : P];
-  float C[MAP ? 1 : kMcQ][MAP ? 4 : P];
-  float Bt[MAP ? 1 : NP][TP];
+  float Bn[kMcQ][P];
+  float C[kMcQ][P];
+  float Bt[NP][TP];
   float Ct[NP][TP];
-  float gate[kMcWB][MAP ? 2 : 4][16][TP];  // f, dy, w, i as [channel][row]; later dfl, du, dil
-  float pool[MAP ? 1 : kMcWB][POOL];
+  float gate[kMcWB][4][16][TP];  // f, dy, w, i as [channel][row]; later dfl, du, dil
+  float pool[kMcWB][POOL];
 };
 
-template <int NP, bool MAP, typename TU, typename TG, typename TB>
+template <int NP, typename TU, typename TG, typename TB>
 struct McInB {
   Raw4<TG> f, i;
   Raw4<TU> dy, u;
@@ -757,7 +650,7 @@ struct McInB {
       const uint32_t o = off + (uint32_t)(dw + cq);
       ld4r<TG>((const TG*)a.fl + base, o, f);
       ld4r<TU>((const TU*)a.dy + base, o, dy);
-      if constexpr (!MAP) {
+      {
         ld4r<TG>((const TG*)a.il + base, o, i);
         ld4r<TU>((const TU*)a.u + base, o, u);
       }
@@ -767,7 +660,7 @@ struct McInB {
       for (int e = 0; e < 4; ++e) o[e] = off + (uint32_t)(dw + cq + e < D ? dw + cq + e : D - 1);
       ld4r_at<TG>((const TG*)a.fl + base, o, f);
       ld4r_at<TU>((const TU*)a.dy + base, o, dy);
-      if constexpr (!MAP) {
+      {
         ld4r_at<TG>((const TG*)a.il + base, o, i);
         ld4r_at<TU>((const TU*)a.u + base, o, u);
       }
@@ -779,13 +672,13 @@ struct McInB {
       const uint32_t ro = (uint32_t)((row < rows ? row : rows - 1) * a.ldbc);
       if (N == NP) {
         ld4r<TB>((const TB*)a.Cm + bb, ro + n0, c);
-        if constexpr (!MAP) ld4r<TB>((const TB*)a.Bm + bb, ro + n0, b);
+        ld4r<TB>((const TB*)a.Bm + bb, ro + n0, b);
       } else {
         uint32_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = ro + (uint32_t)(n0 + e < N ? n0 + e : N - 1);
         ld4r_at<TB>((const TB*)a.Cm + bb, o, c);
-        if constexpr (!MAP) ld4r_at<TB>((const TB*)a.Bm + bb, o, b);
+        ld4r_at<TB>((const TB*)a.Bm + bb, o, b);
       }
     }
   }
@@ -806,7 +699,7 @@ struct McInB {
   // different banks, and each [t][n] tile takes one 16-byte write per lane
   // (the forward's row-per-16-lanes map costs 14 and 6 extra LDS cycles per
   // write there, about 1.4% of this kernel).
-  __device__ __forceinline__ void stage(McBwdLds<NP, MAP>& sh, const ScanArgs& a, int64_t t0, int tid) const {
+  __device__ __forceinline__ void stage(McBwdLds<NP>& sh, const ScanArgs& a, int64_t t0, int tid) const {
     if (tid < 4 * NP) {
       const int row = tid % kMcQ, n0 = 4 * (tid / kMcQ);
       const bool rok = t0 + row < a.T;
@@ -817,12 +710,12 @@ struct McInB {
         const bool ok = rok && n0 + e < a.N;
         vc[e] = ok ? c.get(e) : 0.f;
         sh.Ct[n0 + e][pr] = vc[e];
-        if constexpr (!MAP) {
+        {
           vb[e] = ok ? b.get(e) : 0.f;
           sh.Bt[n0 + e][pr] = vb[e];
         }
       }
-      if constexpr (!MAP) {
+      {
         *(float4*)&sh.Bn[row][n0] = make_float4(vb[0], vb[1], vb[2], vb[3]);
         *(float4*)&sh.C[row][n0] = make_float4(vc[0], vc[1], vc[2], vc[3]);
       }
@@ -916,17 +809,17 @@ __device__ __forceinline__ void store_row4(void* p, uint32_t o, const float (*tl
   }
 }
 
-template <int NP, bool MAP, typename TU, typename TG, typename TB>
+template <int NP, typename TU, typename TG, typename TB>
 __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, int du_dt, int dg_dt) {
   constexpr int MT = NP / 16;
   constexpr int P = NP + 4;
-  using In = McInB<NP, MAP, TU, TG, TB>;
-  __shared__ __align__(16) McBwdLds<NP, MAP> sh;
+  using In = McInB<NP, TU, TG, TB>;
+  __shared__ __align__(16) McBwdLds<NP> sh;
 
   const int N = a.N;
   const int64_t T = a.T, D = a.D;
   const int tile = (int)(blockIdx.x % (uint32_t)a.n_tiles);
-  const int seg = (int)(blockIdx.x / (uint32_t)a.n_tiles) + (MAP ? 1 : 0);
+  const int seg = (int)(blockIdx.x / (uint32_t)a.n_tiles);
   const int b = tile / a.n_dtiles;
   const int dtile = tile - b * a.n_dtiles;
   const int tid = (int)threadIdx.x;
@@ -942,13 +835,13 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
   const bool vec = dw + 16 <= D && D % 4 == 0;
   const int rho = lane >> 2, cq = (lane & 3) * 4;
   const int ncq = (int)(D - dw - cq < 4 ? (D - dw - cq < 0 ? 0 : D - dw - cq) : 4);  // valid of cq .. cq+3
-  float Dv = (!MAP && dok) ? a.Dsk[d] : 0.f;
+  float Dv = dok ? a.Dsk[d] : 0.f;
   asm volatile("" : "+v"(Dv));
 
   // adjoint carry in the D layout: gh[m][r] = entry 16m + 4g + r of channel j
   f4_t gh[MT];
   {
-    const float* gin = (!MAP && a.nseg > 1) ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * N : nullptr;
+    const float* gin = a.nseg > 1 ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * N : nullptr;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -960,7 +853,6 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
     for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(gh[m]));
   }
-  float Fseg = 1.f;
   float dDacc[4] = {0.f, 0.f, 0.f, 0.f};
   float sgf = 0.f, sgi = 0.f;  // dfl, dil summed over this lane's rows (channel j)
 
@@ -973,11 +865,11 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
   In cur, nxt;
   // the checkpointed state entering the current (xc) and the next (xn)
   // sub-block, loaded one sub-block ahead like the inputs
-  f4_t xc[MAP ? 1 : MT], xn[MAP ? 1 : MT];
+  f4_t xc[MT], xn[MT];
   if (sb0 < sb1) {
     cur.load(a, b, (int64_t)(sb1 - 1) * Q, dw, rho, cq, tid, vec);
     cur.settle();
-    if constexpr (!MAP) {
+    {
       load_ckpt<MT>(xc, a, b, sb1 - 1, dok ? d : D - 1, g);
 #pragma unroll
       for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(xc[m]));
@@ -1012,7 +904,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       asm volatile("" : "+v"(sf));
       Tf[cq + e][rho] = ok ? sf : 1.f;
       Tdy[cq + e][rho] = ok ? cur.dy.get(e) : 0.f;
-      if constexpr (!MAP) {
+      {
         float si = sigm(cur.i.get(e));
         asm volatile("" : "+v"(si));
         const float ig = ok ? si : 0.f;
@@ -1024,7 +916,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
     __syncthreads();  // staging visible
     if (sb - 1 >= sb0) {
       nxt.load(a, b, t0 - Q, dw, rho, cq, tid, vec);
-      if constexpr (!MAP) load_ckpt<MT>(xn, a, b, sb - 1, dcl, g);
+      load_ckpt<MT>(xn, a, b, sb - 1, dcl, g);
     }
     asm volatile("" ::: "memory");
 
@@ -1044,7 +936,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
     for (int r = 0; r < 4; ++r) pfdy[r] = pf[r] * dy_o[r];
 
-    if constexpr (!MAP) {
+    {
       float (*Tw)[TP] = sh.gate[wv][2];
       float (*Ti)[TP] = sh.gate[wv][3];
       float* pl = sh.pool[wv];
@@ -1055,7 +947,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       // H in the pool's last two tiles, past the dC / dB partials (which take
       // its first 32 P floats) and the scratch tiles: other waves read it
       // after the partial-sum barrier
-      constexpr int kPH = McBwdLds<NP, MAP>::POOL - 32 * TP;
+      constexpr int kPH = McBwdLds<NP>::POOL - 32 * TP;
       static_assert(32 * P <= kPH && 7 * 16 * TP <= kPH, "H tiles clear of the partials and scratch tiles");
       float (*TH)[TP] = (float (*)[TP])(pl + kPH);             // H[t][p(r)]
       float (*THT)[TP] = (float (*)[TP])(pl + kPH + 16 * TP);  // H[s][t] at [t][p(s)]
@@ -1497,32 +1389,17 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
           }
         }
       }
-    } else {
-      // MAP: the adjoint map of the segment (ghat from zero, decay product)
-      Fseg *= Pall;
-      carry_update<TB, MT>(gh, sh.Ct, Pall, pfdy, j, g);
     }
     // every wave is done with the staged B / C (and, in the scan, with the
     // pools and H tiles its output tile reads) before they are restaged
     __syncthreads();
     cur = nxt;
-    if constexpr (!MAP) {
+    {
 #pragma unroll
       for (int m = 0; m < MT; ++m) xc[m] = xn[m];
     }
   }
-  if constexpr (MAP) {
-    if (!dok) return;
-    const int64_t o = ((int64_t)b * a.nseg + seg) * D + d;
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = 16 * m + 4 * g + r;
-        if (n < N) a.segZ[o * N + n] = gh[m][r];
-      }
-    if (g == 0) a.segF[o] = Fseg;
-  } else {
+  {
     if (a.dh0 && seg == 0 && dok) {
 #pragma unroll
       for (int m = 0; m < MT; ++m)
@@ -1570,60 +1447,59 @@ int np16(int64_t N) { return N <= 16 ? 16 : (N <= 32 ? 32 : 64); }
 typedef void (*mc_fwd_t)(ScanArgs, int);
 
 template <typename TU, typename TG, typename TB>
-mc_fwd_t pick_fwd_np(int np, bool map) {
+mc_fwd_t pick_fwd_np(int np, bool rec) {
   switch (np) {
-    case 16: return map ? mc_fwd_kernel<16, true, TU, TG, TB> : mc_fwd_kernel<16, false, TU, TG, TB>;
-    case 32: return map ? mc_fwd_kernel<32, true, TU, TG, TB> : mc_fwd_kernel<32, false, TU, TG, TB>;
-    default: return map ? mc_fwd_kernel<64, true, TU, TG, TB> : mc_fwd_kernel<64, false, TU, TG, TB>;
+    case 16: return rec ? mc_fwd_kernel<16, true, TU, TG, TB> : mc_fwd_kernel<16, false, TU, TG, TB>;
+    case 32: return rec ? mc_fwd_kernel<32, true, TU, TG, TB> : mc_fwd_kernel<32, false, TU, TG, TB>;
+    default: return rec ? mc_fwd_kernel<64, true, TU, TG, TB> : mc_fwd_kernel<64, false, TU, TG, TB>;
   }
 }
 
 // The served dtype combinations (u; gates f32 or u's; B/C f32 or u's).
 template <typename TU>
-mc_fwd_t pick_fwd_u(int g_dt, int bc_dt, int np, bool map) {
+mc_fwd_t pick_fwd_u(int g_dt, int bc_dt, int np, bool rec) {
   const bool gf = g_dt == NAJU_DTYPE_F32, bf = bc_dt == NAJU_DTYPE_F32;
-  if (gf) return bf ? pick_fwd_np<TU, float, float>(np, map) : pick_fwd_np<TU, float, TU>(np, map);
-  return bf ? pick_fwd_np<TU, TU, float>(np, map) : pick_fwd_np<TU, TU, TU>(np, map);
+  if (gf) return bf ? pick_fwd_np<TU, float, float>(np, rec) : pick_fwd_np<TU, float, TU>(np, rec);
+  return bf ? pick_fwd_np<TU, TU, float>(np, rec) : pick_fwd_np<TU, TU, TU>(np, rec);
 }
 
 typedef void (*mc_bwd_t)(ScanArgs, int, int);
 
 template <typename TU, typename TG, typename TB>
-mc_bwd_t pick_bwd_np(int np, bool map) {
+mc_bwd_t pick_bwd_np(int np) {
   switch (np) {
-    case 16: return map ? mc_bwd_kernel<16, true, TU, TG, TB> : mc_bwd_kernel<16, false, TU, TG, TB>;
-    case 32: return map ? mc_bwd_kernel<32, true, TU, TG, TB> : mc_bwd_kernel<32, false, TU, TG, TB>;
-    default: return map ? mc_bwd_kernel<64, true, TU, TG, TB> : mc_bwd_kernel<64, false, TU, TG, TB>;
+    case 16: return mc_bwd_kernel<16, TU, TG, TB>;
+    case 32: return mc_bwd_kernel<32, TU, TG, TB>;
+    default: return mc_bwd_kernel<64, TU, TG, TB>;
   }
 }
 
 template <typename TU>
-mc_bwd_t pick_bwd_u(int g_dt, int bc_dt, int np, bool map) {
+mc_bwd_t pick_bwd_u(int g_dt, int bc_dt, int np) {
   const bool gf = g_dt == NAJU_DTYPE_F32, bf = bc_dt == NAJU_DTYPE_F32;
-  if (gf) return bf ? pick_bwd_np<TU, float, float>(np, map) : pick_bwd_np<TU, float, TU>(np, map);
-  return bf ? pick_bwd_np<TU, TU, float>(np, map) : pick_bwd_np<TU, TU, TU>(np, map);
+  if (gf) return bf ? pick_bwd_np<TU, float, float>(np) : pick_bwd_np<TU, float, TU>(np);
+  return bf ? pick_bwd_np<TU, TU, float>(np) : pick_bwd_np<TU, TU, TU>(np);
 }
 
-hipError_t mc_fwd_launch(const ScanArgs& a, bool map, int x_dt, int g_dt, int y_dt, hipStream_t st) {
-  const int segs = map ? a.nseg - 1 : a.nseg;
-  const unsigned grid = (unsigned)((int64_t)a.n_tiles * segs);
+hipError_t mc_fwd_launch(const ScanArgs& a, int x_dt, int g_dt, int y_dt, hipStream_t st) {
+  const bool rec = a.recomp != 0;
+  const unsigned grid = (unsigned)((int64_t)a.n_tiles * a.nseg);
   if (grid == 0) return hipSuccess;
   const int np = np16(a.N);
-  mc_fwd_t k = x_dt == NAJU_DTYPE_F32    ? pick_fwd_np<float, float, float>(np, map)
-               : x_dt == NAJU_DTYPE_BF16 ? pick_fwd_u<bf16_t>(g_dt, a.bc_dt, np, map)
-                                         : pick_fwd_u<f16_t>(g_dt, a.bc_dt, np, map);
+  mc_fwd_t k = x_dt == NAJU_DTYPE_F32    ? pick_fwd_np<float, float, float>(np, rec)
+               : x_dt == NAJU_DTYPE_BF16 ? pick_fwd_u<bf16_t>(g_dt, a.bc_dt, np, rec)
+                                         : pick_fwd_u<f16_t>(g_dt, a.bc_dt, np, rec);
   hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kMcW), 0, st, a, y_dt);
   return hipGetLastError();
 }
 
-hipError_t mc_bwd_launch(const ScanArgs& a, bool map, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st) {
-  const int segs = map ? a.nseg - 1 : a.nseg;
-  const unsigned grid = (unsigned)((int64_t)a.n_tiles * segs);
+hipError_t mc_bwd_launch(const ScanArgs& a, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st) {
+  const unsigned grid = (unsigned)((int64_t)a.n_tiles * a.nseg);
   if (grid == 0) return hipSuccess;
   const int np = np16(a.N);
-  mc_bwd_t k = x_dt == NAJU_DTYPE_F32    ? pick_bwd_np<float, float, float>(np, map)
-               : x_dt == NAJU_DTYPE_BF16 ? pick_bwd_u<bf16_t>(g_dt, a.bc_dt, np, map)
-                                         : pick_bwd_u<f16_t>(g_dt, a.bc_dt, np, map);
+  mc_bwd_t k = x_dt == NAJU_DTYPE_F32    ? pick_bwd_np<float, float, float>(np)
+               : x_dt == NAJU_DTYPE_BF16 ? pick_bwd_u<bf16_t>(g_dt, a.bc_dt, np)
+                                         : pick_bwd_u<f16_t>(g_dt, a.bc_dt, np);
   hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kMcWB), 0, st, a, du_dt, dg_dt);
   return hipGetLastError();
 }

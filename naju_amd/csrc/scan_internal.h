@@ -106,10 +106,10 @@ struct ScanArgs {
   int K;
   int ck_rows;  // rows per checkpoint interval of ckpt
   int Kc;       // number of checkpoint intervals of ckpt
-  // Chunked matrix-core forward map launch with recomp = 1: the backward's
+  // Chunked matrix-core forward launch with recomp = 1: the backward's
   // recompute of the state entering every sub-block (into ckpt, Kc of them)
   // from the forward's checkpoint ck_src (Kc_src intervals, one segment
-  // each) instead of a segment map.
+  // each) instead of the scan.
   // (With a checkpoint interval longer than the sub-block the forward's time
   // segments start at interval boundaries, so every state the recompute
   // starts from is a checkpoint entry.)
@@ -209,12 +209,14 @@ constexpr float kMcRatioMin = 0x1p-30f;
 // True when the chunked kernels serve this state size.
 inline bool mc_ok(int64_t N) { return N > 8 && N <= 64; }
 
-// Forward: map = true computes the maps of segments 0 .. nseg-2 (segF /
-// segZ); map = false the scan itself from h0 or the carried segment states.
-hipError_t mc_fwd_launch(const ScanArgs& a, bool map, int x_dt, int g_dt, int y_dt, hipStream_t st);
-// Backward: map = true the adjoint maps of segments 1 .. nseg-1; map = false
-// du, dfl, dil, dh0 and the dB / dC / dD partials.
-hipError_t mc_bwd_launch(const ScanArgs& a, bool map, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st);
+// The maps of segments 0 .. nseg-2 (forward) or 1 .. nseg-1 (backward) into
+// segF / segZ (naju_scan_map.hip).
+hipError_t mc_map_launch(const ScanArgs& a, bool bwd, int x_dt, int g_dt, hipStream_t st);
+// Forward: the scan from h0 or the carried segment states, or with a.recomp
+// the recompute of the states from a memory-light checkpoint.
+hipError_t mc_fwd_launch(const ScanArgs& a, int x_dt, int g_dt, int y_dt, hipStream_t st);
+// Backward: du, dfl, dil, dh0 and the dB / dC / dD partials.
+hipError_t mc_bwd_launch(const ScanArgs& a, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st);
 
 }  // namespace naju_detail
 
