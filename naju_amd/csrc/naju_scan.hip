@@ -1583,30 +1583,52 @@ __global__ __launch_bounds__(64 * kGcW) void gc_fwd_kernel(const ScanArgs a, int
 
 // Carry over the time segments, one thread per (b, d, n): the state entering
 // each segment (dir = +1, from h0) or the adjoint carry entering it from the
-// future (dir = -1, from zero), into seg0.
-__global__ void gn_seg_carry_kernel(const ScanArgs a, int dir) {
+// future (dir = -1, from zero), into seg0. The maps of kCarryU segments are
+// loaded together, ahead of the chain of FMAs over them: one load latency per
+// kCarryU segments instead of one per segment (2 x 1024 x 256, N = 64, 64
+// segments: 22 -> 8 us).
+constexpr int kCarryU = 8;
+__global__ __launch_bounds__(256) void gn_seg_carry_kernel(const ScanArgs a, int dir) {
   const int64_t DN = a.D * (int64_t)a.N;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)a.batch * DN) return;
   const int64_t b = i / DN, dn = i - b * DN, d = dn / a.N;
   const int ns = a.nseg;
-  if (dir > 0) {
-    float x = a.h0 ? a.h0[i] : 0.f;
-    for (int sg = 0; sg < ns; ++sg) {
-      const int64_t o = (b * ns + sg) * a.D + d;
-      a.seg0[o * a.N + (dn - d * a.N)] = x;
-      if (sg + 1 < ns) x = fmaf(a.segF[o], x, a.segZ[o * a.N + (dn - d * a.N)]);
+  // step k handles segment k (forward) or ns - 1 - k (backward); the last
+  // step's map is not needed (nor written by the map pass)
+  const int s0 = dir > 0 ? 0 : ns - 1;
+  const float* pF = a.segF + (b * ns + s0) * a.D + d;
+  const float* pZ = a.segZ + (b * ns + s0) * DN + dn;
+  float* po = a.seg0 + (b * ns + s0) * DN + dn;
+  const int64_t sF = dir > 0 ? a.D : -a.D, sZ = dir > 0 ? DN : -DN;
+  float x = dir > 0 && a.h0 ? a.h0[i] : 0.f;
+  int k = 0;
+  for (; k + kCarryU < ns; k += kCarryU) {
+    float F[kCarryU], Z[kCarryU];
+#pragma unroll
+    for (int e = 0; e < kCarryU; ++e) F[e] = pF[e * sF], Z[e] = pZ[e * sZ];
+#pragma unroll
+    for (int e = 0; e < kCarryU; ++e) {
+      po[e * sZ] = x;
+      x = fmaf(F[e], x, Z[e]);
     }
-  } else {
-    float g = 0.f;
-    for (int sg = ns - 1; sg >= 0; --sg) {
-      const int64_t o = (b * ns + sg) * a.D + d;
-      a.seg0[o * a.N + (dn - d * a.N)] = g;
-      if (sg > 0) g = fmaf(a.segF[o], g, a.segZ[o * a.N + (dn - d * a.N)]);
-    }
+    pF += kCarryU * sF, pZ += kCarryU * sZ, po += kCarryU * sZ;
+  }
+  // the last 1 .. kCarryU segments, loads clamped to the maps that exist
+  const int left = ns - k;
+  float F[kCarryU], Z[kCarryU];
+#pragma unroll
+  for (int e = 0; e < kCarryU - 1; ++e) {
+    const int q = e < left - 1 ? e : (left > 1 ? left - 2 : 0);
+    if (left > 1) F[e] = pF[q * sF], Z[e] = pZ[q * sZ];
+  }
+#pragma unroll
+  for (int e = 0; e < kCarryU; ++e) {
+    if (e >= left) break;
+    po[e * sZ] = x;
+    if (e + 1 < left) x = fmaf(F[e], x, Z[e]);
   }
 }
-
 
 // ------------------------------------------------- general N backward kernel
 //
