@@ -39,7 +39,7 @@
  *   NAJU_CKPT_ROWS(r) (bits 8-15): the forward's checkpoint interval for
  *     N > 1, r rows (32, 64 or 128; 0 = the default). The checkpoint holds
  *     the state every r rows (batch*ceil(T/r)*D*N floats).
- *     The default is 16 rows for 9 <= N <= 64 (the state entering every
+ *     The default is 16 rows for 9 <= N <= 128 (the state entering every
  *     sub-block of the matrix-core backward) and 32 rows otherwise; a longer
  *     interval is the memory-light mode of the reference's recompute backend
  *     (naju/cuda/__init__.py:9-12, CK = 32 in naju/cuda/naju_cuda.cu:25):
@@ -51,7 +51,8 @@
  *     and backward shrinks r/16-fold at the cost of that pass. Every output
  *     is bitwise the one of the default interval.
  *     Served for 9 <= N <= 64 by naju_scan_fwd and naju_scan_fwd_noalloc;
- *     other N accept only their default (NAJU_ERR_UNSUPPORTED otherwise).
+ *     other N accept only their default (NAJU_ERR_UNSUPPORTED otherwise;
+ *     at N > 64 its name is 32 rows).
  *     The backward must be given the forward's flags value for these bits,
  *     and the size queries below have _ex forms that take it.
  *

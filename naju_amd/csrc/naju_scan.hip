@@ -1163,41 +1163,6 @@ __device__ __forceinline__ void gn_ld_bc(const ScanArgs& a, const void* p, int b
   }
 }
 
-// The same from a uniform tile base plus 32-bit lane offsets (the gq
-// forward's staging; the segmented forward keeps gn_ld_bc, which measured
-// faster there).
-template <int NP, int EB, int NT = kGnThreads>
-__device__ __forceinline__ void gq_ld_bc(const ScanArgs& a, const void* p, int b, int64_t t0, float (&v)[EB]) {
-  static_assert(NT % NP == 0, "staging rows");
-  // A uniform base (row t0 of batch row b) plus a 32-bit per-lane offset
-  // (at most kGnCK rows x N < 2^12 elements): rows past T are clamped to the
-  // last row, states past N to N - 1.
-  const int64_t tb = t0 < a.T ? t0 : a.T - 1;
-  const int rmax = (int)(a.T - tb < kGnCK ? a.T - tb : kGnCK) - 1;
-  const int64_t row0 = ((int64_t)b * a.T + tb) * a.N;
-  const int n = (int)threadIdx.x % NP;
-  const uint32_t nn = (uint32_t)(n < a.N ? n : a.N - 1);
-  uint32_t off[EB];
-#pragma unroll
-  for (int e = 0; e < EB; ++e) {
-    const int r = e * (NT / NP) + (int)threadIdx.x / NP;
-    off[e] = (uint32_t)(r < rmax ? r : rmax) * (uint32_t)a.N + nn;
-  }
-  if (a.bc_dt == NAJU_DTYPE_F32) {
-    const float* q = (const float*)p + row0;
-#pragma unroll
-    for (int e = 0; e < EB; ++e) v[e] = q[off[e]];
-  } else if (a.bc_dt == NAJU_DTYPE_BF16) {
-    const bf16_t* q = (const bf16_t*)p + row0;
-#pragma unroll
-    for (int e = 0; e < EB; ++e) v[e] = (float)q[off[e]];
-  } else {
-    const f16_t* q = (const f16_t*)p + row0;
-#pragma unroll
-    for (int e = 0; e < EB; ++e) v[e] = (float)q[off[e]];
-  }
-}
-
 // Writes a prefetched B/C tile into LDS, zero where the row is past T or the
 // state index past N.
 template <int NP, int EB>
@@ -1664,165 +1629,6 @@ __device__ __forceinline__ float from_upper(float x) {
     return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
   } else {
     return __shfl_xor(x, m, 64);
-  }
-}
-
-// General-N forward with Q = NP/4 lanes per channel, four states per lane,
-// over the whole of T: lane (channel c, quarter q) holds x[n] for
-// n = 4q .. 4q+3. With Q times the lanes per channel of gc_fwd_kernel it
-// needs no time segments (no segment-map pass, no carry pass) once the
-// batch x channel-group grid fills the GPU on its own. Per
-// 32-row sub-chunk the workgroup stages B and C ([row][n]) and the channels'
-// gates f, w = i*u and u ([row][channel]) in LDS, each value computed once;
-// a lane's part of y_t = sum_n C_t[n] x_t[n] is summed over the channel's Q
-// lanes by a transposing butterfly over 8 rows at a time, and y goes back
-// through LDS so that its stores are row-contiguous.
-constexpr int kGqW = 4;   // waves per workgroup
-constexpr int kGqRG = 8;  // rows per reduction group
-
-template <int NP>
-__global__ __launch_bounds__(64 * kGqW) void gq_fwd_kernel(const ScanArgs a, int x_dt, int g_dt, int y_dt) {
-  constexpr int Q = NP / 4;          // lanes per channel
-  constexpr int CPW = 64 / Q;        // channels per wave
-  constexpr int CPB = CPW * kGqW;    // channels per workgroup
-  constexpr int NT = 64 * kGqW;      // threads
-  constexpr int EB = kGnCK * NP / NT;   // B / C values staged per thread
-  constexpr int EG = kGnCK * CPB / NT;  // gate values staged per thread
-  static_assert(Q >= 4 && Q <= 16 && EB >= 1 && EG >= 1, "tile shape");
-  __shared__ __align__(16) float s_B[kGnCK][NP];
-  __shared__ __align__(16) float s_C[kGnCK][NP];
-  __shared__ float s_f[kGnCK][CPB], s_w[kGnCK][CPB], s_u[kGnCK][CPB], s_y[kGnCK][CPB];
-  const int N = a.N;
-  const int64_t T = a.T, D = a.D;
-  const int ndt = (int)((D + CPB - 1) / CPB);
-  const int b = (int)(blockIdx.x / (uint32_t)ndt);
-  const int dtile = (int)(blockIdx.x - (uint32_t)b * (uint32_t)ndt);
-  const int64_t dbase = (int64_t)dtile * CPB;
-  const int tid = (int)threadIdx.x;
-  const int lane = tid & 63;
-  const int wv = tid >> 6;
-  const int cl = wv * CPW + lane / Q;  // this lane's channel within the workgroup
-  const int q = lane % Q;
-  const int64_t d = dbase + cl;
-  const bool dok = d < D;
-  const int64_t rowbase = (int64_t)b * T;
-  const int KC = (int)((T + kGnCK - 1) / kGnCK);
-  const int sc0 = 0, sc1 = KC;
-  const float* xin = a.h0 ? a.h0 + (int64_t)b * D * N : nullptr;
-  float x[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int n = 4 * q + k;
-    x[k] = (xin && dok && n < N) ? xin[d * N + n] : 0.f;
-  }
-  // staging roles for the gates: entry k = e * NT + tid -> (row, channel)
-  // two register sets of staged inputs: sub-chunk sc is loaded while
-  // sc - 2 is computed (a wave's compute of one sub-chunk is shorter than
-  // the load latency)
-  float gu0[EG], gf0[EG], gi0[EG], vb0[EB], vc0[EB];
-  float gu1[EG], gf1[EG], gi1[EG], vb1[EB], vc1[EB];
-  auto load = [&](int64_t t0, float (&gu)[EG], float (&gf)[EG], float (&gi)[EG], float (&vb)[EB],
-                  float (&vc)[EB]) {
-#pragma unroll
-    for (int e = 0; e < EG; ++e) {
-      const int k = e * NT + tid;
-      const int r = k / CPB, c = k % CPB;
-      const int64_t t = t0 + r < T ? t0 + r : T - 1;
-      const int64_t dc = dbase + c < D ? dbase + c : D - 1;
-      const int64_t o = (rowbase + t) * D + dc;
-      gu[e] = ld_any(a.u, x_dt, o);
-      gf[e] = ld_any(a.fl, g_dt, o);
-      gi[e] = ld_any(a.il, g_dt, o);
-    }
-    gq_ld_bc<NP, EB, NT>(a, a.Bm, b, t0, vb);
-    gq_ld_bc<NP, EB, NT>(a, a.Cm, b, t0, vc);
-  };
-  auto body = [&](int sc, float (&gu)[EG], float (&gf)[EG], float (&gi)[EG], float (&vb)[EB], float (&vc)[EB]) {
-    const int64_t t0 = (int64_t)sc * kGnCK;
-    const int rows = (int)((T - t0) < kGnCK ? (T - t0) : kGnCK);
-    __syncthreads();  // the previous sub-chunk's tiles are consumed, its y stored
-#pragma unroll
-    for (int e = 0; e < EG; ++e) {
-      const int k = e * NT + tid;
-      const int r = k / CPB, c = k % CPB;
-      const bool ok = r < rows && dbase + c < D;
-      const float f = sigm(gf[e]);
-      s_f[r][c] = ok ? f : 1.f;
-      s_w[r][c] = ok ? sigm(gi[e]) * gu[e] : 0.f;
-      s_u[r][c] = ok ? gu[e] : 0.f;
-    }
-#pragma unroll
-    for (int e = 0; e < EB; ++e) {
-      const int k = e * NT + tid;
-      const int r = k / NP, n = k % NP;
-      const bool ok = r < rows && n < N;
-      s_B[r][n] = ok ? vb[e] : 0.f;
-      s_C[r][n] = ok ? vc[e] : 0.f;
-    }
-    __syncthreads();
-    if (sc + 2 < sc1) load(t0 + 2 * kGnCK, gu, gf, gi, vb, vc);  // while this one runs
-    // the state entering this sub-chunk: the backward's checkpoint
-    if (a.ckpt && dok) {
-      float* ck = a.ckpt + (((int64_t)b * KC + sc) * D + d) * N;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (4 * q + k < N) ck[4 * q + k] = x[k];
-    }
-#pragma unroll
-    for (int g = 0; g < kGnCK; g += kGqRG) {
-      float yp[kGqRG];
-#pragma unroll
-      for (int rr = 0; rr < kGqRG; ++rr) {
-        const int r = g + rr;
-        const float f = s_f[r][cl], w = s_w[r][cl];
-        const float4 b4 = *(const float4*)&s_B[r][4 * q];
-        const float4 c4 = *(const float4*)&s_C[r][4 * q];
-        float acc = 0.f;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          x[k] *= f;
-          x[k] = fmaf(w, (&b4.x)[k], x[k]);
-          acc = fmaf((&c4.x)[k], x[k], acc);
-        }
-        yp[rr] = acc;
-      }
-      // sums over the channel's Q lanes: lane q then holds row q / (Q / 8)
-      // of the group (Q >= 8), or rows 2q, 2q+1 (Q = 4)
-      trd_step<Q, kGqRG, kGqRG>(yp, lane);
-      if constexpr (Q >= kGqRG) {
-        constexpr int SP = Q / kGqRG;
-        if (q % SP == 0) {
-          const int r = g + q / SP;
-          s_y[r][cl] = fmaf(a.Dsk[dok ? d : 0], s_u[r][cl], yp[0]);
-        }
-      } else {
-        constexpr int PER = kGqRG / Q;
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-          const int r = g + q * PER + j;
-          s_y[r][cl] = fmaf(a.Dsk[dok ? d : 0], s_u[r][cl], yp[j]);
-        }
-      }
-    }
-    __syncthreads();
-    // y of the sub-chunk, row-contiguous stores
-#pragma unroll
-    for (int e = 0; e < EG; ++e) {
-      const int k = e * NT + tid;
-      const int r = k / CPB, c = k % CPB;
-      if (r < rows && dbase + c < D) st_any(a.y, y_dt, (rowbase + t0 + r) * D + dbase + c, s_y[r][c]);
-    }
-  };
-  load((int64_t)sc0 * kGnCK, gu0, gf0, gi0, vb0, vc0);
-  if (sc0 + 1 < sc1) load((int64_t)(sc0 + 1) * kGnCK, gu1, gf1, gi1, vb1, vc1);
-  for (int sc = sc0; sc < sc1; sc += 2) {
-    body(sc, gu0, gf0, gi0, vb0, vc0);
-    if (sc + 1 < sc1) body(sc + 1, gu1, gf1, gi1, vb1, vc1);
-  }
-  if (a.hT && dok) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (4 * q + k < N) a.hT[((int64_t)b * D + d) * N + 4 * q + k] = x[k];
   }
 }
 
@@ -2331,7 +2137,7 @@ struct Layout {
   int V, CH, L, K, n_dtiles, n_tiles;
   int nseg, seg_sc;  // N > 1: time segments
   int ck_rows;       // the forward's checkpoint interval
-  size_t off_agg, off_incl, off_partB, off_partC, off_partD, off_partG, off_segF, off_segZ, off_seg0, off_dense, total;
+  size_t off_agg, off_incl, off_partB, off_partC, off_partD, off_partG, off_segF, off_segZ, off_seg0, off_half, off_dense, total;
 };
 
 // N > 1: enough time segments that about kGnTargetWgs workgroups run per
@@ -2382,15 +2188,12 @@ int mc_seg_sc(int64_t n_tiles, int K, bool bwd, int unit) {
   }
   return best;
 }
-// gq_fwd_kernel serves a forward whose batch x channel-group grid holds at
-// least three 4-wave workgroups per CU (256 CUs); smaller grids take the
-// segmented gc_fwd_kernel, whose time segments supply the parallelism.
-constexpr int kGqMinWgs = 768;
+// The backward's workgroups at N <= 8: 32 channels in 4 waves.
+constexpr int kGnBwdDT = 32, kGnBwdW = 4;
 
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 int np_of(int64_t N);
-bool gq_ok(int64_t N, int64_t batch, int64_t D);
 // The chunked matrix-core kernels serve 9 <= N <= 64 in the directions that
 // have them.
 constexpr bool kMcBwd = true;
@@ -2405,14 +2208,14 @@ int64_t gn_ck_rows(int64_t N) { return use_mc(N, true) ? kMcQ : kGnCK; }
 int ckpt_rows(int flags, int64_t N) {
   const int r = ((flags & NAJU_CKPT_MASK) >> NAJU_CKPT_SHIFT) * 16;
   const int def = N == 1 ? kBChunk : (int)gn_ck_rows(N);
+  // N > 64: 32 rows names the default, which holds the state every sub-block
+  if (mc_ok(N) && !mc_ext_ok(N)) return r == 0 || r == kGnCK ? def : -1;
   if (r == 0 || r == def) return def;
   // 2, 4, ... kMcSegUnit sub-blocks: intervals that divide the forward's
   // segment unit
   const bool served = r > kMcQ && r <= kMcQ * kMcSegUnit && (kMcQ * kMcSegUnit) % r == 0;
-  return (N > 1 && use_mc(N, true) && served) ? r : -1;
+  return (mc_ext_ok(N) && served) ? r : -1;
 }
-int gq_channels(int64_t N);
-int gn_bwd_dt(int np);
 
 // Byte offsets of the workspace regions for the layout's K, tiles and
 // segments (the backward's partial sums only when bwd).
@@ -2432,7 +2235,7 @@ void place_regions(Layout& l, int64_t batch, int64_t T, int64_t D, int64_t N, bo
   off = align_up(off + (bwd ? (size_t)batch * (N == 1 ? l.K : l.nseg) * D * sizeof(float) : 0));
   // the matrix-core backward's per-segment sums of dfl and dil (when asked for)
   l.off_partG = off;
-  off = align_up(off + (bwd && N > 1 && use_mc(N, true) ? (size_t)2 * batch * l.nseg * D * sizeof(float) : 0));
+  off = align_up(off + (bwd && mc_ext_ok(N) ? (size_t)2 * batch * l.nseg * D * sizeof(float) : 0));
   const size_t seg_units = l.nseg > 1 ? (size_t)batch * l.nseg * D : 0;
   l.off_segF = off;
   off = align_up(off + seg_units * sizeof(float));
@@ -2442,7 +2245,11 @@ void place_regions(Layout& l, int64_t batch, int64_t T, int64_t D, int64_t N, bo
   off = align_up(off + seg_units * N * sizeof(float));
   // the backward's recomputed state at every sub-block when the forward's
   // checkpoint interval is longer than the sub-block
-  const bool dense = bwd && N > 1 && use_mc(N, true) && l.ck_rows > kMcQ;
+  // N > 64: the backward's first half's terms of dws and xbar . x
+  const size_t KS = (size_t)((T + kMcQ - 1) / kMcQ);
+  l.off_half = off;
+  off = align_up(off + (bwd && mc_ok(N) && !mc_ext_ok(N) ? (size_t)batch * KS * D * 2 * kMcQ * sizeof(float) : 0));
+  const bool dense = bwd && mc_ext_ok(N) && l.ck_rows > kMcQ;
   l.off_dense = off;
   off = align_up(off + (dense ? (size_t)batch * ((T + kMcQ - 1) / kMcQ) * D * N * sizeof(float) : 0));
   l.total = off;
@@ -2475,7 +2282,7 @@ Layout make_layout(int64_t batch, int64_t T, int64_t D, int64_t N, int x_dt, int
     l.L = kMcQ;
   } else {  // general N: channel tiles walking T, checkpoint every kGnCK rows
     l.V = 1;
-    l.CH = bwd ? gn_bwd_dt(np_of(N)) : kGnDT;  // the backward kernel's tiles (dB/dC partials)
+    l.CH = bwd ? kGnBwdDT : kGnDT;  // the backward kernel's tiles (dB/dC partials)
     l.L = kGnCK;
   }
   l.K = (int)((T + l.L - 1) / l.L);
@@ -2486,15 +2293,14 @@ Layout make_layout(int64_t batch, int64_t T, int64_t D, int64_t N, int x_dt, int
   // sub-blocks per segment must be a multiple of this (the matrix-core
   // forward: kMcSegUnit, whatever the checkpoint interval)
   const int unit = (mc && !bwd) ? kMcSegUnit : 1;
-  if (N > 1 && l.n_tiles > 0 && l.K > 0 && (mc || bwd || !gq_ok(N, batch, D))) {
+  if (N > 1 && l.n_tiles > 0 && l.K > 0) {
     if (mc) {
       l.seg_sc = mc_seg_sc(l.n_tiles, l.K, bwd, unit);
     } else {
       // forward (lanes over channels): about kGcTargetWaves waves; backward
       // (8-wave workgroups over 64 channels): about kGnTargetWgs workgroups
       const int64_t per_seg = bwd ? l.n_tiles : batch * ((D + 63) / 64);
-      // (the 8-wave NP = 128 backward runs one workgroup per CU: 1024)
-      const int64_t target = bwd ? (np_of(N) <= 64 ? kGnTargetWgs : 1024) : kGcTargetWaves;
+      const int64_t target = bwd ? kGnTargetWgs : kGcTargetWaves;
       int64_t want = (target + per_seg - 1) / per_seg;
       if (want > l.K) want = l.K;
       if (want < 1) want = 1;
@@ -2577,51 +2383,22 @@ int np_of(int64_t N) {
 }
 
 
-// Backward workgroup shape per NP: 32 channels in 4 waves (three workgroups
-// fit a CU: 149 VGPRs, 54 KB of LDS) up to NP = 64; 64 channels in 8 waves
-// at NP = 128, whose B/C tiles would not leave room for three.
-int gn_bwd_dt(int np) { return np <= 64 ? 32 : 64; }
-int gn_bwd_waves(int np) { return np <= 64 ? 4 : 8; }
-
 gn_bwd_t pick_gn_bwd(int np) {
   switch (np) {
     case 2: return gn_bwd_kernel<2, 32, 4>;
     case 4: return gn_bwd_kernel<4, 32, 4>;
-    case 8: return gn_bwd_kernel<8, 32, 4>;
-    case 16: return gn_bwd_kernel<16, 32, 4>;
-    case 32: return gn_bwd_kernel<32, 32, 4>;
-    case 64: return gn_bwd_kernel<64, 32, 4>;
-    default: return gn_bwd_kernel<128, 64, 8>;
+    default: return gn_bwd_kernel<8, 32, 4>;
   }
 }
 
 // Workgroups per time segment of the general-N forward.
 int64_t gc_tiles(int64_t batch, int64_t D) { return batch * ((D + kGcCH - 1) / kGcCH); }
 
-// The forward without time segments (gq_fwd_kernel): 16 <= NP <= 64 and a
-// grid that fills the GPU.
-int gq_channels(int64_t N) { return 64 / (np_of((int)N) / 4) * kGqW; }
-bool gq_ok(int64_t N, int64_t batch, int64_t D) {
-  const int np = np_of((int)N);
-  return N > 1 && np >= 16 && np <= 64 && batch * ((D + gq_channels(N) - 1) / gq_channels(N)) >= kGqMinWgs;
-}
-gn_fwd_t pick_gq_fwd(int np) {
-  switch (np) {
-    case 16: return gq_fwd_kernel<16>;
-    case 32: return gq_fwd_kernel<32>;
-    default: return gq_fwd_kernel<64>;
-  }
-}
-
 gn_fwd_t pick_gc_fwd(int np, bool map) {
   switch (np) {
     case 2: return map ? gc_fwd_kernel<2, true> : gc_fwd_kernel<2, false>;
     case 4: return map ? gc_fwd_kernel<4, true> : gc_fwd_kernel<4, false>;
-    case 8: return map ? gc_fwd_kernel<8, true> : gc_fwd_kernel<8, false>;
-    case 16: return map ? gc_fwd_kernel<16, true> : gc_fwd_kernel<16, false>;
-    case 32: return map ? gc_fwd_kernel<32, true> : gc_fwd_kernel<32, false>;
-    case 64: return map ? gc_fwd_kernel<64, true> : gc_fwd_kernel<64, false>;
-    default: return map ? gc_fwd_kernel<128, true> : gc_fwd_kernel<128, false>;
+    default: return map ? gc_fwd_kernel<8, true> : gc_fwd_kernel<8, false>;
   }
 }
 
@@ -2631,11 +2408,7 @@ gn_map_t pick_gn_bwd_map(int np) {
   switch (np) {
     case 2: return gn_bwd_map_kernel<2>;
     case 4: return gn_bwd_map_kernel<4>;
-    case 8: return gn_bwd_map_kernel<8>;
-    case 16: return gn_bwd_map_kernel<16>;
-    case 32: return gn_bwd_map_kernel<32>;
-    case 64: return gn_bwd_map_kernel<64>;
-    default: return gn_bwd_map_kernel<128>;
+    default: return gn_bwd_map_kernel<8>;
   }
 }
 
@@ -2715,13 +2488,35 @@ size_t naju_scan_workspace_bytes(int64_t batch, int64_t T, int64_t D, int64_t N,
 
 namespace {
 
+// The matrix-core passes over N > 64 run as halves of the entries, 0 .. 63 and
+// 64 .. N - 1: their number, and the arguments of half h (every pointer into an
+// array that has the entries innermost moved to its first one).
+int mc_halves(int64_t N) { return N > kMcHalf ? 2 : 1; }
+ScanArgs mc_half_args(const ScanArgs& a, int h, int bc_dt) {
+  ScanArgs r = a;
+  if (mc_halves(a.N) == 1) return r;
+  const int n0 = h * kMcHalf;
+  auto at = [n0](float* p) { return p ? p + n0 : nullptr; };
+  r.N = h ? a.N - kMcHalf : kMcHalf;
+  r.Bm = (const char*)a.Bm + n0 * dsize(bc_dt);
+  r.Cm = (const char*)a.Cm + n0 * dsize(bc_dt);
+  r.ckpt = at(a.ckpt);
+  r.segZ = at(a.segZ);
+  r.seg0 = at(a.seg0);
+  r.dh0 = at(a.dh0);
+  r.partB = at(a.partB);
+  r.partC = at(a.partC);
+  return r;
+}
+
 // B / C (or dB / dC) with rows ld elements apart: ld = N always; another
 // ld only on the matrix-core path (9 <= N <= 64), a multiple of 4 with both
 // pointers aligned to four elements (the staging loads of the kernels).
 int check_bc_ld(const void* p, const void* q, int64_t N, int dt, int64_t ld, bool bwd) {
   if (ld == N) return NAJU_OK;
   if (ld < N) return fail(NAJU_ERR_INVALID, "B / C row stride (%lld) must be >= N (%lld)", (long long)ld, (long long)N);
-  if (N <= 1 || !use_mc(N, bwd))
+  (void)bwd;
+  if (!mc_ext_ok(N))
     return fail(NAJU_ERR_UNSUPPORTED, "a B / C row stride other than N is served at 9 <= N <= 64 only");
   // the kernels address a sub-block's rows with 32-bit offsets
   if (ld > (1 << 24)) return fail(NAJU_ERR_UNSUPPORTED, "B / C row stride (%lld) above 2^24", (long long)ld);
@@ -2787,6 +2582,7 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
   a.T = T;
   a.D = D;
   a.ldbc = ldbc;
+  a.ldn = N;
   a.N = (int)N;
   a.batch = (int)batch;
   a.bc_dt = bc_dtype;
@@ -2809,7 +2605,8 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
       if ((int64_t)l.n_tiles * l.nseg > 0x7fffffff) return fail(NAJU_ERR_UNSUPPORTED, "problem too large");
       hipError_t e = hipSuccess;
       if (l.nseg > 1) {
-        e = mc_map_launch(a, false, x_dtype, gate_dtype, st);
+        for (int h = 0; e == hipSuccess && h < mc_halves(N); ++h)
+          e = mc_map_launch(mc_half_args(a, h, bc_dtype), false, x_dtype, gate_dtype, st);
         if (e == hipSuccess) {
           const int64_t n = (int64_t)a.batch * a.D * a.N;
           hipLaunchKernelGGL(gn_seg_carry_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, 1);
@@ -2817,16 +2614,6 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
         }
       }
       if (e == hipSuccess) e = mc_fwd_launch(a, x_dtype, gate_dtype, y_dt, st);
-      if (e != hipSuccess) return fail(NAJU_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
-      return NAJU_OK;
-    }
-    if (gq_ok(N, batch, D)) {
-      // one workgroup per (batch row, channel group), over all of T
-      const int64_t grid = batch * ((D + gq_channels(N) - 1) / gq_channels(N));
-      if (grid > 0x7fffffff) return fail(NAJU_ERR_UNSUPPORTED, "problem too large");
-      hipLaunchKernelGGL(pick_gq_fwd(np_of(N)), dim3((unsigned)grid), dim3(64 * kGqW), 0, st, a, x_dtype, gate_dtype,
-                         y_dt);
-      const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail(NAJU_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
       return NAJU_OK;
     }
@@ -2958,7 +2745,7 @@ int naju_scan_fwd_noalloc(const void* u, const void* f_logit, const void* i_logi
 int check_gate_ext(const void* dfl, const void* dil, int64_t N, int64_t D, int64_t ldg, int dg_req, int dg_dt,
                    bool sums) {
   if (ldg == D && dg_req < 0 && !sums) return NAJU_OK;
-  if (N <= 1 || !use_mc(N, true))
+  if (!mc_ext_ok(N))
     return fail(NAJU_ERR_UNSUPPORTED, "gate-gradient strides, types and sums are served at 9 <= N <= 64");
   if (ldg < D) return fail(NAJU_ERR_INVALID, "dfl / dil row stride (%lld) must be >= D (%lld)", (long long)ldg,
                            (long long)D);
@@ -3050,6 +2837,7 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
   a.T = T;
   a.D = D;
   a.ldbc = ldbc;
+  a.ldn = N;
   a.ldg = ldg;
   a.N = (int)N;
   a.batch = (int)batch;
@@ -3090,22 +2878,26 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
       }
       a.ck_rows = kMcQ;
       a.Kc = (int)((T + kMcQ - 1) / kMcQ);
+      a.half = (float*)(ws + l.off_half);
+      const int nh = mc_halves(N);
       if (e == hipSuccess && l.nseg > 1) {
-        e = mc_map_launch(a, true, x_dtype, gate_dtype, st);
+        for (int h = 0; e == hipSuccess && h < nh; ++h)
+          e = mc_map_launch(mc_half_args(a, h, bc_dtype), true, x_dtype, gate_dtype, st);
         if (e == hipSuccess) {
           const int64_t n = (int64_t)a.batch * a.D * a.N;
           hipLaunchKernelGGL(gn_seg_carry_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, -1);
           e = hipGetLastError();
         }
       }
-      if (e == hipSuccess) e = mc_bwd_launch(a, x_dtype, gate_dtype, du_dt, dg_dt, st);
+      for (int h = 0; e == hipSuccess && h < nh; ++h)
+        e = mc_bwd_launch(mc_half_args(a, h, bc_dtype), nh > 1 ? h + 1 : 0, x_dtype, gate_dtype, du_dt, dg_dt, st);
       if (e != hipSuccess) return fail(NAJU_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
       goto fold;
     }
     rc = gn_segments(a, l, x_dtype, gate_dtype, true, st);
     if (rc) return rc;
     hipLaunchKernelGGL(pick_gn_bwd(np_of(N)), dim3((unsigned)((int64_t)l.n_tiles * l.nseg)),
-                       dim3(64 * gn_bwd_waves(np_of(N))), 0, st,
+                       dim3(64 * kGnBwdW), 0, st,
                        a, x_dtype, gate_dtype, du_dt, dg_dt);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(NAJU_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));

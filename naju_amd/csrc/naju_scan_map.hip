@@ -357,8 +357,8 @@ __global__ __launch_bounds__(64 * kMapMaxW) __attribute__((amdgpu_waves_per_eu(3
     const int n = 16 * m + 4 * g;
 #pragma unroll
     for (int c = 0; c < V; ++c) {
-      float* p = a.segZ + (o + c) * N + n;
-      if ((N & 3) == 0) {
+      float* p = a.segZ + (o + c) * a.ldn + n;
+      if (((N | a.ldn) & 3) == 0) {
         if (n < N) *(f4_t*)p = z[c];
       } else {
 #pragma unroll

@@ -1,5 +1,6 @@
 // naju_scan_mc.hip -- chunked matrix-core kernels of the Naju scan for
-// 9 <= N <= 64 (the mixer's d_state = 64 among them).
+// 9 <= N <= 128 (the mixer's d_state = 64 among them; the backward above 64 in
+// two halves).
 //
 // Recurrence (reference naju/scan.py:15-19): x_t = f_t x_{t-1} + w_t B_t,
 // y_t = C_t . x_t + D u_t, f = sigmoid(f_logit), w = sigmoid(i_logit) u.
@@ -141,13 +142,15 @@ struct McBC {
 // One sub-block's inputs as a lane loads them: row rho of the wave's 16
 // channels cq .. cq+3 (clamped in bounds; rows past T and channels past D
 // become the neutral step when the gates are formed), and the workgroup's B
-// (and C) groups of four entries: thread tid < 4 NP takes row (4 tid) / NP,
-// entries n0 .. n0+3 with n0 = (4 tid) % NP.
+// (and C) groups of four entries: group id = tid (tid + 256 too at
+// NP = 128) < 4 NP is row (4 id) / NP, entries n0 .. n0+3 with n0 = (4 id) % NP.
 template <int NP, bool RECOMP, typename TU, typename TG, typename TB>
 struct McIn {
+  // B / C groups per thread: one up to NP = 64, two at NP = 128
+  static constexpr int NG = 4 * NP > 64 * kMcW ? 4 * NP / (64 * kMcW) : 1;
   Raw4<TG> f, i;
   Raw4<TU> u;
-  Raw4<TB> b, c;
+  Raw4<TB> b[NG], c[NG];
 
   __device__ __forceinline__ void load(const ScanArgs& a, int b_row, int64_t t0, int64_t dw, int rho, int cq,
                                        int tid, bool vec) {
@@ -171,20 +174,23 @@ struct McIn {
       ld4r_at<TG>((const TG*)a.il + base, o, i);
       ld4r_at<TU>((const TU*)a.u + base, o, u);
     }
-    if (tid < 4 * NP) {
+#pragma unroll
+    for (int q = 0; q < NG; ++q) {
+      const int id = tid + q * 64 * kMcW;
+      if (id >= 4 * NP) continue;
       const int N = a.N;
-      const int row = (4 * tid) / NP, n0 = (4 * tid) % NP;
+      const int row = (4 * id) / NP, n0 = (4 * id) % NP;
       const int64_t bb = ((int64_t)b_row * T + t0) * a.ldbc;  // (t0, 0), uniform
       const uint32_t ro = (uint32_t)((row < rows ? row : rows - 1) * a.ldbc);
       if (N == NP) {
-        ld4r<TB>((const TB*)a.Bm + bb, ro + n0, b);
-        if constexpr (!RECOMP) ld4r<TB>((const TB*)a.Cm + bb, ro + n0, c);
+        ld4r<TB>((const TB*)a.Bm + bb, ro + n0, b[q]);
+        if constexpr (!RECOMP) ld4r<TB>((const TB*)a.Cm + bb, ro + n0, c[q]);
       } else {
         uint32_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = ro + (uint32_t)(n0 + e < N ? n0 + e : N - 1);
-        ld4r_at<TB>((const TB*)a.Bm + bb, o, b);
-        if constexpr (!RECOMP) ld4r_at<TB>((const TB*)a.Cm + bb, o, c);
+        ld4r_at<TB>((const TB*)a.Bm + bb, o, b[q]);
+        if constexpr (!RECOMP) ld4r_at<TB>((const TB*)a.Cm + bb, o, c[q]);
       }
     }
   }
@@ -200,22 +206,27 @@ struct McIn {
 #pragma unroll
     for (int k = 0; k < Raw4<TU>::NW; ++k) asm volatile("" : "+v"(u.w[k]));
 #pragma unroll
-    for (int k = 0; k < Raw4<TB>::NW; ++k) asm volatile("" : "+v"(b.w[k]), "+v"(c.w[k]));
+    for (int q = 0; q < NG; ++q)
+#pragma unroll
+      for (int k = 0; k < Raw4<TB>::NW; ++k) asm volatile("" : "+v"(b[q].w[k]), "+v"(c[q].w[k]));
   }
 
   // B (and C) into LDS buffer buf; zeros past T and past N. (Each 16 lanes
   // read one 64-entry row of B and C, coalesced; the backward's staging takes
   // another lane map, which the forward measured slower with.)
   __device__ __forceinline__ void stage(McBC<NP, RECOMP>& sh, int buf, const ScanArgs& a, int64_t t0, int tid) const {
-    if (tid < 4 * NP) {
-      const int row = (4 * tid) / NP, n0 = (4 * tid) % NP;
+#pragma unroll
+    for (int q = 0; q < NG; ++q) {
+      const int id = tid + q * 64 * kMcW;
+      if (id >= 4 * NP) continue;
+      const int row = (4 * id) / NP, n0 = (4 * id) % NP;
       const bool rok = t0 + row < a.T;
       float vb[4], vc[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const bool ok = rok && n0 + e < a.N;
-        vb[e] = ok ? b.get(e) : 0.f;
-        if constexpr (!RECOMP) vc[e] = ok ? c.get(e) : 0.f;
+        vb[e] = ok ? b[q].get(e) : 0.f;
+        if constexpr (!RECOMP) vc[e] = ok ? c[q].get(e) : 0.f;
         sh.Bt[buf][n0 + e][4 * (row & 3) + (row >> 2)] = vb[e];
       }
       if constexpr (!RECOMP) {
@@ -226,19 +237,19 @@ struct McIn {
   }
 };
 
-// The wave's 16 channels x 64 state entries (X in the D layout: lane (j, g)
+// The wave's 16 channels x 16 MT state entries (X in the D layout: lane (j, g)
 // value r of X[m] is entry 16m + 4g + r of channel j), stored as the
-// contiguous 4 KB run [channel][entry] at ckw. Stored straight from the D
+// contiguous run [channel][entry] at ckw. Stored straight from the D
 // layout, each store would write sixteen 64-byte pieces; transposed through
 // tt (16 x 36 floats of the wave's own LDS, free at the call), each store
-// writes eight whole 128-byte lines. Two halves of 32 entries per channel.
-// (MT = 4 only: the callers test N == 64)
+// writes eight whole 128-byte lines, 32 entries per channel at a time.
+// (MT = 4 or 8: the callers test N == 16 MT)
 template <int MT>
-__device__ __forceinline__ void store_state64(float* ckw, const f4_t (&X)[MT], float* tt, int j, int g, int lane) {
+__device__ __forceinline__ void store_state_lines(float* ckw, const f4_t (&X)[MT], float* tt, int j, int g, int lane) {
   static_assert(16 * 36 <= 2 * 16 * TP, "the transposition fits a wave's two gate tiles");
-  if constexpr (MT == 4) {
+  if constexpr (MT >= 4) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < MT / 2; ++h) {
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int k = 0; k < 2; ++k)
@@ -249,7 +260,7 @@ __device__ __forceinline__ void store_state64(float* ckw, const f4_t (&X)[MT], f
       for (int s2 = 0; s2 < 2; ++s2) {
         const int c = 8 * s2 + (lane >> 3), q = 4 * (lane & 7);
         const float4 v = *(const float4*)(tt + c * 36 + q);
-        *(float4*)(ckw + c * 64 + 32 * h + q) = v;
+        *(float4*)(ckw + c * (16 * MT) + 32 * h + q) = v;
       }
     }
     asm volatile("" ::: "memory");
@@ -266,7 +277,7 @@ __device__ __forceinline__ void store_state64(float* ckw, const f4_t (&X)[MT], f
 // interval), into a.ckpt; otherwise y, the checkpoint and hT from the
 // entering state (h0, or seg0 when T is split into segments).
 template <int NP, bool RECOMP, typename TU, typename TG, typename TB>
-__global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) void mc_fwd_kernel(const ScanArgs a, int y_dt) {
+__global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <= 64 ? 3 : 2))) void mc_fwd_kernel(const ScanArgs a, int y_dt) {
   constexpr int MT = NP / 16;  // 16-entry tiles of the state index
   using In = McIn<NP, RECOMP, TU, TG, TB>;
   __shared__ __align__(16) McBC<NP, RECOMP> sh;
@@ -475,8 +486,8 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
         nxt.stage(sh, buf ^ 1, a, t0 + Q, tid);
       }
       // the state entering this sub-block is the backward's checkpoint
-      if (NP == 64 && N == 64 && a.ckpt && dw + 16 <= D && sb % ck_sb == 0) {
-        store_state64(a.ckpt + (((int64_t)b * a.Kc + sb / ck_sb) * D + dw) * N, X, &s_t[wv][0][0][0], j, g, lane_l);
+      if (NP >= 64 && N == NP && a.ckpt && dw + 16 <= D && sb % ck_sb == 0) {
+        store_state_lines(a.ckpt + (((int64_t)b * a.Kc + sb / ck_sb) * D + dw) * N, X, &s_t[wv][0][0][0], j, g, lane_l);
       } else if (a.ckpt && dok && sb % ck_sb == 0) {
         float* ck = a.ckpt + (((int64_t)b * a.Kc + sb / ck_sb) * D + d) * N;
 #pragma unroll
@@ -524,10 +535,10 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(3))) 
         }
       }
     } else {
-      if (NP == 64 && N == 64 && dw + 16 <= D) {
+      if (NP >= 64 && N == NP && dw + 16 <= D) {
         // the state entering sb, as the scan's checkpoint holds it (the
         // wave's gate tiles are free: f and w are in registers)
-        store_state64(a.ckpt + (((int64_t)b * a.Kc + sb) * D + dw) * N, X, &s_t[wv][0][0][0], j, g, lane_l);
+        store_state_lines(a.ckpt + (((int64_t)b * a.Kc + sb) * D + dw) * N, X, &s_t[wv][0][0][0], j, g, lane_l);
       } else if (dok) {
         // the state entering sb, as the scan's checkpoint holds it
         float* ck = a.ckpt + (((int64_t)b * a.Kc + sb) * D + d) * N;
@@ -670,7 +681,7 @@ struct McInB {
       const int row = tid % kMcQ, n0 = 4 * (tid / kMcQ);
       const int64_t bb = ((int64_t)b_row * T + t0) * a.ldbc;
       const uint32_t ro = (uint32_t)((row < rows ? row : rows - 1) * a.ldbc);
-      if (N == NP) {
+      if (N == NP && (a.ldbc & 3) == 0) {
         ld4r<TB>((const TB*)a.Cm + bb, ro + n0, c);
         ld4r<TB>((const TB*)a.Bm + bb, ro + n0, b);
       } else {
@@ -769,12 +780,12 @@ __device__ __forceinline__ void wr4(float* p, float a0, float a1, float a2, floa
 template <int MT>
 __device__ __forceinline__ void load_ckpt(f4_t (&x)[MT], const ScanArgs& a, int b, int sb, int64_t dcl, int g) {
   const int N = a.N;
-  const float* ck = a.ckpt + ((int64_t)b * a.Kc + sb) * a.D * N;  // uniform
-  const uint32_t co = (uint32_t)(dcl * N);
+  const float* ck = a.ckpt + ((int64_t)b * a.Kc + sb) * a.D * a.ldn;  // uniform
+  const uint32_t co = (uint32_t)(dcl * a.ldn);
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     const int n = 16 * m + 4 * g;
-    if ((N & 3) == 0) {
+    if (((N | a.ldn) & 3) == 0) {
       const float4 v = *(const float4*)(ck + (co + (uint32_t)(n < N ? n : N - 4)));
       x[m][0] = v.x, x[m][1] = v.y, x[m][2] = v.z, x[m][3] = v.w;
     } else {
@@ -809,7 +820,15 @@ __device__ __forceinline__ void store_row4(void* p, uint32_t o, const float (*tl
   }
 }
 
-template <int NP, typename TU, typename TG, typename TB>
+// HALF = 0: all of N. N > 64 runs as two launches over halves of the entries,
+// since a second set of 64 entries of X and ghat per channel does not fit the
+// registers and the LDS beside the first: dB, dC, dh0 and the states are the
+// half's own, and what is summed over the entries, dws and xbar . x, the first
+// (HALF = 1) leaves in a.half and the second (HALF = 2) adds before it forms
+// du, dfl and dil. (bf16 4 x 2048 x 1024, N = 128: 161 + 172 us for the two
+// halves against 744 us on the vector units; the forward, whole at NP = 128,
+// 104 us against 522.)
+template <int NP, int HALF, typename TU, typename TG, typename TB>
 __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, int du_dt, int dg_dt) {
   constexpr int MT = NP / 16;
   constexpr int P = NP + 4;
@@ -841,13 +860,13 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
   // adjoint carry in the D layout: gh[m][r] = entry 16m + 4g + r of channel j
   f4_t gh[MT];
   {
-    const float* gin = a.nseg > 1 ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * N : nullptr;
+    const float* gin = a.nseg > 1 ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * a.ldn : nullptr;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int n = 16 * m + 4 * g + r;
-        gh[m][r] = (gin && dok && n < N) ? gin[d * N + n] : 0.f;
+        gh[m][r] = (gin && dok && n < N) ? gin[d * a.ldn + n] : 0.f;
       }
     // loaded before the loop, waited for here (as McIn::settle)
 #pragma unroll
@@ -914,6 +933,14 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       }
     }
     __syncthreads();  // staging visible
+    // the first half's terms, used at this sub-block's outputs (issued before
+    // the next sub-block's loads, so that waiting for them waits for no others)
+    float* hp_p = nullptr;
+    f4_t hdws = {0.f, 0.f, 0.f, 0.f}, hxx = hdws;
+    if constexpr (HALF != 0) {
+      hp_p = a.half + (((int64_t)b * KS + sb) * D + dcl) * (2 * Q) + 8 * g;
+      if constexpr (HALF == 2) hdws = *(const f4_t*)hp_p, hxx = *(const f4_t*)(hp_p + 4);
+    }
     if (sb - 1 >= sb0) {
       nxt.load(a, b, t0 - Q, dw, rho, cq, tid, vec);
       load_ckpt<MT>(xn, a, b, sb - 1, dcl, g);
@@ -1241,13 +1268,18 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float f_o = Tf[j][4 * r + g], i_o = Ti[j][4 * r + g], w_o = Tw[j][4 * r + g];
-        const float dws = fmaf(pe[r], bg[r], V1[r]);
-        const float xx = fmaf(pf[r], V2[r], A3[r]) + pe[r] * fmaf(pf[r], gX, V3[r]);
+        float dws = fmaf(pe[r], bg[r], V1[r]);
+        float xx = fmaf(pf[r], V2[r], A3[r]) + pe[r] * fmaf(pf[r], gX, V3[r]);
+        q1[r] = pfdy[r];
+        q2[r] = w_o * pe[r];
+        if constexpr (HALF == 1) {
+          hdws[r] = dws, hxx[r] = xx;
+          continue;
+        }
+        if constexpr (HALF == 2) dws += hdws[r], xx += hxx[r];
         const float dfl = f_o == 0.f ? 0.f : (1.f - f_o) * fmaf(-w_o, dws, xx);
         const float du = fmaf(i_o, dws, Dv * dy_o[r]);
         const float dil = (1.f - i_o) * (dws * w_o);
-        q1[r] = pfdy[r];
-        q2[r] = w_o * pe[r];
         sgf += dfl;
         sgi += dil;
         Tf[j][4 * r + g] = dfl;
@@ -1263,7 +1295,10 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
         for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(xn[m]));
       }
-      if (rok && ncq > 0) {
+      if constexpr (HALF == 1) {
+        if (dok) *(f4_t*)hp_p = hdws, *(f4_t*)(hp_p + 4) = hxx;
+      }
+      if (HALF != 1 && rok && ncq > 0) {
         const int64_t ob = ((int64_t)b * T + t0) * D;  // uniform
         const uint32_t o = (uint32_t)(rho * D + dw + cq);
         void* du_p = a.du ? (char*)a.du + ob * (du_dt == NAJU_DTYPE_F32 ? 4 : 2) : nullptr;
@@ -1375,12 +1410,12 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         float* dst = qd == 0 ? a.partC : a.partB;
         const int n = 16 * m + 4 * g;
         if (dst && t0 + j < T && n < N) {
-          const int64_t btn = (int64_t)a.batch * T * N;
-          float* q = dst + (int64_t)dtile * btn + ((int64_t)b * T + t0) * N;  // uniform
-          const uint32_t o = (uint32_t)(j * N + n);
+          const int64_t btn = (int64_t)a.batch * T * a.ldn;
+          float* q = dst + (int64_t)dtile * btn + ((int64_t)b * T + t0) * a.ldn;  // uniform
+          const uint32_t o = (uint32_t)(j * (int)a.ldn + n);
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc[r] += hp[r];
-          if ((N & 3) == 0) {
+          if (((N | a.ldn) & 3) == 0) {
             *(float4*)(q + o) = make_float4(acc[0], acc[1], acc[2], acc[3]);
           } else {
 #pragma unroll
@@ -1406,7 +1441,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int n = 16 * m + 4 * g + r;
-          if (n < N) a.dh0[((int64_t)b * D + d) * N + n] = gh[m][r];
+          if (n < N) a.dh0[((int64_t)b * D + d) * a.ldn + n] = gh[m][r];
         }
     }
     // dD of the segment: lanes with the same cq hold the same four channels
@@ -1419,14 +1454,14 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       v += __shfl_xor(v, 32, 64);
       dDacc[e] = v;
     }
-    if (a.partD && rho == 0) {
+    if (HALF != 1 && a.partD && rho == 0) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (e < ncq) a.partD[((int64_t)b * a.nseg + seg) * D + dw + cq + e] = dDacc[e];
     }
     // the gate gradients' sums of the segment: channel j's four lane groups
     // added (groups 0 + 1, 2 + 3, then the pairs)
-    if (a.partG) {
+    if (HALF != 1 && a.partG) {
       sgf += __shfl_xor(sgf, 16, 64);
       sgi += __shfl_xor(sgi, 16, 64);
       sgf += __shfl_xor(sgf, 32, 64);
@@ -1440,7 +1475,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
   }
 }
 
-int np16(int64_t N) { return N <= 16 ? 16 : (N <= 32 ? 32 : 64); }
+int np16(int64_t N) { return N <= 16 ? 16 : (N <= 32 ? 32 : (N <= 64 ? 64 : 128)); }
 
 }  // namespace
 
@@ -1451,7 +1486,8 @@ mc_fwd_t pick_fwd_np(int np, bool rec) {
   switch (np) {
     case 16: return rec ? mc_fwd_kernel<16, true, TU, TG, TB> : mc_fwd_kernel<16, false, TU, TG, TB>;
     case 32: return rec ? mc_fwd_kernel<32, true, TU, TG, TB> : mc_fwd_kernel<32, false, TU, TG, TB>;
-    default: return rec ? mc_fwd_kernel<64, true, TU, TG, TB> : mc_fwd_kernel<64, false, TU, TG, TB>;
+    case 64: return rec ? mc_fwd_kernel<64, true, TU, TG, TB> : mc_fwd_kernel<64, false, TU, TG, TB>;
+    default: return mc_fwd_kernel<128, false, TU, TG, TB>;  // (no checkpoint intervals at N > 64)
   }
 }
 
@@ -1466,19 +1502,20 @@ mc_fwd_t pick_fwd_u(int g_dt, int bc_dt, int np, bool rec) {
 typedef void (*mc_bwd_t)(ScanArgs, int, int);
 
 template <typename TU, typename TG, typename TB>
-mc_bwd_t pick_bwd_np(int np) {
+mc_bwd_t pick_bwd_np(int np, int half) {
+  if (half) return half == 1 ? mc_bwd_kernel<64, 1, TU, TG, TB> : mc_bwd_kernel<64, 2, TU, TG, TB>;
   switch (np) {
-    case 16: return mc_bwd_kernel<16, TU, TG, TB>;
-    case 32: return mc_bwd_kernel<32, TU, TG, TB>;
-    default: return mc_bwd_kernel<64, TU, TG, TB>;
+    case 16: return mc_bwd_kernel<16, 0, TU, TG, TB>;
+    case 32: return mc_bwd_kernel<32, 0, TU, TG, TB>;
+    default: return mc_bwd_kernel<64, 0, TU, TG, TB>;
   }
 }
 
 template <typename TU>
-mc_bwd_t pick_bwd_u(int g_dt, int bc_dt, int np) {
+mc_bwd_t pick_bwd_u(int g_dt, int bc_dt, int np, int half) {
   const bool gf = g_dt == NAJU_DTYPE_F32, bf = bc_dt == NAJU_DTYPE_F32;
-  if (gf) return bf ? pick_bwd_np<TU, float, float>(np) : pick_bwd_np<TU, float, TU>(np);
-  return bf ? pick_bwd_np<TU, TU, float>(np) : pick_bwd_np<TU, TU, TU>(np);
+  if (gf) return bf ? pick_bwd_np<TU, float, float>(np, half) : pick_bwd_np<TU, float, TU>(np, half);
+  return bf ? pick_bwd_np<TU, TU, float>(np, half) : pick_bwd_np<TU, TU, TU>(np, half);
 }
 
 hipError_t mc_fwd_launch(const ScanArgs& a, int x_dt, int g_dt, int y_dt, hipStream_t st) {
@@ -1493,13 +1530,13 @@ hipError_t mc_fwd_launch(const ScanArgs& a, int x_dt, int g_dt, int y_dt, hipStr
   return hipGetLastError();
 }
 
-hipError_t mc_bwd_launch(const ScanArgs& a, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st) {
+hipError_t mc_bwd_launch(const ScanArgs& a, int half, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st) {
   const unsigned grid = (unsigned)((int64_t)a.n_tiles * a.nseg);
   if (grid == 0) return hipSuccess;
   const int np = np16(a.N);
-  mc_bwd_t k = x_dt == NAJU_DTYPE_F32    ? pick_bwd_np<float, float, float>(np)
-               : x_dt == NAJU_DTYPE_BF16 ? pick_bwd_u<bf16_t>(g_dt, a.bc_dt, np)
-                                         : pick_bwd_u<f16_t>(g_dt, a.bc_dt, np);
+  mc_bwd_t k = x_dt == NAJU_DTYPE_F32    ? pick_bwd_np<float, float, float>(np, half)
+               : x_dt == NAJU_DTYPE_BF16 ? pick_bwd_u<bf16_t>(g_dt, a.bc_dt, np, half)
+                                         : pick_bwd_u<f16_t>(g_dt, a.bc_dt, np, half);
   hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kMcWB), 0, st, a, du_dt, dg_dt);
   return hipGetLastError();
 }

@@ -1,6 +1,7 @@
 // scan_internal.h -- definitions shared by the scan's translation units
 // (naju_scan.hip: the N = 1 kernels, the direct general-N kernels and the C
-// ABI; naju_scan_mc.hip: the chunked matrix-core kernels for 9 <= N <= 64).
+// ABI; naju_scan_mc.hip, naju_scan_map.hip: the chunked matrix-core kernels for
+// 9 <= N <= 128).
 // Internal to the library; not part of the C ABI.
 #ifndef NAJU_SCAN_INTERNAL_H
 #define NAJU_SCAN_INTERNAL_H
@@ -97,6 +98,12 @@ struct ScanArgs {
   int64_t D;
   int64_t ldbc;  // elements between rows of B and C (N unless strided; the matrix-core path only)
   int64_t ldg;   // elements between rows of dfl and dil (D unless strided; the matrix-core backward only)
+  // N > 64 backward on the matrix cores: it runs the entries in two halves of
+  // at most 64 (N: the half's entries), each with its own pointers into the
+  // arrays below; ldn is the whole N, the entries between channels of ckpt,
+  // segZ, seg0 and dh0 and between rows of partB / partC.
+  int64_t ldn;
+  float* half;   // N > 64: the first half's terms of dws and xbar . x, [batch][sub-blocks][D][16 rows x 2]
   float* partG;  // [2][batch * nseg][D]: per-segment sums of dfl, dil (matrix-core backward; NULL: none)
   int N;
   int batch;
@@ -207,7 +214,11 @@ constexpr int kMcDTB = 16 * kMcWB;
 constexpr float kMcRatioMin = 0x1p-30f;
 
 // True when the chunked kernels serve this state size.
-inline bool mc_ok(int64_t N) { return N > 8 && N <= 64; }
+inline bool mc_ok(int64_t N) { return N > 8 && N <= 128; }
+// ... with strided B / C, gate-gradient layouts and checkpoint intervals.
+inline bool mc_ext_ok(int64_t N) { return N > 8 && N <= 64; }
+// Entries of the state in the backward's first half at N > 64.
+constexpr int kMcHalf = 64;
 
 // The maps of segments 0 .. nseg-2 (forward) or 1 .. nseg-1 (backward) into
 // segF / segZ (naju_scan_map.hip).
@@ -215,8 +226,10 @@ hipError_t mc_map_launch(const ScanArgs& a, bool bwd, int x_dt, int g_dt, hipStr
 // Forward: the scan from h0 or the carried segment states, or with a.recomp
 // the recompute of the states from a memory-light checkpoint.
 hipError_t mc_fwd_launch(const ScanArgs& a, int x_dt, int g_dt, int y_dt, hipStream_t st);
-// Backward: du, dfl, dil, dh0 and the dB / dC / dD partials.
-hipError_t mc_bwd_launch(const ScanArgs& a, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st);
+// Backward: du, dfl, dil, dh0 and the dB / dC / dD partials. half = 0: all N
+// entries; 1 and 2: the first and the second half of N > 64 (the first leaves
+// its terms in a.half, the second adds them and writes the outputs).
+hipError_t mc_bwd_launch(const ScanArgs& a, int half, int x_dt, int g_dt, int du_dt, int dg_dt, hipStream_t st);
 
 }  // namespace naju_detail
 
