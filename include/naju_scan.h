@@ -263,6 +263,15 @@ int naju_scan_fwd_noalloc(const void* u, const void* f_logit,
 int naju_scan_workspace_status(const void* workspace, void* stream,
                                uint32_t* status);
 
+/* Gives the workspace's status word a mirror: a kernel that records a nonzero
+ * status also stores it at `mirror`, a word of pinned host memory that device
+ * code can write (hipHostMalloc), which the caller may read at any time and
+ * clears itself. Queued on `stream` (one small kernel); holds until the next
+ * such call (NULL: no mirror) or until the workspace is zero-filled. The word
+ * must outlive every call that uses the workspace. No counterpart in the
+ * reference. */
+int naju_scan_set_status_mirror(void* workspace, uint32_t* mirror, void* stream);
+
 /* naju_scan_workspace_status for the static scratch of
  * naju_scan_fwd_noalloc on the current HIP device (synchronises `stream`):
  * reads its status word and, when it is nonzero, clears it and rewinds the

@@ -221,6 +221,20 @@ __global__ void epoch_bump_kernel(uint32_t* hdr) {
   hdr[HDR_EPOCH] = e;
 }
 
+// Records a failure in the status word, and in its mirror in host memory when
+// the workspace has one: a caller sees it there without a copy per call (two
+// 4 us copy launches per training step before).
+__device__ __forceinline__ void set_status(uint32_t* hdr, uint32_t v) {
+  __hip_atomic_store(hdr + HDR_STATUS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t m = (uint64_t)hdr[HDR_MIRROR] | (uint64_t)hdr[HDR_MIRROR + 1] << 32;
+  if (m) __hip_atomic_store((uint32_t*)m, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void set_mirror_kernel(uint32_t* hdr, uint64_t mirror) {
+  hdr[HDR_MIRROR] = (uint32_t)mirror;
+  hdr[HDR_MIRROR + 1] = (uint32_t)(mirror >> 32);
+}
+
 // Workgroup blockIdx.x serves tile blockIdx.x % n_tiles; the chunk comes from
 // that tile's ticket counter, so a tile's chunks are handed out in the order
 // its workgroups start and every chunk a workgroup waits on is already held
@@ -239,7 +253,7 @@ __device__ __forceinline__ uint32_t take_ticket(const ScanArgs& a, int tile, uin
     if (a.tag == 0u) e = __hip_atomic_load(a.hdr + HDR_EPOCH, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t t = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (t == (uint32_t)a.K - 1) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (t >= (uint32_t)a.K) __hip_atomic_store(a.hdr + HDR_STATUS, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t >= (uint32_t)a.K) set_status(a.hdr, 2u);
     *s_ticket = t;
     *s_tag = a.tag != 0u ? a.tag : epoch_tag(e);
   }
@@ -357,7 +371,7 @@ __device__ __forceinline__ bool lb_consume(const ScanArgs& a, LookShared<V, W, P
     }
     if (!done && consumed == 0 && ++idle > a.spin_limit) {
       // Bounded wait exceeded: record it and end with a NaN carry.
-      if (lane == 0) __hip_atomic_store(a.hdr + HDR_STATUS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0) set_status(a.hdr, 1u);
 #pragma unroll
       for (int j = 0; j < V; ++j) out[j] = __builtin_nanf("");
       done = 1;
@@ -391,7 +405,7 @@ __device__ __forceinline__ void wg_look_back(const ScanArgs& a, LookShared<V, W,
     // the host asked every hand-off to give up at once (a test hook): the
     // failure path of an exceeded wait, taken without polling
     if (wv == 0) {
-      if (lane == 0) __hip_atomic_store(a.hdr + HDR_STATUS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0) set_status(a.hdr, 1u);
 #pragma unroll
       for (int j = 0; j < V; ++j) out[j] = __builtin_nanf("");
     }
@@ -2998,6 +3012,17 @@ int naju_scan_workspace_status(const void* workspace, void* stream, uint32_t* st
         hipStreamSynchronize(st) != hipSuccess)
       return fail(NAJU_ERR_LAUNCH, "could not clear the workspace header");
   }
+  return NAJU_OK;
+}
+
+int naju_scan_set_status_mirror(void* workspace, uint32_t* mirror, void* stream) {
+  g_err[0] = 0;
+  if (!workspace) return fail(NAJU_ERR_INVALID, "null workspace pointer");
+  if (!aligned(workspace, 256)) return fail(NAJU_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (!aligned(mirror, 4)) return fail(NAJU_ERR_INVALID, "the mirror must be 4-byte aligned");
+  hipLaunchKernelGGL(set_mirror_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, (uint32_t*)workspace,
+                     (uint64_t)(uintptr_t)mirror);
+  if (hipGetLastError() != hipSuccess) return fail(NAJU_ERR_LAUNCH, "mirror launch failed");
   return NAJU_OK;
 }
 

@@ -53,9 +53,10 @@ __device__ __forceinline__ void st_any(void* p, int dt, int64_t i, float v) {
 // ever overlaps (so its counters, which must start at zero, are only ever
 // written by the ticket logic below): word 0 is the status word; word 1 the
 // device epoch (look-back tags of launches recorded into a HIP graph, see
-// epoch_bump_kernel); tile t's ticket counter is word kCtrBase + t*kCtrStride,
-// t < kMaxTiles.
-enum { HDR_STATUS = 0, HDR_EPOCH = 1 };
+// epoch_bump_kernel); words 2 and 3 the address of the status word's mirror in
+// host memory (0: none); tile t's ticket counter is word
+// kCtrBase + t*kCtrStride, t < kMaxTiles.
+enum { HDR_STATUS = 0, HDR_EPOCH = 1, HDR_MIRROR = 2 };
 constexpr int kCtrBase = 64;
 constexpr int kCtrStride = 4;
 constexpr int kMaxTiles = 1 << 16;

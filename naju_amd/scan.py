@@ -19,12 +19,12 @@ Public surface, mirroring /root/reference/naju/scan.py:
   with this package: the call raises until one is registered under that
   name (the tests register the oracle's loop).
 * ``workspace_status(device=None)`` -- reads (and clears) the status word of
-  the current stream's workspace. After every N = 1 call (the only kernels
-  that hand carries between workgroups) the wrapper copies that word to
-  pinned host memory asynchronously; the next call or backward on the same
-  stream reads the copy once it has landed (no synchronisation) and raises
-  ``NajuScanError`` when a hand-off failed, clearing the word so the
-  workspace is usable again. ``NAJU_CHECK_STATUS=1`` checks synchronously
+  the current stream's workspace. A kernel whose carry hand-off fails (only
+  N = 1 kernels hand carries between workgroups) also stores it in the
+  workspace's mirror word in pinned host memory; the next call or backward on
+  the same stream reads that word (no synchronisation, no copy) and raises
+  ``NajuScanError`` when a hand-off failed, clearing both so the workspace is
+  usable again. ``NAJU_CHECK_STATUS=1`` checks synchronously
   after every call instead.
 * ``register(name="hip", scan_module=None)`` -- inserts ``naju_scan_hip`` into
   the reference's ``naju.scan._BACKEND_CACHE``. ``_get`` returns cached entries
@@ -58,8 +58,9 @@ def _ptr(t):
 class _Workspace:
     """One zero-filled workspace per (device, stream), grown on demand. The
     kernels return it to a reusable state after every call, so it is zeroed
-    only when (re)allocated. Per workspace also a pinned host copy of its
-    status word and the event that marks when the copy has landed."""
+    only when (re)allocated. Per (device, stream) also the pinned host word
+    that mirrors its status word: the tensor that holds it and its view as a
+    C integer."""
 
     def __init__(self):
         self._bufs = {}
@@ -68,9 +69,19 @@ class _Workspace:
     def get(self, device, stream, nbytes):
         key = (device.index, stream)
         buf = self._bufs.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-            self._bufs[key] = buf
+        ent = self._status.get(key)
+        fresh = buf is None or buf.numel() < nbytes
+        if fresh or ent is None:
+            if fresh:
+                buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+                self._bufs[key] = buf
+            if ent is None and not torch.cuda.is_current_stream_capturing():
+                # (pinned memory is not allocated during a capture: a later
+                # call outside it gives the workspace its mirror)
+                word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+                ent = self._status[key] = (word, ctypes.c_uint32.from_address(word.data_ptr()))
+            if ent is not None:
+                _lib.check(_lib.lib().naju_scan_set_status_mirror(buf.data_ptr(), ent[0].data_ptr(), stream))
         return buf
 
 
@@ -96,7 +107,6 @@ def workspace_status(device=None):
     """Status word of the workspace of (device, current stream): 0 healthy,
     1 or 2 after a failed call (then cleared, so the workspace is usable
     again). Synchronises the stream."""
-    import ctypes
     dev = torch.device("cuda", torch.cuda.current_device() if device is None else torch.device(device).index)
     stream = _stream_handle(dev)
     buf = _WS._bufs.get((dev.index, stream))
@@ -104,6 +114,9 @@ def workspace_status(device=None):
         return 0
     st = ctypes.c_uint32(0)
     _lib.check(_lib.lib().naju_scan_workspace_status(buf.data_ptr(), stream, ctypes.byref(st)))
+    ent = _WS._status.get((dev.index, stream))
+    if ent is not None:  # (the stream is idle here)
+        ent[1].value = 0
     return st.value
 
 
@@ -114,40 +127,20 @@ def _check_status(dev):
             raise _lib.NajuScanError(st, _STATUS_MSG.get(st, f"status {st}"))
 
 
-def _watch_status(dev, stream, ws):
-    """Queue an asynchronous copy of the workspace's status word (word 0) to
-    pinned host memory behind the call just issued on `stream`, and mark its
-    landing with an event. Not while the stream is being captured into a
-    graph (the copy would be recorded too)."""
-    if torch.cuda.is_current_stream_capturing():
-        return
-    key = (dev.index, stream)
-    ent = _WS._status.get(key)
-    if ent is None:
-        ent = (torch.zeros(1, dtype=torch.int32, pin_memory=True), torch.cuda.Event())
-        _WS._status[key] = ent
-    ent[0].copy_(ws[:4].view(torch.int32), non_blocking=True)
-    ent[1].record()
-
-
 def _raise_pending(dev, stream):
-    """Raise NajuScanError if the last landed status copy of this stream's
-    workspace is nonzero (a failed hand-off in an earlier call: its outputs
-    were NaN). Does not wait for a copy still in flight: the word stays set
-    on the device until cleared, so a later copy shows it. On raising, the
-    word is cleared (synchronously), so the workspace is usable again.
-    Nothing is queried while the stream is being captured into a graph."""
-    if torch.cuda.is_current_stream_capturing():
-        return
+    """Raise NajuScanError if the mirror of this stream's workspace status is
+    nonzero (a failed hand-off in an earlier call: its outputs were NaN). Does
+    not wait for calls still in flight: a later call sees their failure. On
+    raising, the word is cleared (synchronously), so the workspace is usable
+    again. Nothing is raised while the stream is being captured into a graph
+    (it cannot be synchronised there)."""
     ent = _WS._status.get((dev.index, stream))
-    if ent is None or not ent[1].query():
+    if ent is None or ent[1].value == 0 or torch.cuda.is_current_stream_capturing():
         return
-    st = int(ent[0][0])
-    if st:
-        ent[0].zero_()
-        workspace_status(dev)  # clears the word and rewinds the counters
-        raise _lib.NajuScanError(st, "an earlier scan call on this stream failed: "
-                                 + _STATUS_MSG.get(st, f"status {st}"))
+    st = ent[1].value
+    workspace_status(dev)  # clears the word and its mirror, rewinds the counters
+    raise _lib.NajuScanError(st, "an earlier scan call on this stream failed: "
+                             + _STATUS_MSG.get(st, f"status {st}"))
 
 
 def _norm_inputs(u, f_logit, i_logit, B, C, D_skip, h0, bc_strided=False):
@@ -255,8 +248,6 @@ class NajuScanHip(torch.autograd.Function):
             _lib.check(L.naju_scan_fwd(
                 _ptr(u_), _ptr(fl_), _ptr(il_), _ptr(B_), _ptr(C_), _ptr(D_), _ptr(h0_),
                 _ptr(y), _ptr(ckpt), _ptr(hT), Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel(), stream))
-        if N == 1:
-            _watch_status(dev, stream, ws)
         _check_status(dev)
         if need_grad:
             # du_skip: the skip coefficient of du's D dy term in place of
@@ -352,8 +343,6 @@ class NajuScanHip(torch.autograd.Function):
                 _ptr(u_), _ptr(fl_), _ptr(il_), _ptr(B_), _ptr(C_), _ptr(D_b), _ptr(ckpt), _ptr(dy),
                 _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD), _ptr(dh0),
                 Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel(), stream))
-        if N == 1:
-            _watch_status(dev, stream, ws)
         _check_status(dev)
         grads = [du, dfl, dil, dB, dC, dD]
         if gtgt is not None:

@@ -2,10 +2,9 @@
 
 The N = 1 kernels hand chunk carries between workgroups with bounded waits; a
 wait that gives up writes NaN outputs and sets the workspace's status word.
-naju_scan_hip copies that word to pinned host memory asynchronously after
-each N = 1 call, and the next call (or backward) on the same stream raises
-NajuScanError once the copy has landed, clearing the word so the workspace
-is usable again. The failures are forced from the host with the library's
+The kernel stores that word's mirror in pinned host memory too, and the next
+naju_scan_hip call (or backward) on the same stream that finds it nonzero
+raises NajuScanError, clearing both so the workspace is usable again. The failures are forced from the host with the library's
 NAJU_DEBUG_SPIN_LIMIT=0 test hook (every hand-off gives up at once, every
 kernel still exits normally)."""
 import pytest
@@ -65,7 +64,7 @@ def test_failed_backward_handoff_raises_at_the_next_call(gpu, monkeypatch):
 
 def test_healthy_calls_never_raise(gpu):
     """Many N = 1 calls in a row on one stream without synchronisation: the
-    status copies of healthy calls read 0."""
+    mirror of a healthy workspace stays 0."""
     from naju_amd import naju_scan_hip
     xs, dy = _inputs(gpu, grad=True)
     for _ in range(20):
@@ -74,3 +73,23 @@ def test_healthy_calls_never_raise(gpu):
     torch.cuda.synchronize()
     naju_scan_hip(*xs)
     torch.cuda.synchronize()
+
+
+def test_grown_workspace_keeps_its_mirror(gpu, monkeypatch):
+    """A stream's workspace that is replaced by a larger one reports failures
+    through the same mirror word."""
+    from naju_amd import naju_scan_hip
+    from naju_amd._lib import NajuScanError
+    stream = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(stream), torch.no_grad():
+        for T in (300, 40000):
+            ins = rand_inputs(2, T, 256, 1, seed=T, dtype=torch.float32)
+            xs = [ins[k].to(gpu) for k in NAMES]
+            naju_scan_hip(*xs)
+            monkeypatch.setenv("NAJU_DEBUG_SPIN_LIMIT", "0")
+            naju_scan_hip(*xs)
+            monkeypatch.delenv("NAJU_DEBUG_SPIN_LIMIT")
+            stream.synchronize()
+            with pytest.raises(NajuScanError):
+                naju_scan_hip(*xs)
+            assert bool(torch.isfinite(naju_scan_hip(*xs)).all())
