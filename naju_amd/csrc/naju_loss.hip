@@ -165,15 +165,25 @@ __global__ __launch_bounds__(kThreads) void xent_fwd_kernel(const T* __restrict_
 
 // One workgroup: loss = sum(row_loss) / sum(row_valid), scale = 1 / count,
 // summed in float64 in a fixed order.
+constexpr int kSumU = 8;
 __global__ __launch_bounds__(1024) void xent_mean_kernel(const float* __restrict__ row_loss,
                                                          const float* __restrict__ row_valid, int64_t n,
                                                          float* __restrict__ loss, float* __restrict__ scale) {
   __shared__ double sa[1024], sc[1024];
   const int t = threadIdx.x;
   double a = 0.0, c = 0.0;
-  for (int64_t i = t; i < n; i += 1024) {
-    a += row_loss[i];
-    c += row_valid[i];
+  // kSumU values loaded together, added in order: one workgroup has little
+  // else to hide a load's latency with (16384 rows: 9.6 -> 5.8 us)
+  for (int64_t i = t; i < n; i += 1024 * kSumU) {
+    float l[kSumU], v[kSumU];
+#pragma unroll
+    for (int e = 0; e < kSumU; ++e) {
+      const int64_t k = i + 1024 * e < n ? i + 1024 * e : i;
+      l[e] = row_loss[k], v[e] = row_valid[k];
+    }
+#pragma unroll
+    for (int e = 0; e < kSumU; ++e)
+      if (i + 1024 * e < n) a += l[e], c += v[e];
   }
   sa[t] = a;
   sc[t] = c;
@@ -244,7 +254,7 @@ __device__ __forceinline__ void grad_row(const T* __restrict__ p, TD* __restrict
   }
 }
 
-// grid: n_rows workgroups of kThreads. g = dloss * scale. With if_scaled
+// grid: n_rows workgroups of kThreads (fewer: each takes rows in turn). g = dloss * scale. With if_scaled
 // (the forward already wrote dx for dloss = 1) a workgroup returns at once
 // when dloss is 1.
 template <typename T, typename TD>
@@ -253,12 +263,13 @@ __global__ __launch_bounds__(kThreads) void xent_bwd_kernel(const T* __restrict_
                                                             int64_t ignore, const float* __restrict__ lse,
                                                             const float* __restrict__ scale,
                                                             const float* __restrict__ dloss, TD* __restrict__ dx,
-                                                            int64_t dld, int if_scaled) {
+                                                            int64_t dld, int64_t n_rows, int if_scaled) {
   if (if_scaled && dloss[0] == 1.f) return;
-  const int64_t r = blockIdx.x;
-  const int64_t t = target[r];
-  const float g = (t >= 0 && t < n_cols) ? dloss[0] * scale[0] : __builtin_nanf("");
-  grad_row<T, TD>(x + r * ld, dx + r * dld, t, n_cols, ignore, g, t == ignore ? 0.f : lse[r], threadIdx.x);
+  for (int64_t r = blockIdx.x; r < n_rows; r += gridDim.x) {
+    const int64_t t = target[r];
+    const float g = (t >= 0 && t < n_cols) ? dloss[0] * scale[0] : __builtin_nanf("");
+    grad_row<T, TD>(x + r * ld, dx + r * dld, t, n_cols, ignore, g, t == ignore ? 0.f : lse[r], threadIdx.x);
+  }
 }
 
 // One workgroup: scale = 1 / (number of rows with target != ignore), the
@@ -268,7 +279,14 @@ __global__ __launch_bounds__(1024) void xent_count_kernel(const int64_t* __restr
   __shared__ double sc[1024];
   const int t = threadIdx.x;
   double c = 0.0;
-  for (int64_t i = t; i < n; i += 1024) c += target[i] != ignore ? 1.0 : 0.0;
+  for (int64_t i = t; i < n; i += 1024 * kSumU) {  // as in xent_mean_kernel
+    int64_t v[kSumU];
+#pragma unroll
+    for (int e = 0; e < kSumU; ++e) v[e] = target[i + 1024 * e < n ? i + 1024 * e : i];
+#pragma unroll
+    for (int e = 0; e < kSumU; ++e)
+      if (i + 1024 * e < n) c += v[e] != ignore ? 1.0 : 0.0;
+  }
   sc[t] = c;
   __syncthreads();
   for (int w = 512; w >= 1; w >>= 1) {
@@ -542,8 +560,11 @@ template <typename T, typename TD>
 void launch_bwd(const void* x, int64_t ld, const int64_t* tgt, int64_t rows, int64_t cols, int64_t ignore,
                 const float* lse, const float* scale, const float* dloss, void* dx, int64_t dld, int if_scaled,
                 hipStream_t st) {
-  xent_bwd_kernel<T, TD><<<dim3((unsigned)rows), dim3(kThreads), 0, st>>>((const T*)x, ld, tgt, cols, ignore, lse,
-                                                                          scale, dloss, (TD*)dx, dld, if_scaled);
+  // with if_scaled the kernel mostly has nothing to do: eight workgroups per CU
+  // that take the rows in turn, not one per row (16384 rows: 5.3 -> 5.0 us)
+  const int64_t wgs = if_scaled && rows > 2048 ? 2048 : rows;
+  xent_bwd_kernel<T, TD><<<dim3((unsigned)wgs), dim3(kThreads), 0, st>>>((const T*)x, ld, tgt, cols, ignore, lse, scale,
+                                                                         dloss, (TD*)dx, dld, rows, if_scaled);
 }
 
 template <typename T>

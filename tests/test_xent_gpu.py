@@ -167,3 +167,12 @@ def test_xent_gradient_from_forward_matches_two_passes(gpu, dloss):
     assert torch.equal(g1, dx)
     assert torch.equal(xg.grad, dx + dx)
     assert torch.count_nonzero(dx[::7]) == 0
+
+
+@pytest.mark.parametrize("rows", [2049, 9000])
+def test_xent_many_rows_scaled(gpu, rows):
+    """More rows than the rewriting backward has workgroups, and than one
+    round of the loss's and the count's sums, with some rows ignored."""
+    loss, lr, gx, gr = _case(gpu, rows, 130, torch.float32, seed=rows, ignore_frac=0.2, dloss=0.5)
+    assert abs(float(loss) - float(lr)) <= 2e-6 * abs(float(lr))
+    assert _rel(gx, gr) < 1e-5
