@@ -2187,7 +2187,7 @@ constexpr int kGcTargetWaves = 2048;
 // pass over its rows and a start-up. Segments are a multiple of `unit`
 // sub-blocks long (the forward with a checkpoint interval of unit
 // sub-blocks: every segment then starts where an interval does).
-int mc_seg_sc(int64_t n_tiles, int K, bool bwd, int unit) {
+int mc_seg_search(int64_t n_tiles, int K, bool bwd, int unit) {
   const int64_t min_wg = (int64_t)kCUs * (bwd ? NAJU_MC_BWD_MIN_PER_CU : NAJU_MC_FWD_MIN_PER_CU);
   int best = K;
   int64_t best_cost = -1;
@@ -2201,6 +2201,21 @@ int mc_seg_sc(int64_t n_tiles, int K, bool bwd, int unit) {
     if (wg >= 8 * min_wg) break;
   }
   return best;
+}
+// The last few answers per thread: the search walks up to K candidates, and
+// every call on one shape asks for the same two.
+int mc_seg_sc(int64_t n_tiles, int K, bool bwd, int unit) {
+  struct Entry {
+    int64_t n_tiles;
+    int K, bwd, unit, sc;
+  };
+  static thread_local Entry got[8] = {};
+  static thread_local unsigned next = 0;
+  for (const Entry& e : got)
+    if (e.sc && e.n_tiles == n_tiles && e.K == K && e.bwd == (int)bwd && e.unit == unit) return e.sc;
+  const int sc = mc_seg_search(n_tiles, K, bwd, unit);
+  got[next++ % 8] = Entry{n_tiles, K, (int)bwd, unit, sc};
+  return sc;
 }
 // The backward's workgroups at N <= 8: 32 channels in 4 waves.
 constexpr int kGnBwdDT = 32, kGnBwdW = 4;

@@ -42,6 +42,7 @@ import ctypes
 import os
 
 import torch
+from torch.autograd import forward_ad as _fwd_ad
 
 from naju_amd import _lib
 from naju_amd.gradsink import acc_sink_of, sink_of
@@ -96,7 +97,29 @@ def _flags():
 
 
 def _stream_handle(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+# (checkpoint elements, workspace bytes) by shape, dtypes and flags: pure
+# functions of these (two C calls of 3 us each otherwise); bounded
+_SIZES = {}
+
+
+def _sizes(Bsz, T, D, N, dts, flags):
+    key = (Bsz, T, D, N, dts, flags)
+    got = _SIZES.get(key)
+    if got is None:
+        L = _lib.lib()
+        n = L.naju_scan_ckpt_elems_ex(Bsz, T, D, N, *dts, flags)
+        if n < 0:
+            _lib.check(_lib.ERR_UNSUPPORTED if "interval" in _lib.last_error() else _lib.ERR_INVALID)
+        nbytes = L.naju_scan_workspace_bytes_ex(Bsz, T, D, N, *dts, flags)
+        if nbytes == 0 and Bsz * T * D > 0:
+            _lib.check(_lib.ERR_UNSUPPORTED if "interval" in _lib.last_error() else _lib.ERR_INVALID)
+        if len(_SIZES) >= 256:
+            _SIZES.clear()
+        got = _SIZES[key] = (n, nbytes)
+    return got
 
 
 _STATUS_MSG = {1: "a carry hand-off between workgroups exceeded its bounded wait (outputs are NaN)",
@@ -121,7 +144,7 @@ def workspace_status(device=None):
 
 
 def _check_status(dev):
-    if os.environ.get("NAJU_CHECK_STATUS", "0") not in ("", "0"):
+    if "NAJU_CHECK_STATUS" in os.environ and os.environ["NAJU_CHECK_STATUS"] not in ("", "0"):
         st = workspace_status(dev)
         if st:
             raise _lib.NajuScanError(st, _STATUS_MSG.get(st, f"status {st}"))
@@ -178,8 +201,9 @@ def _check_shapes(u, f_logit, i_logit, B, C, D_skip, h0):
     N = B.shape[-1]
     if h0 is not None and tuple(h0.shape) != (Bsz, D, N):
         raise ValueError(f"h0 must be [B, D, N]=({Bsz}, {D}, {N}), got {tuple(h0.shape)}")
-    devs = {t.device for t in (u, f_logit, i_logit, B, C, D_skip) + ((h0,) if h0 is not None else ())}
-    if len(devs) != 1 or next(iter(devs)).type != "cuda":
+    dev = u.device
+    if (not u.is_cuda or f_logit.device != dev or i_logit.device != dev or B.device != dev or C.device != dev
+            or D_skip.device != dev or (h0 is not None and h0.device != dev)):
         raise ValueError("all scan inputs must live on one GPU device")
     return Bsz, T, D, N
 
@@ -205,56 +229,56 @@ def _bc_pair(B, C, N, in_place=True):
     return bc[..., :N], bc[..., N:], 2 * N
 
 
+def _forward(u, f_logit, i_logit, B, C, D_skip, h0, want_hT, ckpt_rows, need_grad):
+    """The forward call: (y, hT or None, the backward's tensors and sizes or
+    None)."""
+    Bsz, T, D, N = _check_shapes(u, f_logit, i_logit, B, C, D_skip, h0)
+    out_dtype = u.dtype
+    # a memory-light checkpoint interval keeps B and C as a copy, so the
+    # projection output is not held until the backward
+    Bp, Cp, bc_ld = _bc_pair(B, C, N, in_place=int(ckpt_rows or 0) <= 16)
+    u_, fl_, il_, B_, C_, D_, h0_ = _norm_inputs(u, f_logit, i_logit, Bp, Cp, D_skip, h0, bc_ld != N)
+    if bc_ld != N and (B_.data_ptr() != Bp.data_ptr() or C_.data_ptr() != Cp.data_ptr()):
+        # _norm_inputs converted their dtype: contiguous copies after all
+        B_, C_, bc_ld = B_.contiguous(), C_.contiguous(), N
+    dts = (_DT[u_.dtype], _DT[fl_.dtype], _DT[B_.dtype])
+    dev = u_.device
+    stream = _stream_handle(dev)
+    flags = _flags() | _lib.ckpt_rows_flag(ckpt_rows)
+    n_ckpt, nbytes = _sizes(Bsz, T, D, N, dts, flags)
+    ckpt = torch.empty(max(n_ckpt, 1), dtype=torch.float32, device=dev) if need_grad else None
+    _raise_pending(dev, stream)
+    ws = _WS.get(dev, stream, nbytes)
+    y = torch.empty((Bsz, T, D), dtype=u_.dtype, device=dev)
+    hT = torch.empty((Bsz, D, N), dtype=torch.float32, device=dev) if want_hT else None
+    L = _lib.lib()
+    args = (u_.data_ptr(), fl_.data_ptr(), il_.data_ptr(), B_.data_ptr(), C_.data_ptr(), D_.data_ptr(), _ptr(h0_),
+            y.data_ptr(), _ptr(ckpt), _ptr(hT), Bsz, T, D, N)
+    if bc_ld != N:
+        rc = L.naju_scan_fwd_strided(*args, bc_ld, *dts, flags, ws.data_ptr(), ws.numel(), stream)
+    else:
+        rc = L.naju_scan_fwd(*args, *dts, flags, ws.data_ptr(), ws.numel(), stream)
+    if rc:
+        _lib.check(rc)
+    _check_status(dev)
+    y = y if y.dtype == out_dtype else y.to(out_dtype)
+    return y, hT, ((u_, fl_, il_, B_, C_, D_, ckpt), (Bsz, T, D, N, dts, flags), bc_ld) if need_grad else None
+
+
 class NajuScanHip(torch.autograd.Function):
     """Autograd wrapper of naju_scan_fwd / naju_scan_bwd (include/naju_scan.h)."""
 
     @staticmethod
     def forward(ctx, u, f_logit, i_logit, B, C, D_skip, h0=None, want_hT=False, ckpt_rows=0, du_skip=None,
                 gate_grads=None):
-        Bsz, T, D, N = _check_shapes(u, f_logit, i_logit, B, C, D_skip, h0)
-        out_dtype = u.dtype
-        b_sinks = (sink_of(B), sink_of(C))
-        # a memory-light checkpoint interval keeps B and C as a copy, so the
-        # projection output is not held until the backward
-        Bp, Cp, bc_ld = _bc_pair(B, C, N, in_place=int(ckpt_rows or 0) <= 16)
-        u_, fl_, il_, B_, C_, D_, h0_ = _norm_inputs(u, f_logit, i_logit, Bp, Cp, D_skip, h0, bc_ld != N)
-        if bc_ld != N and (B_.data_ptr() != Bp.data_ptr() or C_.data_ptr() != Cp.data_ptr()):
-            # _norm_inputs converted their dtype: contiguous copies after all
-            B_, C_, bc_ld = B_.contiguous(), C_.contiguous(), N
-        dts = (_DT[u_.dtype], _DT[fl_.dtype], _DT[B_.dtype])
-        L = _lib.lib()
-        dev = u_.device
-        stream = _stream_handle(dev)
-        need_grad = any(ctx.needs_input_grad)
-        flags = _flags() | _lib.ckpt_rows_flag(ckpt_rows)
-        ckpt = None
-        if need_grad:
-            n = L.naju_scan_ckpt_elems_ex(Bsz, T, D, N, *dts, flags)
-            if n < 0:
-                _lib.check(_lib.ERR_UNSUPPORTED if "interval" in _lib.last_error() else _lib.ERR_INVALID)
-            ckpt = torch.empty(max(n, 1), dtype=torch.float32, device=dev)
-        nbytes = L.naju_scan_workspace_bytes_ex(Bsz, T, D, N, *dts, flags)
-        if nbytes == 0 and Bsz * T * D > 0:
-            _lib.check(_lib.ERR_UNSUPPORTED if "interval" in _lib.last_error() else _lib.ERR_INVALID)
-        _raise_pending(dev, stream)
-        ws = _WS.get(dev, stream, nbytes)
-        y = torch.empty((Bsz, T, D), dtype=u_.dtype, device=dev)
-        hT = torch.empty((Bsz, D, N), dtype=torch.float32, device=dev) if want_hT else None
-        if bc_ld != N:
-            _lib.check(L.naju_scan_fwd_strided(
-                _ptr(u_), _ptr(fl_), _ptr(il_), _ptr(B_), _ptr(C_), _ptr(D_), _ptr(h0_),
-                _ptr(y), _ptr(ckpt), _ptr(hT), Bsz, T, D, N, bc_ld, *dts, flags, ws.data_ptr(), ws.numel(), stream))
-        else:
-            _lib.check(L.naju_scan_fwd(
-                _ptr(u_), _ptr(fl_), _ptr(il_), _ptr(B_), _ptr(C_), _ptr(D_), _ptr(h0_),
-                _ptr(y), _ptr(ckpt), _ptr(hT), Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel(), stream))
-        _check_status(dev)
-        if need_grad:
+        y, hT, kept = _forward(u, f_logit, i_logit, B, C, D_skip, h0, want_hT, ckpt_rows, any(ctx.needs_input_grad))
+        if kept is not None:
+            (u_, fl_, il_, B_, C_, D_, ckpt), meta, bc_ld = kept
             # du_skip: the skip coefficient of du's D dy term in place of
             # D_skip (naju_scan_hip's doc)
             D_b = D_ if du_skip is None else du_skip.detach().float().contiguous()
             ctx.save_for_backward(u_, fl_, il_, B_, C_, D_, ckpt, D_b)
-            ctx.meta = (Bsz, T, D, N, dts, flags, h0 is not None,
+            ctx.meta = (*meta, h0 is not None,
                         (u.dtype, f_logit.dtype, i_logit.dtype, B.dtype, C.dtype, D_skip.dtype))
             # u is a gradsink.fanout() alias: du goes into the fan-out's
             # buffer when it is the first gradient there
@@ -265,10 +289,9 @@ class NajuScanHip(torch.autograd.Function):
             ctx.gate_grads = gate_grads
             # B and C are pieces of one gradsink.split (the mixer's
             # projection output): dB and dC can go straight into its buffer
-            s0, s1 = b_sinks
-            ctx.bc_sinks = b_sinks if (bc_ld != N and s0 is not None and s1 is not None and s0[0] is s1[0]
-                                       and s0[0].dtype == B_.dtype) else None
-        y = y if y.dtype == out_dtype else y.to(out_dtype)
+            s0, s1 = sink_of(B), sink_of(C)
+            ctx.bc_sinks = (s0, s1) if (bc_ld != meta[3] and s0 is not None and s1 is not None and s0[0] is s1[0]
+                                        and s0[0].dtype == B_.dtype) else None
         if want_hT:
             ctx.mark_non_differentiable(hT)
             return y, hT
@@ -325,7 +348,7 @@ class NajuScanHip(torch.autograd.Function):
         L = _lib.lib()
         stream = _stream_handle(dev)
         _raise_pending(dev, stream)
-        ws = _WS.get(dev, stream, L.naju_scan_workspace_bytes_ex(Bsz, T, D, N, *dts, flags))
+        ws = _WS.get(dev, stream, _sizes(Bsz, T, D, N, dts, flags)[1])
         if gtgt is not None:
             lay = _lib.ScanBwdLayout(bc_ld=ctx.bc_ld, dbc_ld=dbc_ld, dg_ld=dfl.stride(1), dg_dtype=_DT[dfl.dtype],
                                      dfl_sum=gsum.data_ptr(), dil_sum=gsum.data_ptr() + 4 * D)
@@ -339,10 +362,12 @@ class NajuScanHip(torch.autograd.Function):
                 _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD), _ptr(dh0),
                 Bsz, T, D, N, ctx.bc_ld, dbc_ld, *dts, flags, ws.data_ptr(), ws.numel(), stream))
         else:
-            _lib.check(L.naju_scan_bwd(
-                _ptr(u_), _ptr(fl_), _ptr(il_), _ptr(B_), _ptr(C_), _ptr(D_b), _ptr(ckpt), _ptr(dy),
-                _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD), _ptr(dh0),
-                Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel(), stream))
+            rc = L.naju_scan_bwd(
+                u_.data_ptr(), fl_.data_ptr(), il_.data_ptr(), B_.data_ptr(), C_.data_ptr(), D_b.data_ptr(),
+                ckpt.data_ptr(), dy.data_ptr(), _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD),
+                _ptr(dh0), Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel(), stream)
+            if rc:
+                _lib.check(rc)
         _check_status(dev)
         grads = [du, dfl, dil, dB, dC, dD]
         if gtgt is not None:
@@ -359,8 +384,10 @@ def _default_ckpt_rows(N):
     the environment where it is served (9 <= N <= 64), else the default. It
     lets unmodified NajuMixer / NajuLM code run the memory-light mode, as
     NAJU_SCAN_BACKEND=cuda selects the reference's recompute backend."""
-    v = os.environ.get("NAJU_CKPT_ROWS", "")
-    return int(v) if v and 9 <= N <= 64 else 0
+    if not 9 <= N <= 64 or "NAJU_CKPT_ROWS" not in os.environ:
+        return 0
+    v = os.environ["NAJU_CKPT_ROWS"]
+    return int(v) if v else 0
 
 
 def naju_scan_hip(u, f_logit, i_logit, B, C, D_skip, h0=None, return_final_state=False, ckpt_rows=None,
@@ -380,6 +407,14 @@ def naju_scan_hip(u, f_logit, i_logit, B, C, D_skip, h0=None, return_final_state
     own backward can leave out (one gradient fewer to add)."""
     if ckpt_rows is None:
         ckpt_rows = _default_ckpt_rows(B.shape[-1])
+    if (not torch.is_grad_enabled() and _fwd_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling()):
+        # nothing can be recorded: the call without the autograd function
+        # around it (a fifth of a one-token decode step's time). Forward-mode
+        # AD, functorch transforms, tracing and compilation go through it as
+        # ever (it refuses what it does not support there)
+        y, hT, _ = _forward(u, f_logit, i_logit, B, C, D_skip, h0, bool(return_final_state), int(ckpt_rows), False)
+        return (y, hT) if return_final_state else y
     return NajuScanHip.apply(u, f_logit, i_logit, B, C, D_skip, h0, bool(return_final_state), int(ckpt_rows),
                              du_skip, gate_grads)
 
