@@ -111,14 +111,7 @@ __global__ __launch_bounds__(64 * kMapMaxW) __attribute__((amdgpu_waves_per_eu(3
   const int N = a.N;
   const int64_t T = a.T, D = a.D;
   const int per = n_ctiles * a.batch;
-  // Neighbouring channel tiles share 128-byte lines (a wave's row is 64 bytes
-  // of a 2-byte stream) and B / C: consecutive tiles go to one XCD, whose L2
-  // then holds what they share (workgroups are dealt to the 8 XCDs in turn).
-  uint32_t id = blockIdx.x;
-  {
-    const uint32_t x = id & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
-    id = x * q + (x < r ? x : r) + (id >> 3);
-  }
+  const uint32_t id = xcd_item();
   const int seg = (int)(id / (uint32_t)per) + (BWD ? 1 : 0);
   const int rem = (int)(id % (uint32_t)per);
   const int b = rem / n_ctiles;

@@ -837,8 +837,9 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 
   const int N = a.N;
   const int64_t T = a.T, D = a.D;
-  const int tile = (int)(blockIdx.x % (uint32_t)a.n_tiles);
-  const int seg = (int)(blockIdx.x / (uint32_t)a.n_tiles);
+  const uint32_t item = xcd_item();
+  const int tile = (int)(item % (uint32_t)a.n_tiles);
+  const int seg = (int)(item / (uint32_t)a.n_tiles);
   const int b = tile / a.n_dtiles;
   const int dtile = tile - b * a.n_dtiles;
   const int tid = (int)threadIdx.x;
@@ -1328,15 +1329,25 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       // and ghat (entering this sub-block) per channel and entry come through
       // this wave's pool as [16 channels][P] tiles, written in the D layout
       // and read transposed.
-      // (tiles 0 and 1: the decay phase is done with them)
-      float (*TQ1)[TP] = (float (*)[TP])(pl + 0 * 16 * TP);  // (dy Pf)[t][d]
-      float (*TQ2)[TP] = (float (*)[TP])(pl + 1 * 16 * TP);  // (w Pe)[t][d]
+      // With one output tile per wave (NP = 64) the operands of all waves stay
+      // in LDS and wave w forms tile w over the workgroup's 128 channels after
+      // the barrier; with fewer tiles than waves each wave forms its channels'
+      // part of every tile, and the parts are added after it. (bf16
+      // 8 x 4096 x 1024, with the XCD order of the tiles: 588 -> 569 us; the parts
+      // of all waves went through LDS before.)
+      constexpr bool whole = 2 * MT == kMcWB;
+      // (dy Pf)[t][d], (w Pe)[t][d]: in gate tiles, free once the outputs are
+      // stored, or in pool tiles that the decay phase is done with
+      float (*TQ1)[TP] = whole ? sh.gate[wv][1] : (float (*)[TP])(pl + 0 * 16 * TP);
+      float (*TQ2)[TP] = whole ? sh.gate[wv][0] : (float (*)[TP])(pl + 1 * 16 * TP);
 #pragma unroll
       for (int r = 0; r < 4; ++r) TQ1[4 * r + g][j] = q1[r], TQ2[4 * r + g][j] = q2[r];
       asm volatile("" ::: "memory");
       float qv1[4], qv2[4];
-      rd4(&TQ1[j][4 * g], qv1);
-      rd4(&TQ2[j][4 * g], qv2);
+      if constexpr (!whole) {
+        rd4(&TQ1[j][4 * g], qv1);
+        rd4(&TQ2[j][4 * g], qv2);
+      }
       asm volatile("" ::: "memory");
       float* TX = pl;           // X [channel][n]
       float* TGh = pl + 16 * P;  // ghat [channel][n]
@@ -1354,6 +1365,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       // channels (the H part, B^T H and C^T H^T, is formed once per
       // workgroup from the waves' summed H after the partial-sum barrier)
       f4_t dCt[MT], dBt[MT];
+      if constexpr (!whole)
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         f4_t accC = {0.f, 0.f, 0.f, 0.f}, accB = {0.f, 0.f, 0.f, 0.f};
@@ -1371,6 +1383,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       // are done; other waves read it after the barrier), then the workgroup
       // adds the waves' in wave order
       asm volatile("" ::: "memory");
+      if constexpr (!whole)
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         wr4(pl + (0 * 16 + j) * P + 16 * m + 4 * g, dCt[m][0], dCt[m][1], dCt[m][2], dCt[m][3]);
@@ -1386,15 +1399,35 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         // C^T (sum H)^T with H summed over the waves in wave order
         const int qd = wv / MT, m = wv - qd * MT;
         float hs[4] = {0.f, 0.f, 0.f, 0.f}, acc[4] = {0.f, 0.f, 0.f, 0.f};
+        f4_t ac0 = {0.f, 0.f, 0.f, 0.f}, ac1 = ac0;
 #pragma unroll
         for (int w = 0; w < kMcWB; ++w) {
           const float* pw = sh.pool[w];
           float h4[4], v4[4];
           rd4(pw + kPH + qd * 16 * TP + j * TP + 4 * g, h4);
-          rd4(pw + (qd * 16 + j) * P + 16 * m + 4 * g, v4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) hs[e] += h4[e], acc[e] += v4[e];
+          for (int e = 0; e < 4; ++e) hs[e] += h4[e];
+          if constexpr (whole) {
+            // channels 4g + e of wave w: A = its X (ghat) transposed, B = its
+            // (dy Pf) or (w Pe)
+            rd4(&sh.gate[w][1 - qd][j][4 * g], v4);
+            const float* ax = pw + qd * 16 * P + 4 * g * P + 16 * m + j;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              if (w & 1)
+                ac1 = mma(ax[e * P], v4[e], ac1);
+              else
+                ac0 = mma(ax[e * P], v4[e], ac0);
+            }
+          } else {
+            rd4(pw + (qd * 16 + j) * P + 16 * m + 4 * g, v4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += v4[e];
+          }
         }
+        if constexpr (whole)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] = ac0[e] + ac1[e];
         float a4[4];
         rd4(qd == 0 ? &sh.Bt[16 * m + j][4 * g] : &sh.Ct[16 * m + j][4 * g], a4);
         f4_t hp = {0.f, 0.f, 0.f, 0.f};

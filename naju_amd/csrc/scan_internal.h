@@ -136,6 +136,16 @@ struct ScanArgs {
   uint32_t spin_limit;
 };
 
+// The work item of a workgroup, so that consecutive items run on one XCD:
+// workgroups are dealt to the 8 XCDs in turn, and item order puts the channel
+// tiles of one (batch row, segment) side by side, which read the same B and C
+// (and, where a tile's row is not whole lines, parts of the same lines). One
+// XCD's L2 then serves them all, where eight fetched the same rows before.
+__device__ __forceinline__ uint32_t xcd_item() {
+  const uint32_t id = blockIdx.x, x = id & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
+  return x * q + (x < r ? x : r) + (id >> 3);
+}
+
 // Lane exchange for the butterfly steps below: the value of the partner lane
 // that differs in bit log2(m) (and, for m = 8 / 4, in the lower bits too:
 // row_mirror pairs i with 15 - i, row_half_mirror i with 7 - i).
