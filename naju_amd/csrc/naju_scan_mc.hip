@@ -29,6 +29,8 @@
 // value s: the state chain needs no data movement between lanes.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mc_ops.h"
 #include "naju_scan.h"
 #include "scan_internal.h"
@@ -631,14 +633,20 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
 // (5 KB) and a pool of seven [16][TP] tiles (8.75 KB) that holds G, G^T,
 // gathers, the rectangle sums' partials, (dy Pf) / (w Pe), H / H^T and
 // finally the wave's dB / dC, which the workgroup adds in wave order.
-template <int NP>
+// With bf16 B and C every product that takes them is on the 16-bit matrix
+// cores, so their tiles hold bf16 as loaded: no conversion, half the LDS bytes
+// (the LM layer's backward, 8 x 2048 x 1536: 435 -> 419 us).
+template <int NP, typename TB>
 struct McBwdLds {
   static constexpr int P = NP + 4;
   static constexpr int POOL = 9 * 16 * TP;  // floats of a wave's pool
-  float Bn[kMcQ][P];
-  float C[kMcQ][P];
-  float Bt[NP][TP];
-  float Ct[NP][TP];
+  static constexpr bool H = __is_same(TB, bf16_t);
+  static constexpr int PB = H ? NP + 8 : P, PT = H ? 24 : TP;
+  using TL = std::conditional_t<H, bf16_t, float>;
+  __align__(16) TL Bn[kMcQ][PB];
+  __align__(16) TL C[kMcQ][PB];
+  __align__(16) TL Bt[NP][PT];
+  __align__(16) TL Ct[NP][PT];
   float gate[kMcWB][4][16][TP];  // f, dy, w, i as [channel][row]; later dfl, du, dil
   float pool[kMcWB][POOL];
 };
@@ -710,23 +718,38 @@ struct McInB {
   // different banks, and each [t][n] tile takes one 16-byte write per lane
   // (the forward's row-per-16-lanes map costs 14 and 6 extra LDS cycles per
   // write there, about 1.4% of this kernel).
-  __device__ __forceinline__ void stage(McBwdLds<NP>& sh, const ScanArgs& a, int64_t t0, int tid) const {
+  __device__ __forceinline__ void stage(McBwdLds<NP, TB>& sh, const ScanArgs& a, int64_t t0, int tid) const {
     if (tid < 4 * NP) {
       const int row = tid % kMcQ, n0 = 4 * (tid / kMcQ);
       const bool rok = t0 + row < a.T;
       const int pr = 4 * (row & 3) + (row >> 2);
-      float vb[4], vc[4];
+      if constexpr (McBwdLds<NP, TB>::H) {
+        // pairs of entries as loaded, zeros past T and past N
+        uint32_t wb[2], wc[2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool ok = rok && n0 + e < a.N;
-        vc[e] = ok ? c.get(e) : 0.f;
-        sh.Ct[n0 + e][pr] = vc[e];
-        {
+        for (int k = 0; k < 2; ++k) {
+          const int left = rok ? a.N - (n0 + 2 * k) : 0;
+          const uint32_t keep = left >= 2 ? 0xffffffffu : (left == 1 ? 0xffffu : 0u);
+          wb[k] = b.w[k] & keep;
+          wc[k] = c.w[k] & keep;
+        }
+        *(uint2*)&sh.Bn[row][n0] = make_uint2(wb[0], wb[1]);
+        *(uint2*)&sh.C[row][n0] = make_uint2(wc[0], wc[1]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          *(uint16_t*)&sh.Bt[n0 + e][pr] = (uint16_t)((e & 1) ? wb[e >> 1] >> 16 : wb[e >> 1]);
+          *(uint16_t*)&sh.Ct[n0 + e][pr] = (uint16_t)((e & 1) ? wc[e >> 1] >> 16 : wc[e >> 1]);
+        }
+      } else {
+        float vb[4], vc[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool ok = rok && n0 + e < a.N;
+          vc[e] = ok ? c.get(e) : 0.f;
+          sh.Ct[n0 + e][pr] = vc[e];
           vb[e] = ok ? b.get(e) : 0.f;
           sh.Bt[n0 + e][pr] = vb[e];
         }
-      }
-      {
         *(float4*)&sh.Bn[row][n0] = make_float4(vb[0], vb[1], vb[2], vb[3]);
         *(float4*)&sh.C[row][n0] = make_float4(vc[0], vc[1], vc[2], vc[3]);
       }
@@ -740,20 +763,24 @@ __device__ __forceinline__ void rd4(const float* p, float (&o)[4]) {
   o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
 }
 
+// Four bf16 values at p (8-byte aligned) as the packed pairs of pack4.
+__device__ __forceinline__ void rd4h(const bf16_t* p, uint32_t (&w)[2]) {
+  const uint2 v = *(const uint2*)p;
+  w[0] = v.x, w[1] = v.y;
+}
+
 // The adjoint carry's update ghat <- Pall ghat + C^T (Pf dy) for the lane's
 // entries (k-step e takes rows 4e + g; on the 16-bit path when C is bf16).
 template <typename TB, int MT>
-__device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const float (*Ct)[TP], float Pall, const float (&pfdy)[4],
-                                             int j, int g) {
+__device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const McBwdLds<16 * MT, TB>& sh, float Pall,
+                                             const float (&pfdy)[4], int j, int g) {
   if constexpr (__is_same(TB, bf16_t)) {
     uint32_t qh[2], qm[2], ql[2];
     split4_bf16(pfdy, qh, qm, ql);
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      float ct4[4];
-      rd4(&Ct[16 * m + j][4 * g], ct4);
       uint32_t ac[2];
-      pack4<TB>(ct4, ac);
+      rd4h(&sh.Ct[16 * m + j][4 * g], ac);
       gh[m] *= Pall;
       gh[m] = mma_x3(ac, qh, qm, ql, gh[m]);
     }
@@ -761,7 +788,7 @@ __device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const float (*Ct)[T
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       float ct4[4];
-      rd4(&Ct[16 * m + j][4 * g], ct4);
+      rd4(&sh.Ct[16 * m + j][4 * g], ct4);
       gh[m] *= Pall;
 #pragma unroll
       for (int e = 0; e < 4; ++e) gh[m] = mma(ct4[e], pfdy[e], gh[m]);
@@ -833,7 +860,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
   constexpr int MT = NP / 16;
   constexpr int P = NP + 4;
   using In = McInB<NP, TU, TG, TB>;
-  __shared__ __align__(16) McBwdLds<NP> sh;
+  __shared__ __align__(16) McBwdLds<NP, TB> sh;
 
   const int N = a.N;
   const int64_t T = a.T, D = a.D;
@@ -975,7 +1002,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       // H in the pool's last two tiles, past the dC / dB partials (which take
       // its first 32 P floats) and the scratch tiles: other waves read it
       // after the partial-sum barrier
-      constexpr int kPH = McBwdLds<NP>::POOL - 32 * TP;
+      constexpr int kPH = McBwdLds<NP, TB>::POOL - 32 * TP;
       static_assert(32 * P <= kPH && 7 * 16 * TP <= kPH, "H tiles clear of the partials and scratch tiles");
       float (*TH)[TP] = (float (*)[TP])(pl + kPH);             // H[t][p(r)]
       float (*THT)[TP] = (float (*)[TP])(pl + kPH + 16 * TP);  // H[s][t] at [t][p(s)]
@@ -991,15 +1018,29 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       uint32_t pb[2], pc[2];
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        float c4[4], b4[4];
-        rd4(&sh.C[arow][16 * m + 4 * g], c4);
-        rd4(&sh.Bn[arow][16 * m + 4 * g], b4);
         constexpr bool bx = g16 && __is_same(TB, bf16_t);
+        float c4[4] = {}, b4[4] = {};
+        uint32_t wb[2], wc[2];  // packed pairs, with 16-bit B and C
+        if constexpr (__is_same(TB, bf16_t)) {
+          rd4h(&sh.C[arow][16 * m + 4 * g], wc);
+          rd4h(&sh.Bn[arow][16 * m + 4 * g], wb);
+          if constexpr (!bx)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              c4[e] = __builtin_bit_cast(float, (e & 1) ? wc[e >> 1] & 0xffff0000u : wc[e >> 1] << 16);
+              b4[e] = __builtin_bit_cast(float, (e & 1) ? wb[e >> 1] & 0xffff0000u : wb[e >> 1] << 16);
+            }
+        } else {
+          rd4(&sh.C[arow][16 * m + 4 * g], c4);
+          rd4(&sh.Bn[arow][16 * m + 4 * g], b4);
+          if constexpr (g16) {
+            pack4<TB>(b4, wb);
+            pack4<TB>(c4, wc);
+          }
+        }
         if constexpr (g16) {
           if (m & 1) {
-            uint32_t qb[2], qc[2];
-            pack4<TB>(b4, qb);
-            pack4<TB>(c4, qc);
+            const uint32_t (&qb)[2] = wb, (&qc)[2] = wc;
             Gp = mma_k32<TB>(pb, qb, pc, qc, Gp);
             if constexpr (bx) {
               // C X and B ghat over the pair of entry groups m - 1, m: X and
@@ -1025,8 +1066,8 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
               bg = mma_k32<TB>(pb, qb, l0, l1, bg);
             }
           } else {
-            pack4<TB>(b4, pb);
-            pack4<TB>(c4, pc);
+            pb[0] = wb[0], pb[1] = wb[1];
+            pc[0] = wc[0], pc[1] = wc[1];
           }
         }
 #pragma unroll
@@ -1378,7 +1419,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         dBt[m] = accB;
       }
       // ---- carry update: ghat <- Pall ghat + C^T (Pf dy)
-      carry_update<TB, MT>(gh, sh.Ct, Pall, pfdy, j, g);
+      carry_update<TB, MT>(gh, sh, Pall, pfdy, j, g);
       // ---- the wave's dC / dB [t][n] into its pool (its reads of the pool
       // are done; other waves read it after the barrier), then the workgroup
       // adds the waves' in wave order
@@ -1428,15 +1469,15 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         if constexpr (whole)
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[e] = ac0[e] + ac1[e];
-        float a4[4];
-        rd4(qd == 0 ? &sh.Bt[16 * m + j][4 * g] : &sh.Ct[16 * m + j][4 * g], a4);
         f4_t hp = {0.f, 0.f, 0.f, 0.f};
         if constexpr (__is_same(TB, bf16_t)) {
           uint32_t ab[2], hh[2], hm[2], hl[2];
-          pack4<TB>(a4, ab);
+          rd4h(qd == 0 ? &sh.Bt[16 * m + j][4 * g] : &sh.Ct[16 * m + j][4 * g], ab);
           split4_bf16(hs, hh, hm, hl);
           hp = mma_x3(ab, hh, hm, hl, hp);
         } else {
+          float a4[4];
+          rd4(qd == 0 ? &sh.Bt[16 * m + j][4 * g] : &sh.Ct[16 * m + j][4 * g], a4);
 #pragma unroll
           for (int e = 0; e < 4; ++e) hp = mma(a4[e], hs[e], hp);
         }
