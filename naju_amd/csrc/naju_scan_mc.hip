@@ -643,10 +643,13 @@ struct McBwdLds {
   static constexpr bool H = __is_same(TB, bf16_t);
   static constexpr int PB = H ? NP + 8 : P, PT = H ? 24 : TP;
   using TL = std::conditional_t<H, bf16_t, float>;
-  __align__(16) TL Bn[kMcQ][PB];
-  __align__(16) TL C[kMcQ][PB];
-  __align__(16) TL Bt[NP][PT];
-  __align__(16) TL Ct[NP][PT];
+  // and fit twice: the next sub-block's are staged while a slower wave still
+  // reads this one's, so no barrier is needed at the sub-block's end
+  static constexpr int NB = H ? 2 : 1;
+  __align__(16) TL Bn[NB][kMcQ][PB];
+  __align__(16) TL C[NB][kMcQ][PB];
+  __align__(16) TL Bt[NB][NP][PT];
+  __align__(16) TL Ct[NB][NP][PT];
   float gate[kMcWB][4][16][TP];  // f, dy, w, i as [channel][row]; later dfl, du, dil
   float pool[kMcWB][POOL];
 };
@@ -718,7 +721,7 @@ struct McInB {
   // different banks, and each [t][n] tile takes one 16-byte write per lane
   // (the forward's row-per-16-lanes map costs 14 and 6 extra LDS cycles per
   // write there, about 1.4% of this kernel).
-  __device__ __forceinline__ void stage(McBwdLds<NP, TB>& sh, const ScanArgs& a, int64_t t0, int tid) const {
+  __device__ __forceinline__ void stage(McBwdLds<NP, TB>& sh, int buf, const ScanArgs& a, int64_t t0, int tid) const {
     if (tid < 4 * NP) {
       const int row = tid % kMcQ, n0 = 4 * (tid / kMcQ);
       const bool rok = t0 + row < a.T;
@@ -733,12 +736,12 @@ struct McInB {
           wb[k] = b.w[k] & keep;
           wc[k] = c.w[k] & keep;
         }
-        *(uint2*)&sh.Bn[row][n0] = make_uint2(wb[0], wb[1]);
-        *(uint2*)&sh.C[row][n0] = make_uint2(wc[0], wc[1]);
+        *(uint2*)&sh.Bn[buf][row][n0] = make_uint2(wb[0], wb[1]);
+        *(uint2*)&sh.C[buf][row][n0] = make_uint2(wc[0], wc[1]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          *(uint16_t*)&sh.Bt[n0 + e][pr] = (uint16_t)((e & 1) ? wb[e >> 1] >> 16 : wb[e >> 1]);
-          *(uint16_t*)&sh.Ct[n0 + e][pr] = (uint16_t)((e & 1) ? wc[e >> 1] >> 16 : wc[e >> 1]);
+          *(uint16_t*)&sh.Bt[buf][n0 + e][pr] = (uint16_t)((e & 1) ? wb[e >> 1] >> 16 : wb[e >> 1]);
+          *(uint16_t*)&sh.Ct[buf][n0 + e][pr] = (uint16_t)((e & 1) ? wc[e >> 1] >> 16 : wc[e >> 1]);
         }
       } else {
         float vb[4], vc[4];
@@ -746,12 +749,12 @@ struct McInB {
         for (int e = 0; e < 4; ++e) {
           const bool ok = rok && n0 + e < a.N;
           vc[e] = ok ? c.get(e) : 0.f;
-          sh.Ct[n0 + e][pr] = vc[e];
+          sh.Ct[buf][n0 + e][pr] = vc[e];
           vb[e] = ok ? b.get(e) : 0.f;
-          sh.Bt[n0 + e][pr] = vb[e];
+          sh.Bt[buf][n0 + e][pr] = vb[e];
         }
-        *(float4*)&sh.Bn[row][n0] = make_float4(vb[0], vb[1], vb[2], vb[3]);
-        *(float4*)&sh.C[row][n0] = make_float4(vc[0], vc[1], vc[2], vc[3]);
+        *(float4*)&sh.Bn[buf][row][n0] = make_float4(vb[0], vb[1], vb[2], vb[3]);
+        *(float4*)&sh.C[buf][row][n0] = make_float4(vc[0], vc[1], vc[2], vc[3]);
       }
     }
   }
@@ -772,7 +775,7 @@ __device__ __forceinline__ void rd4h(const bf16_t* p, uint32_t (&w)[2]) {
 // The adjoint carry's update ghat <- Pall ghat + C^T (Pf dy) for the lane's
 // entries (k-step e takes rows 4e + g; on the 16-bit path when C is bf16).
 template <typename TB, int MT>
-__device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const McBwdLds<16 * MT, TB>& sh, float Pall,
+__device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const McBwdLds<16 * MT, TB>& sh, int buf, float Pall,
                                              const float (&pfdy)[4], int j, int g) {
   if constexpr (__is_same(TB, bf16_t)) {
     uint32_t qh[2], qm[2], ql[2];
@@ -780,7 +783,7 @@ __device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const McBwdLds<16 *
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       uint32_t ac[2];
-      rd4h(&sh.Ct[16 * m + j][4 * g], ac);
+      rd4h(&sh.Ct[buf][16 * m + j][4 * g], ac);
       gh[m] *= Pall;
       gh[m] = mma_x3(ac, qh, qm, ql, gh[m]);
     }
@@ -788,7 +791,7 @@ __device__ __forceinline__ void carry_update(f4_t (&gh)[MT], const McBwdLds<16 *
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       float ct4[4];
-      rd4(&sh.Ct[16 * m + j][4 * g], ct4);
+      rd4(&sh.Ct[buf][16 * m + j][4 * g], ct4);
       gh[m] *= Pall;
 #pragma unroll
       for (int e = 0; e < 4; ++e) gh[m] = mma(ct4[e], pfdy[e], gh[m]);
@@ -940,27 +943,38 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
     const int64_t t0 = (int64_t)sb * Q;
     // ---- stage B / C; gates in the load layout (each element once; rows
     // past T and channels past D are the neutral step f = 1, i = w = dy = 0)
-    cur.stage(sh, a, t0, tid);
+    const int buf = McBwdLds<NP, TB>::NB == 2 ? (sb1 - 1 - sb) & 1 : 0;
+    cur.stage(sh, buf, a, t0, tid);
     const int rl = (int)(T - t0 < Q ? T - t0 : Q);  // rows left (uniform)
     const bool rok = rho < rl;
+    float gf[4], gi[4], gw[4], gy[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const bool ok = rok && e < ncq;
       // gates formed on every lane, then selected (no branch per element)
       float sf = sigm(cur.f.get(e));
       asm volatile("" : "+v"(sf));
-      Tf[cq + e][rho] = ok ? sf : 1.f;
-      Tdy[cq + e][rho] = ok ? cur.dy.get(e) : 0.f;
-      {
-        float si = sigm(cur.i.get(e));
-        asm volatile("" : "+v"(si));
-        const float ig = ok ? si : 0.f;
-        sh.gate[wv][3][cq + e][rho] = ig;
-        sh.gate[wv][2][cq + e][rho] = ok ? ig * cur.u.get(e) : 0.f;
-        dDacc[e] = fmaf(ok ? cur.dy.get(e) : 0.f, ok ? cur.u.get(e) : 0.f, dDacc[e]);
-      }
+      gf[e] = ok ? sf : 1.f;
+      gy[e] = ok ? cur.dy.get(e) : 0.f;
+      float si = sigm(cur.i.get(e));
+      asm volatile("" : "+v"(si));
+      gi[e] = ok ? si : 0.f;
+      gw[e] = ok ? gi[e] * cur.u.get(e) : 0.f;
+      dDacc[e] = fmaf(gy[e], ok ? cur.u.get(e) : 0.f, dDacc[e]);
     }
-    __syncthreads();  // staging visible
+    const auto put_gates = [&]() {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        Tf[cq + e][rho] = gf[e];
+        Tdy[cq + e][rho] = gy[e];
+        sh.gate[wv][3][cq + e][rho] = gi[e];
+        sh.gate[wv][2][cq + e][rho] = gw[e];
+      }
+    };
+    if constexpr (McBwdLds<NP, TB>::NB == 1) put_gates();
+    __syncthreads();  // staging visible; every wave is done with the one before
+    // (the gate tiles held operands that other waves read until this barrier)
+    if constexpr (McBwdLds<NP, TB>::NB == 2) put_gates();
     // the first half's terms, used at this sub-block's outputs (issued before
     // the next sub-block's loads, so that waiting for them waits for no others)
     float* hp_p = nullptr;
@@ -1022,8 +1036,8 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         float c4[4] = {}, b4[4] = {};
         uint32_t wb[2], wc[2];  // packed pairs, with 16-bit B and C
         if constexpr (__is_same(TB, bf16_t)) {
-          rd4h(&sh.C[arow][16 * m + 4 * g], wc);
-          rd4h(&sh.Bn[arow][16 * m + 4 * g], wb);
+          rd4h(&sh.C[buf][arow][16 * m + 4 * g], wc);
+          rd4h(&sh.Bn[buf][arow][16 * m + 4 * g], wb);
           if constexpr (!bx)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -1031,8 +1045,8 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
               b4[e] = __builtin_bit_cast(float, (e & 1) ? wb[e >> 1] & 0xffff0000u : wb[e >> 1] << 16);
             }
         } else {
-          rd4(&sh.C[arow][16 * m + 4 * g], c4);
-          rd4(&sh.Bn[arow][16 * m + 4 * g], b4);
+          rd4(&sh.C[buf][arow][16 * m + 4 * g], c4);
+          rd4(&sh.Bn[buf][arow][16 * m + 4 * g], b4);
           if constexpr (g16) {
             pack4<TB>(b4, wb);
             pack4<TB>(c4, wc);
@@ -1419,7 +1433,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         dBt[m] = accB;
       }
       // ---- carry update: ghat <- Pall ghat + C^T (Pf dy)
-      carry_update<TB, MT>(gh, sh, Pall, pfdy, j, g);
+      carry_update<TB, MT>(gh, sh, buf, Pall, pfdy, j, g);
       // ---- the wave's dC / dB [t][n] into its pool (its reads of the pool
       // are done; other waves read it after the barrier), then the workgroup
       // adds the waves' in wave order
@@ -1472,12 +1486,12 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         f4_t hp = {0.f, 0.f, 0.f, 0.f};
         if constexpr (__is_same(TB, bf16_t)) {
           uint32_t ab[2], hh[2], hm[2], hl[2];
-          rd4h(qd == 0 ? &sh.Bt[16 * m + j][4 * g] : &sh.Ct[16 * m + j][4 * g], ab);
+          rd4h(qd == 0 ? &sh.Bt[buf][16 * m + j][4 * g] : &sh.Ct[buf][16 * m + j][4 * g], ab);
           split4_bf16(hs, hh, hm, hl);
           hp = mma_x3(ab, hh, hm, hl, hp);
         } else {
           float a4[4];
-          rd4(qd == 0 ? &sh.Bt[16 * m + j][4 * g] : &sh.Ct[16 * m + j][4 * g], a4);
+          rd4(qd == 0 ? &sh.Bt[buf][16 * m + j][4 * g] : &sh.Ct[buf][16 * m + j][4 * g], a4);
 #pragma unroll
           for (int e = 0; e < 4; ++e) hp = mma(a4[e], hs[e], hp);
         }
@@ -1499,9 +1513,9 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
         }
       }
     }
-    // every wave is done with the staged B / C (and, in the scan, with the
-    // pools and H tiles its output tile reads) before they are restaged
-    __syncthreads();
+    // (one buffer:) every wave is done with the staged B / C, the pools and the
+    // H tiles its output tile reads before they are restaged
+    if constexpr (McBwdLds<NP, TB>::NB == 1) __syncthreads();
     cur = nxt;
     {
 #pragma unroll
