@@ -1611,7 +1611,8 @@ __global__ __launch_bounds__(256) void gn_seg_carry_kernel(const ScanArgs a, int
 
 // ------------------------------------------------- general N backward kernel
 //
-// One workgroup per (batch row, 64-channel tile, time segment), 8 waves.
+// N <= 8. One workgroup per (batch row, tile of DT channels, time segment), W
+// waves.
 // Lanes run over the state index n (LG = min(NP, 64) lanes per channel, S
 // states per lane, G channels per wave instruction). A wave walks its
 // channel passes one after another; per kGnCK-row sub-chunk (the checkpoint
@@ -2223,7 +2224,7 @@ constexpr int kGnBwdDT = 32, kGnBwdW = 4;
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 int np_of(int64_t N);
-// The chunked matrix-core kernels serve 9 <= N <= 64 in the directions that
+// The chunked matrix-core kernels serve 9 <= N <= 128 in the directions that
 // have them.
 constexpr bool kMcBwd = true;
 bool use_mc(int64_t N, bool bwd) { return mc_ok(N) && (!bwd || kMcBwd); }
@@ -2284,8 +2285,6 @@ void place_regions(Layout& l, int64_t batch, int64_t T, int64_t D, int64_t N, bo
   l.total = off;
 }
 
-// cap: at N > 1, fewer time segments (down to one) until the workspace fits
-// in cap bytes; the N = 1 layout has no such freedom.
 // cap: at N > 1, fewer time segments (down to one) until the workspace fits
 // in cap bytes; the N = 1 layout has no such freedom. ck_rows: the
 // checkpoint interval (0 = the default; it sizes the backward's recomputed

@@ -644,7 +644,9 @@ struct McBwdLds {
   static constexpr int PB = H ? NP + 8 : P, PT = H ? 24 : TP;
   using TL = std::conditional_t<H, bf16_t, float>;
   // and fit twice: the next sub-block's are staged while a slower wave still
-  // reads this one's, so no barrier is needed at the sub-block's end
+  // reads this one's, so no barrier is needed at the sub-block's end (training
+  // step at bf16 4 x 4096 x 1024, N = 64: 474 -> 466 us; two buffers of float32
+  // tiles would take 171 KB)
   static constexpr int NB = H ? 2 : 1;
   __align__(16) TL Bn[NB][kMcQ][PB];
   __align__(16) TL C[NB][kMcQ][PB];
