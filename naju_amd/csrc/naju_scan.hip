@@ -2275,7 +2275,7 @@ void place_regions(Layout& l, int64_t batch, int64_t T, int64_t D, int64_t N, bo
   off = align_up(off + seg_units * N * sizeof(float));
   // the backward's recomputed state at every sub-block when the forward's
   // checkpoint interval is longer than the sub-block
-  // N > 64: the backward's first half's terms of dws and xbar . x
+  // N > 64: the backward's first half's terms of dws and f xbar . x_{t-1}
   const size_t KS = (size_t)((T + kMcQ - 1) / kMcQ);
   l.off_half = off;
   off = align_up(off + (bwd && mc_ok(N) && !mc_ext_ok(N) ? (size_t)batch * KS * D * 2 * kMcQ * sizeof(float) : 0));

@@ -608,11 +608,16 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
 // carry ghat entering its last row:
 //   xbar_t = sum_{s>=t} P[s,t] C_s dy_s + Pe_t ghat
 //   dws_t  = xbar_t . B_t = sum_{s>=t} P[s,t] dy_s G[s][t] + Pe_t (B_t . ghat)
-//   xbar_t . x_t = Pf_t sum_{s>=t} P[s,t] dy_s (C_s . X)
-//                + sum_{s>=t>=r} P[s,r] dy_s w_r G[s][r]          (rectangle)
-//                + Pe_t Pf_t (ghat . X) + Pe_t sum_{r<=t} P[t,r] w_r (B_r . ghat)
-//   dfl_t  = (1 - f_t) (xbar_t . x_t - w_t dws_t)  (= f(1-f) xbar_t . x_{t-1},
-//            no division; exactly 0 at f = 1, and set to 0 at f = 0)
+//   f_t xbar_t . x_{t-1} = Pf_t sum_{s>=t} P[s,t] dy_s (C_s . X)
+//                + sum_{s>=t>r} P[s,r] dy_s w_r G[s][r]           (rectangle)
+//                + Pe_t Pf_t (ghat . X) + Pe_t sum_{r<t} P[t,r] w_r (B_r . ghat)
+//   dfl_t  = (1 - f_t) f_t xbar_t . x_{t-1}  (no division; exactly 0 at f = 1,
+//            and set to 0 at f = 0)
+// Every term of f_t xbar_t . x_{t-1} holds the factor f_t. xbar_t . x_t less
+// w_t dws_t is the same number, but the terms without f_t cancel there: with
+// nearly closed gates the difference is of order f, its error of order 2^-24
+// without that factor (restated in float32, N = 128, f_logit around -4 / -9 /
+// -12: dfl off by 1.1e-5 / 1.1e-3 / 2.4e-2 of its norm; 3e-7 as it is here).
 //   du_t   = i_t dws_t + D dy_t,   dil_t = (1 - i_t) dws_t w_t
 //   dC_t   = sum_d (dy Pf)_t[d] X[.][d] + sum_{r<=t} H[t][r] B_r
 //   dB_t   = sum_d (w Pe)_t[d] ghat[.][d] + sum_{s>=t} H[s][t] C_s
@@ -855,7 +860,8 @@ __device__ __forceinline__ void store_row4(void* p, uint32_t o, const float (*tl
 // HALF = 0: all of N. N > 64 runs as two launches over halves of the entries,
 // since a second set of 64 entries of X and ghat per channel does not fit the
 // registers and the LDS beside the first: dB, dC, dh0 and the states are the
-// half's own, and what is summed over the entries, dws and xbar . x, the first
+// half's own, and what is summed over the entries, dws and
+// f xbar . x_{t-1}, the first
 // (HALF = 1) leaves in a.half and the second (HALF = 2) adds before it forms
 // du, dfl and dil. (bf16 4 x 2048 x 1024, N = 128: 161 + 172 us for the two
 // halves against 744 us on the vector units; the forward, whole at NP = 128,
@@ -1100,20 +1106,29 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       gX += __shfl_xor(gX, 16, 64);
       gX += __shfl_xor(gX, 32, 64);
       // ---- the decay terms of the own rows t:
-      //   V1_t = sum_{s>=t} P[s,t] dy_s G[s][t], V2_t = sum_{s>=t} P[s,t] dy_s (C X)_s,
-      //   V3_t = sum_{r<=t} P[t,r] w_r (B ghat)_r,
-      //   A3_t = sum_{s>=t>=r} M[s][r], M[s][r] = P[s,r] dy_s w_r G[s][r],
+      //   V1_t = sum_{s>=t} P[s,t] dy_s G[s][t],
+      //   V2_t = Pf_t sum_{s>=t} P[s,t] dy_s (C X)_s + sum_{s>=t>r} M[s][r]
+      //          with M[s][r] = P[s,r] dy_s w_r G[s][r],
+      //   V3_t = sum_{r<t} P[t,r] w_r (B ghat)_r,
       // and H[s][r] = sum over the wave's channels of P[s,r] dy_s w_r.
-      float V1[4], V2[4], V3[4], A3[4];
-      if (__all(Pall >= kMcRatioMin)) {
+      float V1[4], V2[4], V3[4];
+      float fmin = fa[0];
+#pragma unroll
+      for (int q = 1; q < Q; ++q) fmin = fminf(fmin, fa[q]);
+      if (__all(Pall >= kMcRatioMin && fmin >= kMcGateMin)) {
         // Every channel's decay over the sub-block stays above kMcRatioMin:
         // P[s,t] = Pf[s] / Pf[t] in floating point, with a = Pf dy and
         // b = w / Pf, and every term is a 16 x 16 x 16 product (MFMA row i =
         // time row arow(i), k-step e = row 4e + g, whose a and b this lane
-        // holds): V1 = (masked G^T a) / Pf, V2 = (masked ones (a C X)) / Pf,
-        // V3 = Pf (masked ones (b B ghat)), rowsum = a (masked G b),
-        // colsum = b (masked G^T a), A3 = suffix sums of rowsum minus strict
-        // suffix sums of colsum; H = a^T b over the channels (k = channel).
+        // holds). With G' = G strictly below its diagonal:
+        // V1 = (G'^T a) / Pf + dy diag G, V3 = Pf (masked ones (b B ghat)),
+        // rowsum = a (G' b) and colsum = b (G'^T a), the sums of M's rows and
+        // columns without its diagonal, and since the rectangle s >= t > r is
+        // the rows s >= t less the columns q >= t, V2 = suffix sums of
+        // a C X + rowsum - colsum; H = a^T b over the channels (k = channel).
+        // (The entries of M between t and s cancel in V2 and carry the gates
+        // of their own rows, not f_t: with every gate above kMcGateMin what
+        // they leave stays at float32's rounding of V2.)
         float ip[4], ra[4], rb[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1131,52 +1146,41 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
           Tb[j][4 * r + g] = rb[r];
         }
         asm volatile("" ::: "memory");
-        f4_t D1 = {0.f, 0.f, 0.f, 0.f}, D2 = D1, D3 = D1, R1 = D1, DH = D1, D4 = D1;
+        f4_t D1 = {0.f, 0.f, 0.f, 0.f}, D2 = D1, D3 = D1, R1 = D1, DH = D1;
         // the 0 / 1 masks are exact in bf16: the masked sums take the 16-bit
         // path with the float32 operand split (mask_pk: four masks packed)
         const auto mask_pk = [](bool m0, bool m1, bool m2, bool m3, uint32_t (&w)[2]) {
           w[0] = (m0 ? 0x3f80u : 0u) | (m1 ? 0x3f800000u : 0u);
           w[1] = (m2 ? 0x3f80u : 0u) | (m3 ? 0x3f800000u : 0u);
         };
-        float v2[4], v3[4];
+        float v2[4], v3[4], Gd[4];  // Gd: G[t][t] of the own rows
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int s = 4 * e + g;
-          const bool ge = s >= arow, le = s <= arow;
-          D1 = mma(ge ? TGs[s][arow] : 0.f, ra[e], D1);
-          v2[e] = ra[e] * cx[e];
+          const bool gt = s > arow, lt = s < arow;
+          D1 = mma(gt ? TGs[s][arow] : 0.f, ra[e], D1);
+          Gd[e] = TGs[s][s];
           v3[e] = rb[e] * bg[e];
-          R1 = mma(le ? Gp[e] : 0.f, rb[e], R1);
+          R1 = mma(lt ? Gp[e] : 0.f, rb[e], R1);
           DH = mma(Ta[s][j], Tb[s][j], DH);
         }
-        uint32_t mge[2], mle[2], mgt[2];
+        uint32_t mge[2], mlt[2];
         mask_pk(g >= arow, 4 + g >= arow, 8 + g >= arow, 12 + g >= arow, mge);
-        mask_pk(g <= arow, 4 + g <= arow, 8 + g <= arow, 12 + g <= arow, mle);
-        mask_pk(g > arow, 4 + g > arow, 8 + g > arow, 12 + g > arow, mgt);
+        mask_pk(g < arow, 4 + g < arow, 8 + g < arow, 12 + g < arow, mlt);
         {
           uint32_t h[2], md[2], lo[2];
+          split4_bf16(v3, h, md, lo);
+          D3 = mma_x3(mlt, h, md, lo, D3);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v2[e] = ra[e] * (cx[e] + R1[e]) - rb[e] * D1[e];
           split4_bf16(v2, h, md, lo);
           D2 = mma_x3(mge, h, md, lo, D2);
-          split4_bf16(v3, h, md, lo);
-          D3 = mma_x3(mle, h, md, lo, D3);
-        }
-        {
-          float v4[4], v5[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v4[e] = ra[e] * R1[e], v5[e] = -(rb[e] * D1[e]);
-          uint32_t h4[2], m4[2], l4[2], h5[2], m5[2], l5[2];
-          split4_bf16(v4, h4, m4, l4);
-          split4_bf16(v5, h5, m5, l5);
-          D4 = mma_k32<bf16_t>(mge, mgt, h4, h5, D4);
-          D4 = mma_k32<bf16_t>(mge, mgt, m4, m5, D4);
-          D4 = mma_k32<bf16_t>(mge, mgt, l4, l5, D4);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          V1[r] = D1[r] * ip[r];
-          V2[r] = D2[r] * ip[r];
+          V1[r] = fmaf(D1[r], ip[r], dy_o[r] * Gd[r]);
+          V2[r] = D2[r];
           V3[r] = D3[r] * pf[r];
-          A3[r] = D4[r];
           // lane (j, g) holds H[4g + r][j], zero for j > 4g + r
           const float h = j <= 4 * g + r ? DH[r] : 0.f;
           TH[4 * g + r][4 * (j & 3) + (j >> 2)] = h;
@@ -1190,8 +1194,9 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
           TGm[arow][4 * r + g] = Gp[r];
           TGT[4 * r + g][arow] = Gp[r];
         }
-        // ---- V1 = sum_{s>=t} P[s,t] dy_s G[s][t], V2 = sum_{s>=t} P[s,t] dy_s (C X)_s
-        // (Horner from s = 15 down), V3 = sum_{r<=t} P[t,r] w_r (B ghat)_r
+        // ---- V1 and the C X part of V2 (Horner from s = 15 down), V3 =
+        // sum_{r<t} P[t,r] w_r (B ghat)_r (Horner from r = 0 up, the row t
+        // itself only decays)
 #pragma unroll
         for (int r = 0; r < 4; ++r) Tx1[j][4 * r + g] = cx[r], Tx2[j][4 * r + g] = bg[r];
         asm volatile("" ::: "memory");
@@ -1222,7 +1227,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
             }
           }
           V1[r] = a1;
-          V2[r] = a2;
+          V2[r] = pf[r] * a2;
           float a3 = 0.f;
 #pragma unroll
           for (int q4 = 0; q4 <= 4 * r; q4 += 4) {
@@ -1232,34 +1237,33 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const int q = q4 + e;
-              if (q <= 4 * r) {
+              if (q < 4 * r)
                 a3 = fmaf(a3, fa[q], w4[e] * b4[e]);
-              } else {
-                const bool in = q <= t;
-                a3 = fmaf(a3, in ? fa[q] : 1.f, in ? w4[e] * b4[e] : 0.f);
-              }
+              else
+                a3 = fmaf(a3, q <= t ? fa[q] : 1.f, q < t ? w4[e] * b4[e] : 0.f);
             }
           }
           V3[r] = a3;
         }
-        // ---- rectangle sums A3_t = sum_{s>=t>=r} M[s][r] with M = K G[s][r],
+        // ---- rectangle sums sum_{s>=t>r} M[s][r] with M = K G[s][r],
         // K[s][r] = P[s,r] dy_s w_r; per row block r the K of the own row
         // s = 4r + g (16 slots, q <= 4r + 3) are summed over the wave's 16
         // channels by a transposing butterfly in each 16-lane row, after which
-        // lane j holds slot q = j: H[s][j]
-        float cp[Q], rs[4];
+        // lane j holds slot q = j: H[s][j]. The own row's part of the sum at
+        // t <= s is the running sum of its M before slot t: only entries of
+        // the rectangle are added, so nothing cancels however small f_t is.
+        float cp[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) cp[q] = 0.f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int s = 4 * r + g;
           float hv[Q];
-          float Pz = 0.f, rsum = 0.f;
+          float Pz = 0.f;
 #pragma unroll
           for (int q4 = 4 * r; q4 >= 0; q4 -= 4) {
-            float w4[4], g4[4];
+            float w4[4];
             rd4(&Tw[j][q4], w4);
-            rd4(&TGm[s][q4], g4);
 #pragma unroll
             for (int e = 3; e >= 0; --e) {
               const int q = q4 + e;
@@ -1273,51 +1277,45 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
               } else {
                 Pz = Pz * fa[q + 1];
               }
-              const float kv = Pz * (dy_o[r] * w4[e]);
-              hv[q] = kv;
-              const float mv = kv * g4[e];
-              rsum += mv;
-              cp[q] += mv;
+              hv[q] = Pz * (dy_o[r] * w4[e]);
+            }
+          }
+          float run = 0.f;
+#pragma unroll
+          for (int q4 = 0; q4 <= 4 * r; q4 += 4) {
+            float g4[4];
+            rd4(&TGm[s][q4], g4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int q = q4 + e;
+              cp[q] += q <= s ? run : 0.f;
+              run = fmaf(hv[q], g4[e], run);
             }
           }
 #pragma unroll
           for (int q = 4 * r + 4; q < Q; ++q) hv[q] = 0.f;
-          rs[r] = rsum;
           trd_step<16, Q, Q>(hv, lane);
           // lane j: H[s][j] (zero for j > s: every slot past s held zeros);
           // over r and the lanes every entry of both tiles is written
           TH[s][4 * (j & 3) + (j >> 2)] = hv[0];
           THT[j][4 * (s & 3) + (s >> 2)] = hv[0];
         }
-        // row sums of all 16 rows, and column sums over the channel's lanes
-        // (group g's partials in pool tile 4 + g for g < 3, tile 3 for g = 3)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Tx1[j][4 * r + g] = rs[r];
+        // the sums over the channel's four lanes: group g's parts in pool tile
+        // 4 + g for g < 3, tile 3 for g = 3, with row 4r + g at 4g + r
         {
           float* tc = pl + (g < 3 ? 4 + g : 3) * 16 * TP;
 #pragma unroll
-          for (int q4 = 0; q4 < Q; q4 += 4) wr4(tc + j * TP + q4, cp[q4], cp[q4 + 1], cp[q4 + 2], cp[q4 + 3]);
+          for (int k = 0; k < 4; ++k) wr4(tc + j * TP + 4 * k, cp[k], cp[4 + k], cp[8 + k], cp[12 + k]);
         }
         asm volatile("" ::: "memory");
-        // A3_t = sum_{s>=t} rowsum[s] - sum_{q>t} colsum[q]
         {
-          float sufR = 0.f, sufC = 0.f;
+          float c0[4], c1[4], c2[4], c3[4];
+          rd4(pl + 4 * 16 * TP + j * TP + 4 * g, c0);
+          rd4(pl + 5 * 16 * TP + j * TP + 4 * g, c1);
+          rd4(pl + 6 * 16 * TP + j * TP + 4 * g, c2);
+          rd4(pl + 3 * 16 * TP + j * TP + 4 * g, c3);
 #pragma unroll
-          for (int r = 3; r >= 0; --r) {
-            float r4[4], c0[4], c1[4], c2[4], c3[4], cs[4];
-            rd4(&Tx1[j][4 * r], r4);
-            rd4(pl + 4 * 16 * TP + j * TP + 4 * r, c0);
-            rd4(pl + 5 * 16 * TP + j * TP + 4 * r, c1);
-            rd4(pl + 6 * 16 * TP + j * TP + 4 * r, c2);
-            rd4(pl + 3 * 16 * TP + j * TP + 4 * r, c3);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) cs[e] = (c0[e] + c1[e]) + (c2[e] + c3[e]);
-            const float sR = sufR + r4[3] + (g <= 2 ? r4[2] : 0.f) + (g <= 1 ? r4[1] : 0.f) + (g <= 0 ? r4[0] : 0.f);
-            const float sC = sufC + (g < 3 ? cs[3] : 0.f) + (g < 2 ? cs[2] : 0.f) + (g < 1 ? cs[1] : 0.f);
-            A3[r] = sR - sC;
-            sufR += (r4[0] + r4[1]) + (r4[2] + r4[3]);
-            sufC += (cs[0] + cs[1]) + (cs[2] + cs[3]);
-          }
+          for (int r = 0; r < 4; ++r) V2[r] += (c0[r] + c1[r]) + (c2[r] + c3[r]);
         }
       }
       // ---- outputs of the own rows into the gate tiles (dfl over f, du over
@@ -1327,7 +1325,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       for (int r = 0; r < 4; ++r) {
         const float f_o = Tf[j][4 * r + g], i_o = Ti[j][4 * r + g], w_o = Tw[j][4 * r + g];
         float dws = fmaf(pe[r], bg[r], V1[r]);
-        float xx = fmaf(pf[r], V2[r], A3[r]) + pe[r] * fmaf(pf[r], gX, V3[r]);
+        float xx = V2[r] + pe[r] * fmaf(pf[r], gX, V3[r]);
         q1[r] = pfdy[r];
         q2[r] = w_o * pe[r];
         if constexpr (HALF == 1) {
@@ -1335,7 +1333,7 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
           continue;
         }
         if constexpr (HALF == 2) dws += hdws[r], xx += hxx[r];
-        const float dfl = f_o == 0.f ? 0.f : (1.f - f_o) * fmaf(-w_o, dws, xx);
+        const float dfl = f_o == 0.f ? 0.f : (1.f - f_o) * xx;
         const float du = fmaf(i_o, dws, Dv * dy_o[r]);
         const float dil = (1.f - i_o) * (dws * w_o);
         sgf += dfl;

@@ -104,7 +104,7 @@ struct ScanArgs {
   // arrays below; ldn is the whole N, the entries between channels of ckpt,
   // segZ, seg0 and dh0 and between rows of partB / partC.
   int64_t ldn;
-  float* half;   // N > 64: the first half's terms of dws and xbar . x, [batch][sub-blocks][D][16 rows x 2]
+  float* half;   // N > 64: the first half's terms of dws and f xbar . x_{t-1}, [batch][sub-blocks][D][16 rows x 2]
   float* partG;  // [2][batch * nseg][D]: per-segment sums of dfl, dil (matrix-core backward; NULL: none)
   int N;
   int batch;
@@ -223,6 +223,11 @@ constexpr int kMcDTB = 16 * kMcWB;
 // leaves the normal range only for |dy| below about 2^-96. A hard reset
 // (f = 0) is always below it.
 constexpr float kMcRatioMin = 0x1p-30f;
+// The backward takes them only where also every gate is at least this: the
+// rectangle sums are differences there, whose error does not shrink with f_t
+// (restated in float32, gates at f_logit = +-4, a quarter closed: dfl off by 3.1e-6 of its
+// norm without this bound and 2.1e-6 with it; formed row by row 1.7e-6).
+constexpr float kMcGateMin = 0x1p-6f;
 
 // True when the chunked kernels serve this state size.
 inline bool mc_ok(int64_t N) { return N > 8 && N <= 128; }

@@ -164,3 +164,30 @@ def test_wide_grid_forward_general_n(gpu, N, D):
     y, g = run_hip(ins, gpu)
     ry, rg = oracle_all(ins)
     check_all(y, g, ry, rg)
+
+
+@pytest.mark.parametrize("N", [16, 64, 100, 128])
+@pytest.mark.parametrize("T,f_shift", [(260, -4.0), (260, -9.0), (260, -12.0), (260, -1.5), (2, -3.0), (4, -2.0)])
+def test_deep_gates_general_n(gpu, N, T, f_shift):
+    """Forget gates nearly closed, as test_deep_gates at N = 1: dfl is of the
+    order of the gate and is formed without terms that do not shrink with it.
+    260 rows at -4 and below take the exact decay products but for the last
+    sub-block's four rows; the short ones, and -1.5, take the ratios too."""
+    ins = rand_inputs(2, T, 64, N, seed=N + T, f_shift=f_shift, h0_std=0.3)
+    y, g = run_hip(ins, gpu)
+    ry, rg = oracle_all(ins)
+    check_all(y, g, ry, rg)
+
+
+@pytest.mark.parametrize("N", [24, 64, 128])
+def test_mixed_hard_gates_general_n(gpu, N):
+    """Most gates nearly open, a quarter nearly closed. dfl = (1 - f) f (..) is
+    small for both; its own float32 rounding of 1 - f near f = sigmoid(4) is
+    2^-24 / (1 - f) = 3.3e-6 relative, inside the tolerance."""
+    ins = rand_inputs(2, 200, 64, N, seed=N, h0_std=0.3)
+    g = torch.Generator().manual_seed(N)
+    closed = torch.rand(2, 200, 64, generator=g) < 0.25
+    ins["f_logit"] = torch.where(closed, -4.0, 4.0) + 0.1 * torch.randn(2, 200, 64, generator=g)
+    y, gr = run_hip(ins, gpu)
+    ry, rg = oracle_all(ins)
+    check_all(y, gr, ry, rg)
