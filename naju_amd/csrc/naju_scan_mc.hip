@@ -424,9 +424,12 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
       // intra-sub-block part of y for the own rows t = 4r + g,
       // S[t] = sum_{s<=t} P[t,s] G[t][s] w_s.
       float S[4];
-      if (__all(Pall >= kMcRatioMin)) {
+      const float wsum = (fabsf(w_o[0]) + fabsf(w_o[1])) + (fabsf(w_o[2]) + fabsf(w_o[3]));
+      if (__all(Pall >= kMcRatioMin && wsum < __builtin_inff())) {
         // Every channel of the wave keeps its decay over the sub-block above
-        // kMcRatioMin: P[t,s] = Pf[t] / Pf[s] (products from row 0) in
+        // kMcRatioMin (and its w are finite: the product's zeros above the
+        // diagonal would take a NaN or an infinity of row s into the rows
+        // before it): P[t,s] = Pf[t] / Pf[s] (products from row 0) in
         // floating point, and S = Pf * (masked G) (w / Pf) is one 16 x 16 x 16
         // product: MFMA row i is time row arow(i), k-step e takes row
         // s = 4e + g, whose w / Pf this lane holds (its own row e).
@@ -1115,7 +1118,16 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
       float fmin = fa[0];
 #pragma unroll
       for (int q = 1; q < Q; ++q) fmin = fminf(fmin, fa[q]);
-      if (__all(Pall >= kMcRatioMin && fmin >= kMcGateMin)) {
+      // not finite where any operand of the products below is not (their
+      // masks' zeros would spread it over the rows of the sub-block)
+      float fin = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        fin = fmaf(dy_o[r], Tw[j][4 * r + g], fin);
+        fin = fmaf(cx[r], bg[r], fin);
+        fin = fmaf(Gp[r], Gp[r], fin);
+      }
+      if (__all(Pall >= kMcRatioMin && fmin >= kMcGateMin && fabsf(fin) < __builtin_inff())) {
         // Every channel's decay over the sub-block stays above kMcRatioMin:
         // P[s,t] = Pf[s] / Pf[t] in floating point, with a = Pf dy and
         // b = w / Pf, and every term is a 16 x 16 x 16 product (MFMA row i =
@@ -1277,7 +1289,8 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
               } else {
                 Pz = Pz * fa[q + 1];
               }
-              hv[q] = Pz * (dy_o[r] * w4[e]);
+              // (selected past s, where w may be a NaN of a later row)
+              hv[q] = q < 4 * r || q <= s ? Pz * (dy_o[r] * w4[e]) : 0.f;
             }
           }
           float run = 0.f;

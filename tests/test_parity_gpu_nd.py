@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests._helpers import check_all, oracle_all, rand_inputs, run_abi, run_hip
+from tests._helpers import check, check_all, oracle_all, rand_inputs, run_abi, run_hip, tol_for
 
 pytestmark = pytest.mark.gpu
 
@@ -191,3 +191,28 @@ def test_mixed_hard_gates_general_n(gpu, N):
     y, gr = run_hip(ins, gpu)
     ry, rg = oracle_all(ins)
     check_all(y, gr, ry, rg)
+
+
+@pytest.mark.parametrize("N", [12, 48, 64, 100, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_non_finite_rows_stay_where_they_belong(gpu, N, dtype):
+    """A NaN or an infinity of one row and channel (padding that was never
+    written, say) reaches what the recurrence carries it to and nothing else:
+    y of the rows before it and of the other channels, and every gradient that
+    the float64 loop keeps finite, are those of the loop."""
+    ins = rand_inputs(1, 70, 48, N, seed=N, dtype=dtype, h0_std=0.3)
+    ins["u"][0, 21, 5] = float("nan")
+    ins["u"][0, 44, 17] = float("inf")
+    ins["f_logit"][0, 39, 30] = float("nan")
+    ins["dy"][0, 28, 9] = float("nan")
+    ins["dy"][0, 67, 40] = float("-inf")
+    y, g = run_hip(ins, gpu)
+    with np.errstate(all="ignore"):
+        ry, rg = oracle_all(ins)
+    for k, v, r in [("y", y, ry)] + [(k, v, rg[k]) for k, v in g.items()]:
+        v = v.detach().double().cpu().numpy()
+        ok = np.isfinite(r)
+        assert k == "dD" or ok.any(), k
+        assert np.isfinite(v[ok]).all(), f"{k}: {np.argwhere(ok & ~np.isfinite(v))[:4].tolist()} not finite"
+        if ok.any():
+            check(k, np.where(ok, v, 0.0), np.where(ok, r, 0.0), tol_for(dtype if k not in ("dD", "dh0") else torch.float32))
