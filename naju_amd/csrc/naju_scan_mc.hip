@@ -425,7 +425,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
       // S[t] = sum_{s<=t} P[t,s] G[t][s] w_s.
       float S[4];
       const float wsum = (fabsf(w_o[0]) + fabsf(w_o[1])) + (fabsf(w_o[2]) + fabsf(w_o[3]));
-      if (__all(Pall >= kMcRatioMin && wsum < __builtin_inff())) {
+      if (__all(Pall >= kMcRatioMin && fabsf(wsum) < __builtin_inff())) {
         // Every channel of the wave keeps its decay over the sub-block above
         // kMcRatioMin (and its w are finite: the product's zeros above the
         // diagonal would take a NaN or an infinity of row s into the rows
@@ -1119,15 +1119,18 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
       for (int q = 1; q < Q; ++q) fmin = fminf(fmin, fa[q]);
       // not finite where any operand of the products below is not (their
-      // masks' zeros would spread it over the rows of the sub-block)
-      float fin = 0.f;
+      // masks' zeros would spread it over the rows of the sub-block); G is
+      // not where any entry of B and C is not. (fabsf: without it the compiler
+      // takes a sum of squares to be no NaN.)
+      float fin = 0.f, gsq = 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         fin = fmaf(dy_o[r], Tw[j][4 * r + g], fin);
         fin = fmaf(cx[r], bg[r], fin);
-        fin = fmaf(Gp[r], Gp[r], fin);
+        gsq = fmaf(Gp[r], Gp[r], gsq);
       }
-      if (__all(Pall >= kMcRatioMin && fmin >= kMcGateMin && fabsf(fin) < __builtin_inff())) {
+      const bool bc_fin = __all(fabsf(gsq) < __builtin_inff());
+      if (bc_fin && __all(Pall >= kMcRatioMin && fmin >= kMcGateMin && fabsf(fin) < __builtin_inff())) {
         // Every channel's decay over the sub-block stays above kMcRatioMin:
         // P[s,t] = Pf[s] / Pf[t] in floating point, with a = Pf dy and
         // b = w / Pf, and every term is a 16 x 16 x 16 product (MFMA row i =
@@ -1497,16 +1500,35 @@ __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, in
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[e] = ac0[e] + ac1[e];
         f4_t hp = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (__is_same(TB, bf16_t)) {
-          uint32_t ab[2], hh[2], hm[2], hl[2];
-          rd4h(qd == 0 ? &sh.Bt[buf][16 * m + j][4 * g] : &sh.Ct[buf][16 * m + j][4 * g], ab);
-          split4_bf16(hs, hh, hm, hl);
-          hp = mma_x3(ab, hh, hm, hl, hp);
-        } else {
-          float a4[4];
-          rd4(qd == 0 ? &sh.Bt[buf][16 * m + j][4 * g] : &sh.Ct[buf][16 * m + j][4 * g], a4);
+        const auto& tbc = qd == 0 ? sh.Bt[buf] : sh.Ct[buf];
+        float a4[4];
+        if (bc_fin) {
+          if constexpr (__is_same(TB, bf16_t)) {
+            uint32_t ab[2], hh[2], hm[2], hl[2];
+            rd4h(&tbc[16 * m + j][4 * g], ab);
+            split4_bf16(hs, hh, hm, hl);
+            hp = mma_x3(ab, hh, hm, hl, hp);
+          } else {
+            rd4(&tbc[16 * m + j][4 * g], a4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) hp = mma(a4[e], hs[e], hp);
+            for (int e = 0; e < 4; ++e) hp = mma(a4[e], hs[e], hp);
+          }
+        } else {
+          // a B (C) that is not finite: the zeros of H would take it to the
+          // rows before (after) its own. The finite entries are multiplied;
+          // an output is NaN where an entry in its range is not finite.
+          f4_t bad = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int row = 4 * e + g;
+            a4[e] = (float)tbc[16 * m + j][4 * g + e];
+            const bool ok = fabsf(a4[e]) < __builtin_inff();
+            hp = mma(ok ? a4[e] : 0.f, hs[e], hp);
+            bad = mma(ok ? 0.f : 1.f, (qd == 0 ? row <= j : row >= j) ? 1.f : 0.f, bad);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (bad[r] > 0.f) hp[r] = __builtin_nanf("");
         }
         float* dst = qd == 0 ? a.partC : a.partB;
         const int n = 16 * m + 4 * g;

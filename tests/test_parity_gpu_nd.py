@@ -216,3 +216,22 @@ def test_non_finite_rows_stay_where_they_belong(gpu, N, dtype):
         assert np.isfinite(v[ok]).all(), f"{k}: {np.argwhere(ok & ~np.isfinite(v))[:4].tolist()} not finite"
         if ok.any():
             check(k, np.where(ok, v, 0.0), np.where(ok, r, 0.0), tol_for(dtype if k not in ("dD", "dh0") else torch.float32))
+
+
+@pytest.mark.parametrize("N", [12, 48, 64, 100])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("which,row", [("B", 50), ("C", 36)])
+def test_non_finite_b_or_c_row(gpu, N, dtype, which, row):
+    """A B of one row that is not finite reaches the rows after it only, a C
+    the rows before it in the gradients (and its own y)."""
+    ins = rand_inputs(1, 70, 48, N, seed=N, dtype=dtype, h0_std=0.3)
+    ins[which][0, row, N // 2] = float("nan") if which == "B" else float("inf")
+    y, g = run_hip(ins, gpu)
+    with np.errstate(all="ignore"):
+        ry, rg = oracle_all(ins)
+    for k, v, r in [("y", y, ry)] + [(k, v, rg[k]) for k, v in g.items()]:
+        v = v.detach().double().cpu().numpy()
+        ok = np.isfinite(r)
+        assert np.isfinite(v[ok]).all(), f"{k}: {np.argwhere(ok & ~np.isfinite(v))[:4].tolist()} not finite"
+        if ok.any():
+            check(k, np.where(ok, v, 0.0), np.where(ok, r, 0.0), tol_for(dtype if k not in ("dD", "dh0") else torch.float32))
