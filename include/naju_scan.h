@@ -40,7 +40,8 @@
  *     N > 1, r rows (32, 64 or 128; 0 = the default). The checkpoint holds
  *     the state every r rows (batch*ceil(T/r)*D*N floats).
  *     The default is 16 rows for 9 <= N <= 128 (the state entering every
- *     sub-block of the matrix-core backward) and 32 rows otherwise; a longer
+ *     sub-block of the matrix-core backward; 32 rows at N > 64 up to library
+ *     version 0.1) and 32 rows otherwise; a longer
  *     interval is the memory-light mode of the reference's recompute backend
  *     (naju/cuda/__init__.py:9-12, CK = 32 in naju/cuda/naju_cuda.cu:25):
  *     the forward's time segments always start at multiples of 128 rows
@@ -50,9 +51,9 @@
  *     over u, f_logit, i_logit and B), so the memory held between forward
  *     and backward shrinks r/16-fold at the cost of that pass. Every output
  *     is bitwise the one of the default interval.
- *     Served for 9 <= N <= 64 by naju_scan_fwd and naju_scan_fwd_noalloc;
- *     other N accept only their default (NAJU_ERR_UNSUPPORTED otherwise;
- *     at N > 64 its name is 32 rows).
+ *     Served by naju_scan_fwd and naju_scan_fwd_noalloc: 32, 64 and 128
+ *     rows for 9 <= N <= 64, 32 rows for N > 64; other N accept only their
+ *     default (NAJU_ERR_UNSUPPORTED otherwise).
  *     The backward must be given the forward's flags value for these bits,
  *     and the size queries below have _ex forms that take it.
  *
@@ -99,7 +100,8 @@ extern "C" {
 #define NAJU_ERR_WORKSPACE -3   /* workspace missing or too small          */
 #define NAJU_ERR_LAUNCH -4      /* the HIP runtime rejected a launch       */
 
-/* Library version, (major << 16) | minor. */
+/* Library version, (major << 16) | minor. 0.2: the default checkpoint interval
+ * of N > 64 is 16 rows (32 before). */
 int naju_scan_version(void);
 
 /* Message of the last failing call on this thread ("" if none). */

@@ -2234,12 +2234,12 @@ int64_t gn_ck_rows(int64_t N) { return use_mc(N, true) ? kMcQ : kGnCK; }
 // The checkpoint interval the flags ask for (NAJU_CKPT_ROWS; 0 = the
 // default: the backward's chunk at N = 1, gn_ck_rows at N > 1), or -1 when
 // the shape does not serve it: longer intervals than the default only on the
-// matrix-core path, whose backward recomputes the states between.
+// matrix-core path, whose backward recomputes the states between (at N > 64
+// 32 rows, and 16 by the default's name 0 only, as before that path).
 int ckpt_rows(int flags, int64_t N) {
   const int r = ((flags & NAJU_CKPT_MASK) >> NAJU_CKPT_SHIFT) * 16;
   const int def = N == 1 ? kBChunk : (int)gn_ck_rows(N);
-  // N > 64: 32 rows names the default, which holds the state every sub-block
-  if (mc_ok(N) && !mc_ext_ok(N)) return r == 0 || r == kGnCK ? def : -1;
+  if (mc_ok(N) && !mc_ext_ok(N)) return r == 0 ? def : (r == kGnCK ? r : -1);
   if (r == 0 || r == def) return def;
   // 2, 4, ... kMcSegUnit sub-blocks: intervals that divide the forward's
   // segment unit
@@ -2273,15 +2273,15 @@ void place_regions(Layout& l, int64_t batch, int64_t T, int64_t D, int64_t N, bo
   off = align_up(off + seg_units * N * sizeof(float));
   l.off_seg0 = off;
   off = align_up(off + seg_units * N * sizeof(float));
-  // the backward's recomputed state at every sub-block when the forward's
-  // checkpoint interval is longer than the sub-block
   // N > 64: the backward's first half's terms of dws and f xbar . x_{t-1}
   const size_t KS = (size_t)((T + kMcQ - 1) / kMcQ);
   l.off_half = off;
   off = align_up(off + (bwd && mc_ok(N) && !mc_ext_ok(N) ? (size_t)batch * KS * D * 2 * kMcQ * sizeof(float) : 0));
-  const bool dense = bwd && mc_ext_ok(N) && l.ck_rows > kMcQ;
+  // the backward's recomputed state at every sub-block when the forward's
+  // checkpoint interval is longer than the sub-block
+  const bool dense = bwd && mc_ok(N) && l.ck_rows > kMcQ;
   l.off_dense = off;
-  off = align_up(off + (dense ? (size_t)batch * ((T + kMcQ - 1) / kMcQ) * D * N * sizeof(float) : 0));
+  off = align_up(off + (dense ? (size_t)batch * KS * D * N * sizeof(float) : 0));
   l.total = off;
 }
 
@@ -2475,7 +2475,7 @@ unsigned small_grid(int64_t n) {
 
 extern "C" {
 
-int naju_scan_version(void) { return (0 << 16) | 1; }
+int naju_scan_version(void) { return (0 << 16) | 2; }
 
 const char* naju_scan_last_error(void) { return g_err; }
 
@@ -2483,7 +2483,7 @@ int64_t naju_scan_ckpt_elems_ex(int64_t batch, int64_t T, int64_t D, int64_t N, 
                                 int bc_dtype, int flags) {
   if (check_common(batch, T, D, N, x_dtype, gate_dtype, bc_dtype) != NAJU_OK) return -1;
   const int rows = ckpt_rows(flags, N);
-  if (rows < 0) return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64)",
+  if (rows < 0) return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64, 32 rows at N > 64)",
                             ((flags & NAJU_CKPT_MASK) >> NAJU_CKPT_SHIFT) * 16, (long long)N), -1;
   // N = 1: one state per backward chunk; N > 1: the state every `rows` rows
   if (N > 1) return batch * ((T + rows - 1) / rows) * D * N;
@@ -2500,7 +2500,7 @@ size_t naju_scan_workspace_bytes_ex(int64_t batch, int64_t T, int64_t D, int64_t
                                     int bc_dtype, int flags) {
   if (check_common(batch, T, D, N, x_dtype, gate_dtype, bc_dtype) != NAJU_OK) return 0;
   const int rows = ckpt_rows(flags, N);
-  if (rows < 0) return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64)",
+  if (rows < 0) return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64, 32 rows at N > 64)",
                             ((flags & NAJU_CKPT_MASK) >> NAJU_CKPT_SHIFT) * 16, (long long)N), 0;
   const size_t f = make_layout(batch, T, D, N, x_dtype, gate_dtype, false, SIZE_MAX, rows).total;
   const size_t b = make_layout(batch, T, D, N, x_dtype, gate_dtype, true, SIZE_MAX, rows).total;
@@ -2569,7 +2569,7 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
     return fail(NAJU_ERR_INVALID, "unknown flag bits 0x%x", flags);
   const int ck_rows = ckpt_rows(flags, N);
   if (ck_rows < 0)
-    return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64)",
+    return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64, 32 rows at N > 64)",
                 ((flags & NAJU_CKPT_MASK) >> NAJU_CKPT_SHIFT) * 16, (long long)N);
   const int out_f32 = flags & NAJU_FLAG_OUT_F32;
   hipStream_t st = (hipStream_t)stream;
@@ -2808,7 +2808,7 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
     return fail(NAJU_ERR_INVALID, "unknown flag bits 0x%x", flags);
   const int ck_rows = ckpt_rows(flags, N);
   if (ck_rows < 0)
-    return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64)",
+    return fail(NAJU_ERR_UNSUPPORTED, "checkpoint interval %d rows is not served at N=%lld (served: 32, 64 and 128 rows at 9 <= N <= 64, 32 rows at N > 64)",
                 ((flags & NAJU_CKPT_MASK) >> NAJU_CKPT_SHIFT) * 16, (long long)N);
   const int out_f32 = flags & NAJU_FLAG_OUT_F32;
   hipStream_t st = (hipStream_t)stream;

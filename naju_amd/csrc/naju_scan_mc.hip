@@ -1610,7 +1610,7 @@ mc_fwd_t pick_fwd_np(int np, bool rec) {
     case 16: return rec ? mc_fwd_kernel<16, true, TU, TG, TB> : mc_fwd_kernel<16, false, TU, TG, TB>;
     case 32: return rec ? mc_fwd_kernel<32, true, TU, TG, TB> : mc_fwd_kernel<32, false, TU, TG, TB>;
     case 64: return rec ? mc_fwd_kernel<64, true, TU, TG, TB> : mc_fwd_kernel<64, false, TU, TG, TB>;
-    default: return mc_fwd_kernel<128, false, TU, TG, TB>;  // (no checkpoint intervals at N > 64)
+    default: return rec ? mc_fwd_kernel<128, true, TU, TG, TB> : mc_fwd_kernel<128, false, TU, TG, TB>;
   }
 }
 

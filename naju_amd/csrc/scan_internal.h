@@ -231,7 +231,7 @@ constexpr float kMcGateMin = 0x1p-6f;
 
 // True when the chunked kernels serve this state size.
 inline bool mc_ok(int64_t N) { return N > 8 && N <= 128; }
-// ... with strided B / C, gate-gradient layouts and checkpoint intervals.
+// ... with strided B / C, gate-gradient layouts and every checkpoint interval.
 inline bool mc_ext_ok(int64_t N) { return N > 8 && N <= 64; }
 // Entries of the state in the backward's first half at N > 64.
 constexpr int kMcHalf = 64;

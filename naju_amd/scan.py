@@ -395,9 +395,9 @@ def naju_scan_hip(u, f_logit, i_logit, B, C, D_skip, h0=None, return_final_state
     """y = scan(u, f_logit, i_logit, B, C, D_skip[, h0]) on the GPU (see module
     doc); (y, hT) with return_final_state=True. ckpt_rows: the checkpoint
     interval kept for the backward (None = NAJU_CKPT_ROWS from the
-    environment where served, else the default; 32, 64 or 128 rows, served
-    at 9 <= N <= 64, is the memory-light mode: the backward recomputes the
-    states between, with bitwise the same outputs).
+    environment at 9 <= N <= 64, else the default; 32, 64 or 128 rows, served
+    at 9 <= N <= 64, and 32 rows at N > 64 are the memory-light mode: the
+    backward recomputes the states between, with bitwise the same outputs).
 
     du_skip ([D], no gradient): the backward forms du = i dws + du_skip dy
     instead of i dws + D_skip dy (the forward still adds D_skip u to y). A

@@ -399,7 +399,7 @@ def test_checkpoint_interval_size_queries_and_checks():
     assert ws64 >= ws0 + B_ * (T // 16) * D * 64 * 4
     # ragged T: the last interval is partial
     assert L.naju_scan_ckpt_elems_ex(2, 300, 96, 33, F32, F32, F32, fl(64)) == 2 * 5 * 96 * 33
-    # other N: only the default interval (32 rows at N <= 8 and N > 64, the
+    # other N: only the default interval (32 rows at N <= 8, the
     # backward's chunk at N = 1)
     assert L.naju_scan_ckpt_elems_ex(2, 300, 96, 4, F32, F32, F32, fl(32)) == 2 * 10 * 96 * 4
     for N, rows in ((4, 64), (128, 64), (1, 32), (8, 16)):
