@@ -101,7 +101,8 @@ extern "C" {
 #define NAJU_ERR_LAUNCH -4      /* the HIP runtime rejected a launch       */
 
 /* Library version, (major << 16) | minor. 0.2: the default checkpoint interval
- * of N > 64 is 16 rows (32 before). */
+ * of N > 64 is 16 rows (32 before); the status mirror is an argument of the
+ * calls (naju_scan_fwd_mirrored, naju_scan_bwd_mirrored). */
 int naju_scan_version(void);
 
 /* Message of the last failing call on this thread ("" if none). */
@@ -265,14 +266,24 @@ int naju_scan_fwd_noalloc(const void* u, const void* f_logit,
 int naju_scan_workspace_status(const void* workspace, void* stream,
                                uint32_t* status);
 
-/* Gives the workspace's status word a mirror: a kernel that records a nonzero
- * status also stores it at `mirror`, a word of pinned host memory that device
- * code can write (hipHostMalloc), which the caller may read at any time and
- * clears itself. Queued on `stream` (one small kernel); holds until the next
- * such call (NULL: no mirror) or until the workspace is zero-filled. The word
- * must outlive every call that uses the workspace. No counterpart in the
- * reference. */
-int naju_scan_set_status_mirror(void* workspace, uint32_t* mirror, void* stream);
+/* naju_scan_fwd / naju_scan_bwd with a mirror of the status word: a kernel
+ * that records a nonzero status also stores it at `status_mirror`, a word of
+ * pinned host memory that device code can write (hipHostMalloc), which the
+ * caller may read at any time and clears itself. NULL: no mirror. The word
+ * must outlive the call's kernels and, where the call is recorded into a HIP
+ * graph, the graph. (Library version 0.1 kept the mirror's address in the
+ * workspace, naju_scan_set_status_mirror; a failure may mean that the
+ * workspace was never zero-filled, so the address comes with the call now.)
+ * Only the N = 1 kernels record a status. No counterpart in the reference. */
+int naju_scan_fwd_mirrored(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
+                           const float* D_skip, const float* h0, void* y, float* ckpt, float* hT, int64_t batch,
+                           int64_t T, int64_t D, int64_t N, int x_dtype, int gate_dtype, int bc_dtype, int flags,
+                           void* workspace, size_t workspace_bytes, uint32_t* status_mirror, void* stream);
+int naju_scan_bwd_mirrored(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
+                           const float* D_skip, const float* ckpt, const void* dy, void* du, void* dfl, void* dil,
+                           void* dB, void* dC, float* dD, float* dh0, int64_t batch, int64_t T, int64_t D, int64_t N,
+                           int x_dtype, int gate_dtype, int bc_dtype, int flags, void* workspace,
+                           size_t workspace_bytes, uint32_t* status_mirror, void* stream);
 
 /* naju_scan_workspace_status for the static scratch of
  * naju_scan_fwd_noalloc on the current HIP device (synchronises `stream`):

@@ -50,7 +50,8 @@ EXPORTED = (
     "naju_scan_bwd_strided",
     "naju_scan_bwd_ex",
     "naju_scan_workspace_status",
-    "naju_scan_set_status_mirror",
+    "naju_scan_fwd_mirrored",
+    "naju_scan_bwd_mirrored",
     "naju_scan_fwd_noalloc",
     "naju_scan_noalloc_status",
     "naju_mixer_last_error",
@@ -137,8 +138,11 @@ def lib():
     # u, fl, il, B, C, D_skip, h0, y, ckpt, hT, batch, T, D, N, x_dt, g_dt, bc_dt, flags, stream
     L.naju_scan_fwd_noalloc.argtypes = [P] * 10 + [I64] * 4 + [I] * 4 + [P]
     L.naju_scan_fwd_noalloc.restype = I
-    L.naju_scan_set_status_mirror.argtypes = [P, P, P]
-    L.naju_scan_set_status_mirror.restype = I
+    # naju_scan_fwd's / naju_scan_bwd's arguments with the status mirror before the stream
+    L.naju_scan_fwd_mirrored.argtypes = [P] * 10 + [I64] * 4 + [I] * 4 + [P, SZ, P, P]
+    L.naju_scan_fwd_mirrored.restype = I
+    L.naju_scan_bwd_mirrored.argtypes = [P] * 15 + [I64] * 4 + [I] * 4 + [P, SZ, P, P]
+    L.naju_scan_bwd_mirrored.restype = I
     L.naju_scan_workspace_status.argtypes = [P, P, ctypes.POINTER(ctypes.c_uint32)]
     L.naju_scan_workspace_status.restype = I
     L.naju_scan_noalloc_status.argtypes = [P, ctypes.POINTER(ctypes.c_uint32)]

@@ -222,17 +222,13 @@ __global__ void epoch_bump_kernel(uint32_t* hdr) {
 }
 
 // Records a failure in the status word, and in its mirror in host memory when
-// the workspace has one: a caller sees it there without a copy per call (two
-// 4 us copy launches per training step before).
-__device__ __forceinline__ void set_status(uint32_t* hdr, uint32_t v) {
-  __hip_atomic_store(hdr + HDR_STATUS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint64_t m = (uint64_t)hdr[HDR_MIRROR] | (uint64_t)hdr[HDR_MIRROR + 1] << 32;
-  if (m) __hip_atomic_store((uint32_t*)m, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-__global__ void set_mirror_kernel(uint32_t* hdr, uint64_t mirror) {
-  hdr[HDR_MIRROR] = (uint32_t)mirror;
-  hdr[HDR_MIRROR + 1] = (uint32_t)(mirror >> 32);
+// the call gave one: a caller sees it there without a copy per call (two 4 us
+// copy launches per training step before). The mirror's address is a launch
+// argument: a failure may mean that the workspace was never zero-filled, so no
+// address is taken from it.
+__device__ __forceinline__ void set_status(const ScanArgs& a, uint32_t v) {
+  __hip_atomic_store(a.hdr + HDR_STATUS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (a.mirror) __hip_atomic_store(a.mirror, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Workgroup blockIdx.x serves tile blockIdx.x % n_tiles; the chunk comes from
@@ -253,7 +249,7 @@ __device__ __forceinline__ uint32_t take_ticket(const ScanArgs& a, int tile, uin
     if (a.tag == 0u) e = __hip_atomic_load(a.hdr + HDR_EPOCH, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t t = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (t == (uint32_t)a.K - 1) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (t >= (uint32_t)a.K) set_status(a.hdr, 2u);
+    if (t >= (uint32_t)a.K) set_status(a, 2u);
     *s_ticket = t;
     *s_tag = a.tag != 0u ? a.tag : epoch_tag(e);
   }
@@ -371,7 +367,7 @@ __device__ __forceinline__ bool lb_consume(const ScanArgs& a, LookShared<V, W, P
     }
     if (!done && consumed == 0 && ++idle > a.spin_limit) {
       // Bounded wait exceeded: record it and end with a NaN carry.
-      if (lane == 0) set_status(a.hdr, 1u);
+      if (lane == 0) set_status(a, 1u);
 #pragma unroll
       for (int j = 0; j < V; ++j) out[j] = __builtin_nanf("");
       done = 1;
@@ -405,7 +401,7 @@ __device__ __forceinline__ void wg_look_back(const ScanArgs& a, LookShared<V, W,
     // the host asked every hand-off to give up at once (a test hook): the
     // failure path of an exceeded wait, taken without polling
     if (wv == 0) {
-      if (lane == 0) set_status(a.hdr, 1u);
+      if (lane == 0) set_status(a, 1u);
 #pragma unroll
       for (int j = 0; j < V; ++j) out[j] = __builtin_nanf("");
     }
@@ -2560,7 +2556,8 @@ int check_bc_ld(const void* p, const void* q, int64_t N, int dt, int64_t ld, boo
 int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
                   const float* D_skip, const float* h0, void* y, float* ckpt, float* hT, int64_t batch, int64_t T,
                   int64_t D, int64_t N, int x_dtype, int gate_dtype, int bc_dtype, int flags, void* workspace,
-                  size_t workspace_bytes, void* stream, size_t cap, int64_t ldbc) {
+                  size_t workspace_bytes, void* stream, size_t cap, int64_t ldbc,
+                  uint32_t* mirror = nullptr) {
   g_err[0] = 0;
   int rc = check_common(batch, T, D, N, x_dtype, gate_dtype, bc_dtype);
   if (rc) return rc;
@@ -2588,6 +2585,7 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
     return fail(NAJU_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", l.total,
                 workspace ? workspace_bytes : (size_t)0);
   if (!aligned(workspace, 256)) return fail(NAJU_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (!aligned(mirror, 4)) return fail(NAJU_ERR_INVALID, "the status mirror must be 4-byte aligned");
   const size_t va_x = l.V * dsize(x_dtype), va_g = l.V * dsize(gate_dtype);
   const size_t va_y = l.V * (out_f32 ? 4 : dsize(x_dtype));
   const bool vec = (D % l.V == 0) && aligned(u, va_x) && aligned(y, va_y) && aligned(f_logit, va_g) &&
@@ -2605,6 +2603,7 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
   a.hT = hT;
   char* ws = (char*)workspace;
   a.hdr = (uint32_t*)ws;
+  a.mirror = mirror;
   a.agg = (uint64_t*)(ws + l.off_agg);
   a.incl = (uint64_t*)(ws + l.off_incl);
   a.T = T;
@@ -2735,6 +2734,14 @@ int naju_scan_fwd(const void* u, const void* f_logit, const void* i_logit, const
                        bc_dtype, flags, workspace, workspace_bytes, stream, SIZE_MAX, N);
 }
 
+int naju_scan_fwd_mirrored(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
+                           const float* D_skip, const float* h0, void* y, float* ckpt, float* hT, int64_t batch,
+                           int64_t T, int64_t D, int64_t N, int x_dtype, int gate_dtype, int bc_dtype, int flags,
+                           void* workspace, size_t workspace_bytes, uint32_t* status_mirror, void* stream) {
+  return scan_fwd_impl(u, f_logit, i_logit, B, C, D_skip, h0, y, ckpt, hT, batch, T, D, N, x_dtype, gate_dtype,
+                       bc_dtype, flags, workspace, workspace_bytes, stream, SIZE_MAX, N, status_mirror);
+}
+
 int naju_scan_fwd_strided(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
                           const float* D_skip, const float* h0, void* y, float* ckpt, float* hT, int64_t batch,
                           int64_t T, int64_t D, int64_t N, int64_t bc_ld, int x_dtype, int gate_dtype, int bc_dtype,
@@ -2791,7 +2798,8 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
                          void* dB, void* dC, float* dD, float* dh0, int64_t batch, int64_t T, int64_t D, int64_t N,
                          int x_dtype, int gate_dtype, int bc_dtype, int flags, void* workspace,
                          size_t workspace_bytes, void* stream, int64_t ldbc, int64_t lddbc, int64_t ldg = -1,
-                         int dg_req = -1, float* dfl_sum = nullptr, float* dil_sum = nullptr) {
+                         int dg_req = -1, float* dfl_sum = nullptr, float* dil_sum = nullptr,
+                         uint32_t* mirror = nullptr) {
   g_err[0] = 0;
   int rc = check_common(batch, T, D, N, x_dtype, gate_dtype, bc_dtype);
   if (rc) return rc;
@@ -2837,6 +2845,7 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
     return fail(NAJU_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", l.total,
                 workspace ? workspace_bytes : (size_t)0);
   if (!aligned(workspace, 256)) return fail(NAJU_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (!aligned(mirror, 4)) return fail(NAJU_ERR_INVALID, "the status mirror must be 4-byte aligned");
   const size_t va_x = l.V * dsize(x_dtype), va_g = l.V * dsize(gate_dtype);
   const size_t vo_x = out_f32 ? l.V * 4 : va_x, vo_g = out_f32 ? l.V * 4 : va_g;
   const bool vec = (D % l.V == 0) && aligned(u, va_x) && aligned(dy, va_x) && aligned(du, vo_x) &&
@@ -2856,6 +2865,7 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
   a.dh0 = dh0;
   char* ws = (char*)workspace;
   a.hdr = (uint32_t*)ws;
+  a.mirror = mirror;
   a.agg = (uint64_t*)(ws + l.off_agg);
   a.incl = (uint64_t*)(ws + l.off_incl);
   a.partB = dB ? (float*)(ws + l.off_partB) : nullptr;
@@ -2983,6 +2993,16 @@ int naju_scan_bwd(const void* u, const void* f_logit, const void* i_logit, const
                        x_dtype, gate_dtype, bc_dtype, flags, workspace, workspace_bytes, stream, N, N);
 }
 
+int naju_scan_bwd_mirrored(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
+                           const float* D_skip, const float* ckpt, const void* dy, void* du, void* dfl, void* dil,
+                           void* dB, void* dC, float* dD, float* dh0, int64_t batch, int64_t T, int64_t D, int64_t N,
+                           int x_dtype, int gate_dtype, int bc_dtype, int flags, void* workspace,
+                           size_t workspace_bytes, uint32_t* status_mirror, void* stream) {
+  return scan_bwd_impl(u, f_logit, i_logit, B, C, D_skip, ckpt, dy, du, dfl, dil, dB, dC, dD, dh0, batch, T, D, N,
+                       x_dtype, gate_dtype, bc_dtype, flags, workspace, workspace_bytes, stream, N, N, -1, -1, nullptr,
+                       nullptr, status_mirror);
+}
+
 int naju_scan_bwd_strided(const void* u, const void* f_logit, const void* i_logit, const void* B, const void* C,
                           const float* D_skip, const float* ckpt, const void* dy, void* du, void* dfl, void* dil,
                           void* dB, void* dC, float* dD, float* dh0, int64_t batch, int64_t T, int64_t D, int64_t N,
@@ -3010,7 +3030,7 @@ int naju_scan_bwd_ex(const void* u, const void* f_logit, const void* i_logit, co
 int naju_scan_workspace_status(const void* workspace, void* stream, uint32_t* status) {
   if (!workspace || !status) return fail(NAJU_ERR_INVALID, "null workspace or status pointer");
   hipStream_t st = (hipStream_t)stream;
-  uint32_t hdr[4];
+  uint32_t hdr[2];
   if (hipMemcpyAsync(hdr, workspace, sizeof(hdr), hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return fail(NAJU_ERR_LAUNCH, "could not read the workspace header");
@@ -3026,17 +3046,6 @@ int naju_scan_workspace_status(const void* workspace, void* stream, uint32_t* st
         hipStreamSynchronize(st) != hipSuccess)
       return fail(NAJU_ERR_LAUNCH, "could not clear the workspace header");
   }
-  return NAJU_OK;
-}
-
-int naju_scan_set_status_mirror(void* workspace, uint32_t* mirror, void* stream) {
-  g_err[0] = 0;
-  if (!workspace) return fail(NAJU_ERR_INVALID, "null workspace pointer");
-  if (!aligned(workspace, 256)) return fail(NAJU_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-  if (!aligned(mirror, 4)) return fail(NAJU_ERR_INVALID, "the mirror must be 4-byte aligned");
-  hipLaunchKernelGGL(set_mirror_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, (uint32_t*)workspace,
-                     (uint64_t)(uintptr_t)mirror);
-  if (hipGetLastError() != hipSuccess) return fail(NAJU_ERR_LAUNCH, "mirror launch failed");
   return NAJU_OK;
 }
 

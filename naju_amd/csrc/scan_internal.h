@@ -53,10 +53,9 @@ __device__ __forceinline__ void st_any(void* p, int dt, int64_t i, float v) {
 // ever overlaps (so its counters, which must start at zero, are only ever
 // written by the ticket logic below): word 0 is the status word; word 1 the
 // device epoch (look-back tags of launches recorded into a HIP graph, see
-// epoch_bump_kernel); words 2 and 3 the address of the status word's mirror in
-// host memory (0: none); tile t's ticket counter is word
-// kCtrBase + t*kCtrStride, t < kMaxTiles.
-enum { HDR_STATUS = 0, HDR_EPOCH = 1, HDR_MIRROR = 2 };
+// epoch_bump_kernel); tile t's ticket counter is word kCtrBase + t*kCtrStride,
+// t < kMaxTiles.
+enum { HDR_STATUS = 0, HDR_EPOCH = 1 };
 constexpr int kCtrBase = 64;
 constexpr int kCtrStride = 4;
 constexpr int kMaxTiles = 1 << 16;
@@ -93,6 +92,7 @@ struct ScanArgs {
   int nseg;      // N > 1: time segments (one workgroup each per channel tile)
   int seg_sc;    // N > 1: sub-chunks per time segment
   uint32_t* hdr;
+  uint32_t* mirror;  // N = 1: host word that a failing kernel also stores its status in (or null)
   uint64_t* agg;   // [K][n_tiles][2][CH]
   uint64_t* incl;  // [K][n_tiles][CH]
   int64_t T;

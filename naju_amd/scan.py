@@ -21,7 +21,7 @@ Public surface, mirroring /root/reference/naju/scan.py:
 * ``workspace_status(device=None)`` -- reads (and clears) the status word of
   the current stream's workspace. A kernel whose carry hand-off fails (only
   N = 1 kernels hand carries between workgroups) also stores it in the
-  workspace's mirror word in pinned host memory; the next call or backward on
+  stream's mirror word in pinned host memory; the next call or backward on
   the same stream reads that word (no synchronisation, no copy) and raises
   ``NajuScanError`` when a hand-off failed, clearing both so the workspace is
   usable again. ``NAJU_CHECK_STATUS=1`` checks synchronously
@@ -60,8 +60,8 @@ class _Workspace:
     """One zero-filled workspace per (device, stream), grown on demand. The
     kernels return it to a reusable state after every call, so it is zeroed
     only when (re)allocated. Per (device, stream) also the pinned host word
-    that mirrors its status word: the tensor that holds it and its view as a
-    C integer."""
+    that N = 1 calls mirror its status word in: the tensor that holds it and
+    its view as a C integer."""
 
     def __init__(self):
         self._bufs = {}
@@ -70,20 +70,22 @@ class _Workspace:
     def get(self, device, stream, nbytes):
         key = (device.index, stream)
         buf = self._bufs.get(key)
-        ent = self._status.get(key)
-        fresh = buf is None or buf.numel() < nbytes
-        if fresh or ent is None:
-            if fresh:
-                buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-                self._bufs[key] = buf
-            if ent is None and not torch.cuda.is_current_stream_capturing():
-                # (pinned memory is not allocated during a capture: a later
-                # call outside it gives the workspace its mirror)
-                word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-                ent = self._status[key] = (word, ctypes.c_uint32.from_address(word.data_ptr()))
-            if ent is not None:
-                _lib.check(_lib.lib().naju_scan_set_status_mirror(buf.data_ptr(), ent[0].data_ptr(), stream))
+        if buf is None or buf.numel() < nbytes:
+            buf = self._bufs[key] = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         return buf
+
+    def mirror(self, device, stream):
+        """Address of the stream's mirror word, or None in a capture that
+        comes before the stream's first call outside one (pinned memory is
+        not allocated during a capture)."""
+        key = (device.index, stream)
+        ent = self._status.get(key)
+        if ent is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            ent = self._status[key] = (word, ctypes.c_uint32.from_address(word.data_ptr()), word.data_ptr())
+        return ent[2]
 
 
 _WS = _Workspace()
@@ -254,7 +256,9 @@ def _forward(u, f_logit, i_logit, B, C, D_skip, h0, want_hT, ckpt_rows, need_gra
     L = _lib.lib()
     args = (u_.data_ptr(), fl_.data_ptr(), il_.data_ptr(), B_.data_ptr(), C_.data_ptr(), D_.data_ptr(), _ptr(h0_),
             y.data_ptr(), _ptr(ckpt), _ptr(hT), Bsz, T, D, N)
-    if bc_ld != N:
+    if N == 1:
+        rc = L.naju_scan_fwd_mirrored(*args, *dts, flags, ws.data_ptr(), ws.numel(), _WS.mirror(dev, stream), stream)
+    elif bc_ld != N:
         rc = L.naju_scan_fwd_strided(*args, bc_ld, *dts, flags, ws.data_ptr(), ws.numel(), stream)
     else:
         rc = L.naju_scan_fwd(*args, *dts, flags, ws.data_ptr(), ws.numel(), stream)
@@ -362,10 +366,11 @@ class NajuScanHip(torch.autograd.Function):
                 _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD), _ptr(dh0),
                 Bsz, T, D, N, ctx.bc_ld, dbc_ld, *dts, flags, ws.data_ptr(), ws.numel(), stream))
         else:
-            rc = L.naju_scan_bwd(
-                u_.data_ptr(), fl_.data_ptr(), il_.data_ptr(), B_.data_ptr(), C_.data_ptr(), D_b.data_ptr(),
-                ckpt.data_ptr(), dy.data_ptr(), _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD),
-                _ptr(dh0), Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel(), stream)
+            args = (u_.data_ptr(), fl_.data_ptr(), il_.data_ptr(), B_.data_ptr(), C_.data_ptr(), D_b.data_ptr(),
+                    ckpt.data_ptr(), dy.data_ptr(), _ptr(du), _ptr(dfl), _ptr(dil), _ptr(dB), _ptr(dC), _ptr(dD),
+                    _ptr(dh0), Bsz, T, D, N, *dts, flags, ws.data_ptr(), ws.numel())
+            rc = L.naju_scan_bwd_mirrored(*args, _WS.mirror(dev, stream), stream) if N == 1 else L.naju_scan_bwd(
+                *args, stream)
             if rc:
                 _lib.check(rc)
         _check_status(dev)

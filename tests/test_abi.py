@@ -476,3 +476,15 @@ def test_gate_gradient_layout_rejections():
     assert bwd(16, dg_ld=8) == _lib.ERR_INVALID
     assert bwd(16, dg_ld=18) == _lib.ERR_UNSUPPORTED
     assert bwd(16, dg_dtype=7) == _lib.ERR_INVALID
+
+
+def test_status_mirror_must_be_aligned():
+    """The mirrored calls check the host word before any device work."""
+    L = _lib.lib()
+    fake = 0x1000
+    args = [fake] * 6 + [None, fake, fake, None, 2, 300, 96, 1, F32, F32, F32, 0, fake, 1 << 30]
+    assert L.naju_scan_fwd_mirrored(*args, 0x1002, None) == _lib.ERR_INVALID
+    assert b"mirror" in L.naju_scan_last_error()
+    args = [fake] * 8 + [None] * 7 + [2, 300, 96, 1, F32, F32, F32, 0, fake, 1 << 30]
+    assert L.naju_scan_bwd_mirrored(*args, 0x1002, None) == _lib.ERR_INVALID
+    assert b"mirror" in L.naju_scan_last_error()

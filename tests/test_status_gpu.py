@@ -2,7 +2,7 @@
 
 The N = 1 kernels hand chunk carries between workgroups with bounded waits; a
 wait that gives up writes NaN outputs and sets the workspace's status word.
-The kernel stores that word's mirror in pinned host memory too, and the next
+The kernel stores that word in pinned host memory too, and the next
 naju_scan_hip call (or backward) on the same stream that finds it nonzero
 raises NajuScanError, clearing both so the workspace is usable again. The failures are forced from the host with the library's
 NAJU_DEBUG_SPIN_LIMIT=0 test hook (every hand-off gives up at once, every
@@ -93,3 +93,38 @@ def test_grown_workspace_keeps_its_mirror(gpu, monkeypatch):
             with pytest.raises(NajuScanError):
                 naju_scan_hip(*xs)
             assert bool(torch.isfinite(naju_scan_hip(*xs)).all())
+
+
+def test_workspace_that_was_never_zeroed(gpu):
+    """Every word of the workspace holds the same arbitrary value, the ticket
+    counters and what lies beside them among it: every workgroup's ticket is
+    out of range, so the outputs are NaN and the status is 2, in the header and
+    in the mirror that the call gave. (No address is read from the workspace.)
+    Clearing the status makes it usable."""
+    import ctypes
+    from naju_amd import _lib
+    L = _lib.lib()
+    B, T, D = 2, 1000, 256
+    ins = rand_inputs(B, T, D, 1, seed=5, dtype=torch.float32)
+    xs = [ins[k].to(gpu) for k in NAMES]
+    dts = (_lib.DT_F32,) * 3
+    nb = L.naju_scan_workspace_bytes(B, T, D, 1, *dts)
+    st = torch.cuda.current_stream(gpu).cuda_stream
+    word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+
+    def run(ws):
+        y = torch.empty_like(xs[0])
+        _lib.check(L.naju_scan_fwd_mirrored(*[x.data_ptr() for x in xs], None, y.data_ptr(), None, None, B, T, D, 1,
+                                            *dts, _lib.FLAG_DETERMINISTIC, ws.data_ptr(), nb, word.data_ptr(), st))
+        torch.cuda.synchronize()
+        return y
+
+    good = run(torch.zeros(nb, dtype=torch.uint8, device=gpu))
+    assert int(word[0]) == 0 and bool(torch.isfinite(good).all())
+    ws = torch.full((nb,), 0x40, dtype=torch.uint8, device=gpu)
+    assert bool(torch.isnan(run(ws)).all()) and int(word[0]) == 2
+    got = ctypes.c_uint32(0)
+    _lib.check(L.naju_scan_workspace_status(ws.data_ptr(), st, ctypes.byref(got)))
+    assert got.value == 2
+    word.zero_()
+    assert torch.equal(run(ws), good) and int(word[0]) == 0
