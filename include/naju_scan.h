@@ -285,6 +285,12 @@ int naju_scan_bwd_mirrored(const void* u, const void* f_logit, const void* i_log
                            int x_dtype, int gate_dtype, int bc_dtype, int flags, void* workspace,
                            size_t workspace_bytes, uint32_t* status_mirror, void* stream);
 
+/* The id of the HIP-graph capture that `stream` is part of, 0 when it is not
+ * being captured: a workspace whose zero fill is recorded into a graph is
+ * zeroed when that graph is replayed, so it serves the calls of that capture
+ * only. No counterpart in the reference. */
+uint64_t naju_scan_capture_id(void* stream);
+
 /* naju_scan_workspace_status for the static scratch of
  * naju_scan_fwd_noalloc on the current HIP device (synchronises `stream`):
  * reads its status word and, when it is nonzero, clears it and rewinds the

@@ -52,6 +52,7 @@ EXPORTED = (
     "naju_scan_workspace_status",
     "naju_scan_fwd_mirrored",
     "naju_scan_bwd_mirrored",
+    "naju_scan_capture_id",
     "naju_scan_fwd_noalloc",
     "naju_scan_noalloc_status",
     "naju_mixer_last_error",
@@ -143,6 +144,8 @@ def lib():
     L.naju_scan_fwd_mirrored.restype = I
     L.naju_scan_bwd_mirrored.argtypes = [P] * 15 + [I64] * 4 + [I] * 4 + [P, SZ, P, P]
     L.naju_scan_bwd_mirrored.restype = I
+    L.naju_scan_capture_id.argtypes = [P]
+    L.naju_scan_capture_id.restype = ctypes.c_uint64
     L.naju_scan_workspace_status.argtypes = [P, P, ctypes.POINTER(ctypes.c_uint32)]
     L.naju_scan_workspace_status.restype = I
     L.naju_scan_noalloc_status.argtypes = [P, ctypes.POINTER(ctypes.c_uint32)]

@@ -3049,6 +3049,13 @@ int naju_scan_workspace_status(const void* workspace, void* stream, uint32_t* st
   return NAJU_OK;
 }
 
+uint64_t naju_scan_capture_id(void* stream) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &cs, &id) != hipSuccess) return 0;
+  return cs == hipStreamCaptureStatusActive ? (uint64_t)id : 0;
+}
+
 int naju_scan_noalloc_status(void* stream, uint32_t* status) {
   g_err[0] = 0;
   if (!status) return fail(NAJU_ERR_INVALID, "null status pointer");

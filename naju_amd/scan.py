@@ -59,19 +59,29 @@ def _ptr(t):
 class _Workspace:
     """One zero-filled workspace per (device, stream), grown on demand. The
     kernels return it to a reusable state after every call, so it is zeroed
-    only when (re)allocated. Per (device, stream) also the pinned host word
-    that N = 1 calls mirror its status word in: the tensor that holds it and
-    its view as a C integer."""
+    only when (re)allocated. A workspace allocated while the stream is captured
+    into a graph is zeroed by that graph's replays, so it serves that capture
+    alone: (capture id, buffer) per key, apart from the others. Per (device,
+    stream) also the pinned host word that N = 1 calls mirror its status word
+    in: the tensor that holds it, its view as a C integer and its address."""
 
     def __init__(self):
         self._bufs = {}
+        self._captured = {}
         self._status = {}
 
     def get(self, device, stream, nbytes):
         key = (device.index, stream)
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
-            buf = self._bufs[key] = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            capture = _lib.lib().naju_scan_capture_id(stream)
+            cid, buf = self._captured.get(key, (0, None))
+            if not capture or cid != capture or buf.numel() < nbytes:
+                buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+                if capture:
+                    self._captured[key] = (capture, buf)
+                else:
+                    self._bufs[key] = buf
         return buf
 
     def mirror(self, device, stream):
@@ -131,18 +141,22 @@ _STATUS_MSG = {1: "a carry hand-off between workgroups exceeded its bounded wait
 def workspace_status(device=None):
     """Status word of the workspace of (device, current stream): 0 healthy,
     1 or 2 after a failed call (then cleared, so the workspace is usable
-    again). Synchronises the stream."""
+    again). Synchronises the stream. Where calls captured on this stream have
+    a workspace of their own, its word is read too."""
     dev = torch.device("cuda", torch.cuda.current_device() if device is None else torch.device(device).index)
     stream = _stream_handle(dev)
-    buf = _WS._bufs.get((dev.index, stream))
-    if buf is None:
-        return 0
-    st = ctypes.c_uint32(0)
-    _lib.check(_lib.lib().naju_scan_workspace_status(buf.data_ptr(), stream, ctypes.byref(st)))
-    ent = _WS._status.get((dev.index, stream))
+    key = (dev.index, stream)
+    found = 0
+    for buf in (_WS._bufs.get(key), _WS._captured.get(key, (0, None))[1]):
+        if buf is not None:
+            st = ctypes.c_uint32(0)
+            _lib.check(_lib.lib().naju_scan_workspace_status(buf.data_ptr(), stream, ctypes.byref(st)))
+            # (a captured workspace holds anything until its first replay)
+            found = found or (st.value if st.value in _STATUS_MSG else 0)
+    ent = _WS._status.get(key)
     if ent is not None:  # (the stream is idle here)
         ent[1].value = 0
-    return st.value
+    return found
 
 
 def _check_status(dev):

@@ -132,8 +132,8 @@ def test_graph_back_to_back_replays_with_new_inputs(gpu, N, shape, dtype):
 @pytest.mark.parametrize("N,shape,dtype", [(1, (2, 1000, 256), torch.bfloat16), (16, (2, 300, 128), torch.float32)])
 def test_wrapper_inference_forward_captures(gpu, N, shape, dtype):
     """naju_scan_hip's no-grad forward captured into a graph through the
-    Python wrapper: its asynchronous status watching stays out of the capture
-    (no copy recorded, no event queried while capturing), and every replay on
+    Python wrapper: nothing of its status watching is recorded (a failing
+    kernel stores to the stream's mirror word by itself), and every replay on
     new inputs equals an eager call on them bitwise (with torch's
     deterministic mode on, which selects fixed-order N = 1 carries)."""
     from naju_amd import naju_scan_hip
@@ -163,3 +163,50 @@ def test_wrapper_inference_forward_captures(gpu, N, shape, dtype):
             assert torch.equal(y, ref), f"replay {rep} differs from an eager call on its inputs"
     finally:
         torch.use_deterministic_algorithms(was)
+
+
+@pytest.mark.parametrize("N", [1, 16])
+def test_workspace_born_in_a_capture(gpu, monkeypatch, N):
+    """A stream's first calls are captured ones: their workspace is zeroed by
+    the graph's replays, so neither an eager call nor a second capture uses it.
+    The second graph is right when it is replayed before the first, eager calls
+    between replays are right, and a failed hand-off of an eager call after
+    replays is still reported."""
+    from naju_amd import naju_scan_hip
+    from naju_amd._lib import NajuScanError
+    from naju_amd.scan import _WS
+    names = ("u", "f_logit", "i_logit", "B", "C", "D_skip")
+    ins = rand_inputs(2, 4096, 256, N, seed=7, dtype=torch.float32)
+    t = [ins[k].to(gpu) for k in names]
+    with torch.no_grad():
+        ref = naju_scan_hip(*t)
+        torch.cuda.synchronize()
+        s = torch.cuda.Stream(gpu)
+        key = (gpu.index, s.cuda_stream)
+        for d in (_WS._bufs, _WS._captured, _WS._status):  # (a stream handle may be one that was used before)
+            d.pop(key, None)
+        graphs = []
+        with torch.cuda.stream(s):
+            for _ in range(2):
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, stream=s):
+                    y = naju_scan_hip(*t)
+                graphs.append((g, y))
+            assert key not in _WS._bufs
+            for g, y in reversed(graphs + graphs):
+                y.fill_(float("nan"))
+                g.replay()
+                e = naju_scan_hip(*t)
+                s.synchronize()
+                torch.testing.assert_close(y, ref, rtol=1e-6, atol=1e-6)
+                torch.testing.assert_close(e, ref, rtol=1e-6, atol=1e-6)
+            if N == 1:
+                monkeypatch.setenv("NAJU_DEBUG_SPIN_LIMIT", "0")
+                naju_scan_hip(*t)
+                monkeypatch.delenv("NAJU_DEBUG_SPIN_LIMIT")
+                graphs[0][0].replay()
+                s.synchronize()
+                with pytest.raises(NajuScanError):
+                    naju_scan_hip(*t)
+            torch.testing.assert_close(naju_scan_hip(*t), ref, rtol=1e-6, atol=1e-6)
+            s.synchronize()
