@@ -70,11 +70,9 @@ struct RawV {
     }
   }
   __device__ __forceinline__ void load(const void* base, uint32_t byte_off) {
-    typedef uint32_t vw __attribute__((ext_vector_type(NW)));
+    typedef typename UserVec<uint32_t, NW, sizeof(TT)>::type vw;
     if constexpr (V * sizeof(TT) == 2) {
       w[0] = *(const uint16_t*)((const char*)base + byte_off);
-    } else if constexpr (NW == 1) {
-      w[0] = *(const uint32_t*)((const char*)base + byte_off);
     } else {
       const vw v = *(const vw*)((const char*)base + byte_off);
 #pragma unroll

@@ -69,21 +69,6 @@ __device__ __forceinline__ float own_decays(const float (&fa)[Q], int g, float (
   return all;
 }
 
-// Four consecutive elements of a stream of element type TT at element
-// offset i from p (4-element aligned when VEC), as float.
-template <typename TT, bool VEC>
-__device__ __forceinline__ void ld4v(const TT* __restrict__ p, uint32_t i, float (&o)[4]) {
-  if constexpr (VEC) {
-    typedef TT v4 __attribute__((ext_vector_type(4)));
-    const v4 v = *reinterpret_cast<const v4*>(p + i);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = to_f32(v[e]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = to_f32(p[i + e]);
-  }
-}
-
 // Four consecutive elements of a stream as loaded: the raw bits (8 bytes
 // for 2-byte types, 16 for float), turned into floats only where they are
 // used. A conversion right after the load would make the wave wait for the
@@ -103,13 +88,13 @@ struct Raw4 {
   }
 };
 
-// Raw4 load of elements i .. i+3 at p (4-element aligned; VEC: one 8- or
-// 16-byte load) or of the elements at offsets o[0..3] (clamped edge lanes).
+// Raw4 load of elements i .. i+3 at p (one 8- or 16-byte load) or of the
+// elements at offsets o[0..3] (clamped edge lanes).
 template <typename TT>
 __device__ __forceinline__ void ld4r(const TT* __restrict__ p, uint32_t i, Raw4<TT>& r) {
   // a clang vector type (not HIP's uint2 / uint4 structs, whose member
   // reads are split into one 4-byte load each)
-  typedef uint32_t vw __attribute__((ext_vector_type(Raw4<TT>::NW)));
+  typedef typename UserVec<uint32_t, Raw4<TT>::NW, sizeof(TT)>::type vw;
   const vw v = *reinterpret_cast<const vw*>(p + i);
 #pragma unroll
   for (int k = 0; k < Raw4<TT>::NW; ++k) r.w[k] = v[k];
@@ -262,7 +247,7 @@ __device__ __forceinline__ void store_state_lines(float* ckw, const f4_t (&X)[MT
       for (int s2 = 0; s2 < 2; ++s2) {
         const int c = 8 * s2 + (lane >> 3), q = 4 * (lane & 7);
         const float4 v = *(const float4*)(tt + c * 36 + q);
-        *(float4*)(ckw + c * (16 * MT) + 32 * h + q) = v;
+        *(user_f4*)(ckw + c * (16 * MT) + 32 * h + q) = user_f4{v.x, v.y, v.z, v.w};
       }
     }
     asm volatile("" ::: "memory");
@@ -499,7 +484,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
         for (int m = 0; m < MT; ++m) {
           const int n = 16 * m + 4 * g;
           if ((N & 3) == 0) {
-            if (n < N) *(float4*)(ck + n) = make_float4(X[m][0], X[m][1], X[m][2], X[m][3]);
+            if (n < N) *(user_f4*)(ck + n) = X[m];
           } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -520,13 +505,13 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
         const int64_t o = ((int64_t)b * T + t0 + rho) * D + dw + cq;
         if (y_dt == NAJU_DTYPE_F32) {
           if (vec)
-            *(float4*)((float*)a.y + o) = make_float4(yv[0], yv[1], yv[2], yv[3]);
+            *(user_f4*)((float*)a.y + o) = user_f4{yv[0], yv[1], yv[2], yv[3]};
           else
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               if (dw + cq + e < D) ((float*)a.y)[o + e] = yv[e];
         } else {
-          typedef TU v4 __attribute__((ext_vector_type(4)));
+          typedef typename UserVec<TU, 4, sizeof(TU)>::type v4;
           if (vec) {
             v4 v;
 #pragma unroll
@@ -551,7 +536,7 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
         for (int m = 0; m < MT; ++m) {
           const int n = 16 * m + 4 * g;
           if ((N & 3) == 0) {
-            if (n < N) *(float4*)(ck + n) = make_float4(X[m][0], X[m][1], X[m][2], X[m][3]);
+            if (n < N) *(user_f4*)(ck + n) = X[m];
           } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -826,8 +811,7 @@ __device__ __forceinline__ void load_ckpt(f4_t (&x)[MT], const ScanArgs& a, int 
   for (int m = 0; m < MT; ++m) {
     const int n = 16 * m + 4 * g;
     if (((N | a.ldn) & 3) == 0) {
-      const float4 v = *(const float4*)(ck + (co + (uint32_t)(n < N ? n : N - 4)));
-      x[m][0] = v.x, x[m][1] = v.y, x[m][2] = v.z, x[m][3] = v.w;
+      x[m] = *(const user_f4*)(ck + (co + (uint32_t)(n < N ? n : N - 4)));
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[m][r] = ck[co + (uint32_t)(n + r < N ? n + r : N - 1)];
@@ -846,7 +830,7 @@ __device__ __forceinline__ float ckpt_val(const f4_t& xm, int r, int n, int N, b
 template <typename TT>
 __device__ __forceinline__ void store_row4(void* p, uint32_t o, const float (*tl)[TP], int cq, int rho, bool vec,
                                            int nval) {
-  typedef TT v4 __attribute__((ext_vector_type(4)));
+  typedef typename UserVec<TT, 4, sizeof(TT)>::type v4;
   v4 x;
 #pragma unroll
   for (int e = 0; e < 4; ++e) x[e] = (TT)tl[cq + e][rho];

@@ -34,6 +34,17 @@ __device__ __forceinline__ float sigm(float x) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
 }
 
+// Vectors in the callers' arrays, of N values of type W. At N > 1 these arrays
+// are aligned to their elements (EB bytes) and no more: a tensor may start one
+// element past an aligned address. The loads and stores are as wide as the
+// vector either way (the target serves unaligned global accesses), but only a
+// type that states the alignment keeps the compiler from counting on more.
+template <typename W, int N, int EB>
+struct UserVec {
+  typedef W type __attribute__((ext_vector_type(N), aligned(EB)));
+};
+typedef UserVec<float, 4, 4>::type user_f4;
+
 // Load with a runtime dtype code (B_t / C_t scalars and other small streams).
 __device__ __forceinline__ float ld_any(const void* p, int dt, int64_t i) {
   if (dt == NAJU_DTYPE_F32) return ((const float*)p)[i];

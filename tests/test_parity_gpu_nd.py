@@ -235,3 +235,38 @@ def test_non_finite_b_or_c_row(gpu, N, dtype, which, row):
         assert np.isfinite(v[ok]).all(), f"{k}: {np.argwhere(ok & ~np.isfinite(v))[:4].tolist()} not finite"
         if ok.any():
             check(k, np.where(ok, v, 0.0), np.where(ok, r, 0.0), tol_for(dtype if k not in ("dD", "dh0") else torch.float32))
+
+
+@pytest.mark.parametrize("N", [8, 24, 32, 64, 100, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_misaligned_streams_general_n(gpu, N, dtype):
+    """Every input one element past an aligned address (and the outputs of the
+    C calls too): bitwise the results of aligned ones, at several segments."""
+    from naju_amd import _lib
+    L = _lib.lib()
+    b, T, D = 2, 290, 96
+    ins = rand_inputs(b, T, D, N, seed=N, dtype=dtype, h0_std=0.3)
+    dts = (_lib.DT_F32 if dtype == torch.float32 else _lib.DT_BF16,) * 3
+    n_ck = L.naju_scan_ckpt_elems(b, T, D, N, *dts)
+    nb = L.naju_scan_workspace_bytes(b, T, D, N, *dts)
+    st = torch.cuda.current_stream(gpu).cuda_stream
+    got = []
+    for off in (0, 1):
+        def at(shape, dt, fill=None):
+            n = int(np.prod(shape))
+            buf = torch.zeros(n + 2, dtype=dt, device=gpu)
+            v = buf[off:off + n].view(shape)
+            return v if fill is None else v.copy_(fill)
+        x = {k: at(v.shape, v.dtype, v.to(gpu)) for k, v in ins.items()}
+        assert off == 0 or x["u"].data_ptr() % (2 * x["u"].element_size()) != 0
+        y, ck = at((b, T, D), dtype), at((n_ck,), torch.float32)
+        g = [at(x[k].shape, x[k].dtype) for k in ("u", "f_logit", "i_logit", "B", "C", "D_skip", "h0")]
+        ws = torch.zeros(nb, dtype=torch.uint8, device=gpu)
+        p = [x[k].data_ptr() for k in ("u", "f_logit", "i_logit", "B", "C", "D_skip")]
+        _lib.check(L.naju_scan_fwd(*p, x["h0"].data_ptr(), y.data_ptr(), ck.data_ptr(), None, b, T, D, N, *dts, 0,
+                                   ws.data_ptr(), nb, st))
+        _lib.check(L.naju_scan_bwd(*p, ck.data_ptr(), x["dy"].data_ptr(), *[v.data_ptr() for v in g], b, T, D, N, *dts,
+                                   0, ws.data_ptr(), nb, st))
+        torch.cuda.synchronize()
+        got.append([y, *g])
+    assert all(torch.equal(v, w) for v, w in zip(*got))
