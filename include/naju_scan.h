@@ -135,6 +135,15 @@ size_t naju_scan_workspace_bytes_ex(int64_t batch, int64_t T, int64_t D,
                                     int64_t N, int x_dtype, int gate_dtype,
                                     int bc_dtype, int flags);
 
+/* Number of time segments that naju_scan_fwd (backward = 0) or naju_scan_bwd
+ * (1) splits T into at this shape (1: none; always at N = 1), or a negative
+ * NAJU_ERR_*. `rows`, if not NULL, gets the rows of a segment (the last one may
+ * be shorter), `map_waves` the waves that form one segment's map at
+ * 9 <= N <= 128 with more than one segment (0 otherwise). The shape alone
+ * decides. No counterpart in the reference. */
+int naju_scan_time_segments(int64_t batch, int64_t T, int64_t D, int64_t N,
+                            int backward, int64_t* rows, int* map_waves);
+
 /* Forward scan. Replaces the forward of every reference backend: the
  * sequential loop of naju/scan.py:79-93, _ChunkScanTriton.forward
  * (naju/chunk_triton.py:148-181), _AffineChunkScan.forward

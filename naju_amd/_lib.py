@@ -44,6 +44,7 @@ EXPORTED = (
     "naju_scan_workspace_bytes",
     "naju_scan_ckpt_elems_ex",
     "naju_scan_workspace_bytes_ex",
+    "naju_scan_time_segments",
     "naju_scan_fwd",
     "naju_scan_bwd",
     "naju_scan_fwd_strided",
@@ -120,6 +121,8 @@ def lib():
     L.naju_scan_ckpt_elems_ex.restype = I64
     L.naju_scan_workspace_bytes_ex.argtypes = [I64] * 4 + [I] * 4
     L.naju_scan_workspace_bytes_ex.restype = SZ
+    L.naju_scan_time_segments.argtypes = [I64] * 4 + [I, ctypes.POINTER(I64), ctypes.POINTER(I)]
+    L.naju_scan_time_segments.restype = I
     # u, fl, il, B, C, D_skip, h0, y, ckpt, hT, batch, T, D, N, x_dt, g_dt, bc_dt, flags, ws, ws_bytes,
     # stream
     L.naju_scan_fwd.argtypes = [P] * 10 + [I64] * 4 + [I] * 4 + [P, SZ, P]

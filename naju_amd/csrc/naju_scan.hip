@@ -2508,6 +2508,17 @@ size_t naju_scan_workspace_bytes(int64_t batch, int64_t T, int64_t D, int64_t N,
   return naju_scan_workspace_bytes_ex(batch, T, D, N, x_dtype, gate_dtype, bc_dtype, 0);
 }
 
+int naju_scan_time_segments(int64_t batch, int64_t T, int64_t D, int64_t N, int backward, int64_t* rows,
+                            int* map_waves) {
+  g_err[0] = 0;
+  const int rc = check_common(batch, T, D, N, NAJU_DTYPE_F32, NAJU_DTYPE_F32, NAJU_DTYPE_F32);
+  if (rc) return rc;
+  const Layout l = make_layout(batch, T, D, N, NAJU_DTYPE_F32, NAJU_DTYPE_F32, backward != 0);
+  if (rows) *rows = (int64_t)l.seg_sc * l.L;
+  if (map_waves) *map_waves = mc_ok(N) && l.nseg > 1 ? mc_map_waves(l.seg_sc * kMcQ) : 0;
+  return l.nseg;
+}
+
 }  // extern "C"
 
 namespace {

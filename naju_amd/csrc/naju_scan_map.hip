@@ -395,6 +395,16 @@ MapPick map_pick(int x_dt, int g_dt, int bc_dt, int64_t N, int64_t D) {
 
 }  // namespace
 
+// As many as leave each four blocks of rows. More waves hide more latency
+// (bf16, 8 x 4096 x 1024, N = 64, 512-row segments: 1 / 2 / 4 waves took 62 / 57
+// / 55 us), but their maps are added at the end (float32, 8 x 2048 x 512, 128
+// rows, backward: 1 / 2 waves 26 / 31 us).
+int mc_map_waves(int rows) {
+  int W = 1;
+  while (W < kMapMaxW && rows >= 2 * W * 4 * KB) W *= 2;
+  return W;
+}
+
 hipError_t mc_map_launch(const ScanArgs& a, bool bwd, int x_dt, int g_dt, hipStream_t st) {
   if (a.nseg <= 1) return hipSuccess;
   const MapPick p = bwd ? map_pick<true>(x_dt, g_dt, a.bc_dt, a.N, a.D)
@@ -402,13 +412,8 @@ hipError_t mc_map_launch(const ScanArgs& a, bool bwd, int x_dt, int g_dt, hipStr
   const int64_t n_ctiles = (a.D + 16 * p.V - 1) / (16 * p.V);
   const int64_t wgs = n_ctiles * a.batch * (a.nseg - 1);
   if (wgs > 0x7fffffff) return hipErrorInvalidValue;
-  // Waves per workgroup: as many as leave each four blocks of rows. More
-  // waves hide more latency (bf16, 8 x 4096 x 1024, N = 64, 512-row segments:
-  // 1 / 2 / 4 waves took 62 / 57 / 55 us), but their maps are added at the
-  // end (float32, 8 x 2048 x 512, 128 rows, backward: 1 / 2 waves 26 / 31 us).
   const int rows = a.seg_sc * kMcQ;
-  int W = 1;
-  while (W < kMapMaxW && rows >= 2 * W * 4 * KB) W *= 2;
+  const int W = mc_map_waves(rows);
   const int wave_rows = (rows + W * KB - 1) / (W * KB) * KB;
   hipLaunchKernelGGL(p.k, dim3((unsigned)wgs), dim3(64 * W), (size_t)W * (p.lds + 16 * p.V * 4), st, a, wave_rows,
                      (int)n_ctiles);

@@ -249,6 +249,8 @@ constexpr int kMcHalf = 64;
 
 // The maps of segments 0 .. nseg-2 (forward) or 1 .. nseg-1 (backward) into
 // segF / segZ (naju_scan_map.hip).
+// Its waves per workgroup, for segments of `rows` rows.
+int mc_map_waves(int rows);
 hipError_t mc_map_launch(const ScanArgs& a, bool bwd, int x_dt, int g_dt, hipStream_t st);
 // Forward: the scan from h0 or the carried segment states, or with a.recomp
 // the recompute of the states from a memory-light checkpoint.

@@ -488,3 +488,15 @@ def test_status_mirror_must_be_aligned():
     args = [fake] * 8 + [None] * 7 + [2, 300, 96, 1, F32, F32, F32, 0, fake, 1 << 30]
     assert L.naju_scan_bwd_mirrored(*args, 0x1002, None) == _lib.ERR_INVALID
     assert b"mirror" in L.naju_scan_last_error()
+
+
+def test_time_segments_query():
+    """naju_scan_time_segments: one segment at N = 1, whole 128-row ones in the
+    matrix-core forward, and the checks of every call."""
+    L = _lib.lib()
+    rows, waves = ctypes.c_int64(), ctypes.c_int()
+    assert L.naju_scan_time_segments(8, 4096, 1024, 1, 0, None, None) == 1
+    n = L.naju_scan_time_segments(8, 4096, 1024, 64, 0, ctypes.byref(rows), ctypes.byref(waves))
+    assert n > 1 and rows.value % 128 == 0 and n == -(-4096 // rows.value) and waves.value in (1, 2, 4)
+    assert L.naju_scan_time_segments(8, 4096, 1024, 129, 0, None, None) == _lib.ERR_UNSUPPORTED
+    assert L.naju_scan_time_segments(8, -1, 1024, 64, 1, None, None) == _lib.ERR_INVALID
