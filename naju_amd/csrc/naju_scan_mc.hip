@@ -409,8 +409,12 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
       // intra-sub-block part of y for the own rows t = 4r + g,
       // S[t] = sum_{s<=t} P[t,s] G[t][s] w_s.
       float S[4];
-      const float wsum = (fabsf(w_o[0]) + fabsf(w_o[1])) + (fabsf(w_o[2]) + fabsf(w_o[3]));
-      if (__all(Pall >= kMcRatioMin && fabsf(wsum) < __builtin_inff())) {
+      bool ratio = __all(Pall >= kMcRatioMin);
+      if (ratio) {
+        const float wsum = (fabsf(w_o[0]) + fabsf(w_o[1])) + (fabsf(w_o[2]) + fabsf(w_o[3]));
+        ratio = __all(fabsf(wsum) < __builtin_inff());
+      }
+      if (ratio) {
         // Every channel of the wave keeps its decay over the sub-block above
         // kMcRatioMin (and its w are finite: the product's zeros above the
         // diagonal would take a NaN or an infinity of row s into the rows
