@@ -163,38 +163,6 @@ __device__ __forceinline__ void st_row_at(T* __restrict__ p, uint32_t lo, int64_
   }
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
-  return x;
-}
-
-// Wave-wide sums of the M entries of v (M a power of two, M <= 64): a
-// transposing butterfly (each lane keeps half of its entries and trades the
-// other half with its partner, masks 32, 16, ...) until one entry is left,
-// then a plain butterfly over the remaining lane bits. Afterwards lane l
-// holds the sum of entry l / (64 / M) in v[0]. Fixed order.
-template <int MASK, int K, int M>
-__device__ __forceinline__ void wave_sums_step(float (&v)[M], int lane) {
-  if constexpr (K > 1) {
-    const bool hi = (lane & MASK) != 0;
-#pragma unroll
-    for (int j = 0; j < K / 2; ++j) {
-      const float lo_v = v[j], hi_v = v[j + K / 2];
-      v[j] = (hi ? hi_v : lo_v) + __shfl_xor(hi ? lo_v : hi_v, MASK, 64);
-    }
-    wave_sums_step<MASK / 2, K / 2, M>(v, lane);
-  } else {
-#pragma unroll
-    for (int m = MASK; m >= 1; m >>= 1) v[0] += __shfl_xor(v[0], m, 64);
-  }
-}
-template <int M>
-__device__ __forceinline__ void wave_sums(float (&v)[M], int lane) {
-  static_assert(M >= 1 && M <= 64 && (M & (M - 1)) == 0, "M must be a power of two <= 64");
-  wave_sums_step<32, M, M>(v, lane);
-}
-
 // Tagged words of the look-back: {value bits, tag} in one 64-bit atomic.
 __device__ __forceinline__ uint64_t ld_word(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1089,66 +1057,7 @@ constexpr int kGnCK = 32;  // rows per sub-chunk = checkpoint interval
 constexpr int kGnDT = 64;  // channels per workgroup
 constexpr int kGnW = 8;    // waves per workgroup
 
-template <int LG>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int m = LG / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
-}
-
-// Sums over aligned groups of LG lanes of the M entries of v, by a
-// transposing butterfly: at each step a lane keeps half of its entries and
-// trades the other half with its partner, so the M sums cost M-1 lane
-// exchanges instead of M*log2(LG). Afterwards lane l of a group holds the
-// sums of entries [l*M/LG, (l+1)*M/LG) in v[0 .. M/LG). Fixed order, so the
-// sums are run-to-run identical.
-template <int LG, int K, int M>
-__device__ __forceinline__ void tr_reduce_step(float (&v)[M], int lane) {
-  if constexpr (LG > 1) {
-    constexpr int m = LG / 2;
-    const bool hi = (lane & m) != 0;
-#pragma unroll
-    for (int j = 0; j < K / 2; ++j) {
-      const float lo_v = v[j], hi_v = v[j + K / 2];
-      v[j] = (hi ? hi_v : lo_v) + __shfl_xor(hi ? lo_v : hi_v, m, 64);
-    }
-    tr_reduce_step<m, K / 2, M>(v, lane);
-  }
-}
-template <int LG, int M>
-__device__ __forceinline__ void tr_reduce(float (&v)[M], int lane) {
-  tr_reduce_step<LG, M, M>(v, lane);
-}
-
 constexpr int kGnThreads = 64 * kGnW;
-constexpr int kGnE = kGnCK * kGnDT / kGnThreads;  // tile elements per thread
-
-// This thread's kGnE elements (element k = e*kGnThreads + tid is row k/kGnDT,
-// channel k%kGnDT) of a [kGnCK][kGnDT] tile of one [batch,T,D] stream
-// starting at row t0, channel dbase. Rows past T and channels past D read a
-// clamped in-bounds element, which the caller replaces. The dtype switch is
-// outside the element loop, so the loads issue back to back.
-__device__ __forceinline__ void gn_ld_tile(const ScanArgs& a, const void* p, int dt, int b, int64_t t0,
-                                           int64_t dbase, float (&v)[kGnE]) {
-  int64_t idx[kGnE];
-#pragma unroll
-  for (int e = 0; e < kGnE; ++e) {
-    const int k = e * kGnThreads + (int)threadIdx.x;
-    const int64_t t = t0 + k / kGnDT, d = dbase + k % kGnDT;
-    idx[e] = ((int64_t)b * a.T + (t < a.T ? t : a.T - 1)) * a.D + (d < a.D ? d : a.D - 1);
-  }
-  if (dt == NAJU_DTYPE_F32) {
-#pragma unroll
-    for (int e = 0; e < kGnE; ++e) v[e] = ((const float*)p)[idx[e]];
-  } else if (dt == NAJU_DTYPE_BF16) {
-#pragma unroll
-    for (int e = 0; e < kGnE; ++e) v[e] = (float)((const bf16_t*)p)[idx[e]];
-  } else {
-#pragma unroll
-    for (int e = 0; e < kGnE; ++e) v[e] = (float)((const f16_t*)p)[idx[e]];
-  }
-}
-
 // The same for a [kGnCK][NP] tile of B or C ([batch,T,N]); entries past T or
 // N are replaced by the caller.
 template <int NP, int EB, int NT = kGnThreads>
@@ -1173,36 +1082,6 @@ __device__ __forceinline__ void gn_ld_bc(const ScanArgs& a, const void* p, int b
   }
 }
 
-// Writes a prefetched B/C tile into LDS, zero where the row is past T or the
-// state index past N.
-template <int NP, int EB>
-__device__ __forceinline__ void gn_st_bc(const ScanArgs& a, int64_t t0, const float (&vb)[EB],
-                                         const float (&vc)[EB], float (&sB)[kGnCK][NP], float (&sC)[kGnCK][NP]) {
-#pragma unroll
-  for (int e = 0; e < EB; ++e) {
-    const int k = e * kGnThreads + (int)threadIdx.x;
-    if (k < kGnCK * NP) {
-      const int r = k / NP, n = k % NP;
-      const bool ok = t0 + r < a.T && n < a.N;
-      sB[r][n] = ok ? vb[e] : 0.f;
-      sC[r][n] = ok ? vc[e] : 0.f;
-    }
-  }
-}
-
-// Writes one prefetched [kGnCK][NP] tile of B or C into LDS (zeros outside).
-template <int NP, int EB>
-__device__ __forceinline__ void gn_st_one(const ScanArgs& a, int64_t t0, const float (&v)[EB], float (&sv)[kGnCK][NP]) {
-#pragma unroll
-  for (int e = 0; e < EB; ++e) {
-    const int k = e * kGnThreads + (int)threadIdx.x;
-    if (k < kGnCK * NP) {
-      const int r = k / NP, n = k % NP;
-      sv[r][n] = (t0 + r < a.T && n < a.N) ? v[e] : 0.f;
-    }
-  }
-}
-
 // Time segments. With nseg > 1 the sub-chunks of T are split into nseg
 // segments of seg_sc sub-chunks, each scanned by its own workgroup per
 // channel tile (grid = tiles * segments, tile = blockIdx % tiles). The state
@@ -1223,8 +1102,8 @@ constexpr int kGmRP = kGnCK + 4;  // LDS row pitch of the transposed tiles
 
 template <int NP>
 __global__ __launch_bounds__(64 * kGnW) void gn_bwd_map_kernel(const ScanArgs a, int x_dt, int g_dt) {
-  constexpr int LG = NP < 64 ? NP : 64;
-  constexpr int S = NP / LG;
+  static_assert(NP <= 8, "a channel's states are lanes of one wave");
+  constexpr int LG = NP;  // lanes per channel
   constexpr int G = 64 / LG;
   constexpr int NPASS = kGnDT / G;
   constexpr int PPW = (NPASS + kGnW - 1) / kGnW;
@@ -1256,12 +1135,11 @@ __global__ __launch_bounds__(64 * kGnW) void gn_bwd_map_kernel(const ScanArgs a,
   const bool bn_act = tid < BCT;
   const int bnc = bn < N ? bn : N - 1;
 
-  float gc[PPW][S], Ac[PPW];
+  float gc[PPW], Ac[PPW];
 #pragma unroll
   for (int q = 0; q < PPW; ++q) {
     Ac[q] = 1.f;
-#pragma unroll
-    for (int s2 = 0; s2 < S; ++s2) gc[q][s2] = 0.f;
+    gc[q] = 0.f;
   }
   float vf[4], vg[4], vc[EB];
   // this thread's rows 4*wv .. 4*wv+3 of channel lane (f, dy) and rows
@@ -1345,15 +1223,12 @@ __global__ __launch_bounds__(64 * kGnW) void gn_bwd_map_kernel(const ScanArgs a,
         // blocks they would need hundreds of registers
         __builtin_amdgcn_sched_barrier(0);
         const float4 f4 = *(const float4*)&s_x[0][c][r4], y4 = *(const float4*)&s_x[1][c][r4];
-        float4 C4[S];
-#pragma unroll
-        for (int s2 = 0; s2 < S; ++s2) C4[s2] = *(const float4*)&s_c[nl + 64 * s2][r4];
+        const float4 C4 = *(const float4*)&s_c[nl][r4];
 #pragma unroll
         for (int e = 3; e >= 0; --e) {
           const float f = (&f4.x)[e], gy = (&y4.x)[e];
           Ac[q] *= f;
-#pragma unroll
-          for (int s2 = 0; s2 < S; ++s2) gc[q][s2] = f * fmaf(gy, (&C4[s2].x)[e], gc[q][s2]);
+          gc[q] = f * fmaf(gy, (&C4.x)[e], gc[q]);
         }
       }
     }
@@ -1365,11 +1240,7 @@ __global__ __launch_bounds__(64 * kGnW) void gn_bwd_map_kernel(const ScanArgs a,
     const int64_t d = dbase + (int64_t)pass * G + gl;
     if (d >= D) continue;
     const int64_t o = ((int64_t)b * a.nseg + seg) * D + d;
-#pragma unroll
-    for (int s2 = 0; s2 < S; ++s2) {
-      const int n = nl + 64 * s2;
-      if (n < N) a.segZ[o * N + n] = gc[q][s2];
-    }
+    if (nl < N) a.segZ[o * N + nl] = gc[q];
     if (nl == 0) a.segF[o] = Ac[q];
   }
 }
@@ -1609,8 +1480,8 @@ __global__ __launch_bounds__(256) void gn_seg_carry_kernel(const ScanArgs a, int
 //
 // N <= 8. One workgroup per (batch row, tile of DT channels, time segment), W
 // waves.
-// Lanes run over the state index n (LG = min(NP, 64) lanes per channel, S
-// states per lane, G channels per wave instruction). A wave walks its
+// Lanes run over the state index n (LG = NP lanes per channel, G channels
+// per wave instruction). A wave walks its
 // channel passes one after another; per kGnCK-row sub-chunk (the checkpoint
 // interval, walked from the last to the first) and per 16-row half (the later
 // half first) it
@@ -1631,23 +1502,11 @@ constexpr int kGnH = 16;          // rows per adjoint half
 constexpr int kGnRG = 8;          // rows per reduction group
 constexpr int kGnRP = kGnCK + 4;  // LDS row pitch (floats) of the transposed tiles
 
-// Value of lane l ^ m for the lanes with bit log2(m) clear.
-template <int m>
-__device__ __forceinline__ float from_upper(float x) {
-  if constexpr (m == 32) {
-    return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
-  } else if constexpr (m == 16) {
-    return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
-  } else {
-    return __shfl_xor(x, m, 64);
-  }
-}
-
 template <int NP, int DT, int W>
 __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_dt, int g_dt, int du_dt,
                                                            int dg_dt) {
-  constexpr int LG = NP < 64 ? NP : 64;
-  constexpr int S = NP / LG;
+  static_assert(NP <= 8, "a channel's states are lanes of one wave");
+  constexpr int LG = NP;  // lanes per channel
   constexpr int G = 64 / LG;
   constexpr int TH = 64 * W;         // threads
   constexpr int RGS = TH / DT;        // staging row groups of 4 rows
@@ -1694,15 +1553,11 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
   // adjoint carry f_{t+1} x̄_{t+1} per channel pass: zero past the end of T,
   // else the carry entering the segment from the future
   const float* gin = a.nseg > 1 ? a.seg0 + ((int64_t)b * a.nseg + seg) * D * N : nullptr;
-  float gc[PPW][S];
+  float gc[PPW];
 #pragma unroll
   for (int q = 0; q < PPW; ++q) {
     const int64_t d = dbase + (int64_t)(wv + q * W) * G + gl;
-#pragma unroll
-    for (int s2 = 0; s2 < S; ++s2) {
-      const int n = nl + 64 * s2;
-      gc[q][s2] = (gin && n < N && d < D) ? gin[d * N + n] : 0.f;
-    }
+    gc[q] = (gin && nl < N && d < D) ? gin[d * N + nl] : 0.f;
   }
   float dDacc = 0.f;
 
@@ -1769,19 +1624,15 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
         }
       }
     }
-    float x0[PPW][S];
+    float x0[PPW];
     {
       const float* ck = a.ckpt + (((int64_t)b * KC + sc) * D + dbase) * N;
 #pragma unroll
       for (int q = 0; q < PPW; ++q) {
         const int cq = (wv + q * W) * G;  // first channel of the pass (uniform)
         const float* ckq = ck + (int64_t)cq * N;
-#pragma unroll
-        for (int s2 = 0; s2 < S; ++s2) {
-          const int n = nl + 64 * s2;
-          const bool ok = n < N && dbase + cq + gl < D && wv + q * W < NPASS;
-          x0[q][s2] = ok ? *(const float*)((const char*)ckq + ((uint32_t)gl * (uint32_t)N + (uint32_t)n) * 4u) : 0.f;
-        }
+        const bool ok = nl < N && dbase + cq + gl < D && wv + q * W < NPASS;
+        x0[q] = ok ? *(const float*)((const char*)ckq + ((uint32_t)gl * (uint32_t)N + (uint32_t)nl) * 4u) : 0.f;
       }
     }
     __syncthreads();  // the previous sub-chunk's LDS tiles are stored
@@ -1820,11 +1671,9 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
     for (int h = 1; h >= 0; --h) {
       const int hr0 = h * kGnH;
       if (hr0 >= rows) continue;  // uniform over the workgroup
-      float accB[kGnH][S], accC[kGnH][S];
+      float accB[kGnH], accC[kGnH];
 #pragma unroll
-      for (int r = 0; r < kGnH; ++r)
-#pragma unroll
-        for (int s2 = 0; s2 < S; ++s2) accB[r][s2] = accC[r][s2] = 0.f;
+      for (int r = 0; r < kGnH; ++r) accB[r] = accC[r] = 0.f;
 #pragma unroll
       for (int q = 0; q < PPW; ++q) {
         const int pass = wv + q * W;
@@ -1835,28 +1684,22 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
         // (their live registers would add up)
         __builtin_amdgcn_sched_barrier(0);
         const int c = pass * G + gl;
-        float xs[S];
-#pragma unroll
-        for (int s2 = 0; s2 < S; ++s2) xs[s2] = x0[q][s2];
+        float xs = x0[q];
         // forward states: rows [0, hr0) unstored, then the half's rows
         for (int r4 = 0; r4 < hr0; r4 += 4) {
           const float4 f4 = *(const float4*)&s_x[0][c][r4];
           const float4 u4 = *(const float4*)&s_x[2][c][r4];
-          float4 B4[S];
-#pragma unroll
-          for (int s2 = 0; s2 < S; ++s2) B4[s2] = *(const float4*)&s_bc[0][nl + 64 * s2][r4];
+          const float4 B4 = *(const float4*)&s_bc[0][nl][r4];
           const float* pf = &f4.x;
           const float* pu = &u4.x;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float iu = pu[e];
-#pragma unroll
-            for (int s2 = 0; s2 < S; ++s2) xs[s2] = fmaf(iu, (&B4[s2].x)[e], xs[s2] * pf[e]);
+            xs = fmaf(iu, (&B4.x)[e], xs * pf[e]);
           }
         }
-        float xin[S], hist[kGnH][S];
-#pragma unroll
-        for (int s2 = 0; s2 < S; ++s2) xin[s2] = xs[s2];
+        const float xin = xs;
+        float hist[kGnH];
         // The LDS reads of each 4-row block are issued right before the
         // block (scheduling fences): hoisting all of a half's reads would
         // hold 16 rows of operands in registers at once.
@@ -1866,19 +1709,14 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
           const int r = hr0 + r4;
           const float4 f4 = *(const float4*)&s_x[0][c][r];
           const float4 u4 = *(const float4*)&s_x[2][c][r];
-          float4 B4[S];
-#pragma unroll
-          for (int s2 = 0; s2 < S; ++s2) B4[s2] = *(const float4*)&s_bc[0][nl + 64 * s2][r];
+          const float4 B4 = *(const float4*)&s_bc[0][nl][r];
           const float* pf = &f4.x;
           const float* pu = &u4.x;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float iu = pu[e];
-#pragma unroll
-            for (int s2 = 0; s2 < S; ++s2) {
-              xs[s2] = fmaf(iu, (&B4[s2].x)[e], xs[s2] * pf[e]);
-              hist[r4 + e][s2] = xs[s2];
-            }
+            xs = fmaf(iu, (&B4.x)[e], xs * pf[e]);
+            hist[r4 + e] = xs;
           }
         }
         // adjoint over the half's rows, last first, reduced every kGnRG rows.
@@ -1895,12 +1733,8 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
             const int r = hr0 + lr;
             const float4 f4 = *(const float4*)&s_x[0][c][r];
             const float4 u4 = *(const float4*)&s_x[2][c][r], y4 = *(const float4*)&s_x[3][c][r];
-            float4 B4[S], C4[S];
-#pragma unroll
-            for (int s2 = 0; s2 < S; ++s2) {
-              B4[s2] = *(const float4*)&s_bc[0][nl + 64 * s2][r];
-              C4[s2] = *(const float4*)&s_bc[1][nl + 64 * s2][r];
-            }
+            const float4 B4 = *(const float4*)&s_bc[0][nl][r];
+            const float4 C4 = *(const float4*)&s_bc[1][nl][r];
             const float* pf = &f4.x;
             const float* pu = &u4.x;
             const float* py = &y4.x;
@@ -1909,19 +1743,16 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
               const int j = r4 + e;  // row within the group
               const float iu = pu[e], gy = py[e];
               float tf = 0.f, tw = 0.f;
-#pragma unroll
-              for (int s2 = 0; s2 < S; ++s2) {
-                const float xprev = lr + e > 0 ? hist[lr + e - 1][s2] : xin[s2];
-                const float xb = fmaf(gy, (&C4[s2].x)[e], gc[q][s2]);
-                tf = fmaf(xb, xprev, tf);
-                tw = fmaf(xb, (&B4[s2].x)[e], tw);
-                accB[lr + e][s2] = fmaf(xb, iu, accB[lr + e][s2]);
-                accC[lr + e][s2] = fmaf(gy, hist[lr + e][s2], accC[lr + e][s2]);
-                // keep the updates here: sunk to the end of the pass they
-                // would hold every row's operands in registers
-                asm volatile("" : "+v"(accB[lr + e][s2]), "+v"(accC[lr + e][s2]));
-                gc[q][s2] = pf[e] * xb;
-              }
+              const float xprev = lr + e > 0 ? hist[lr + e - 1] : xin;
+              const float xb = fmaf(gy, (&C4.x)[e], gc[q]);
+              tf = fmaf(xb, xprev, tf);
+              tw = fmaf(xb, (&B4.x)[e], tw);
+              accB[lr + e] = fmaf(xb, iu, accB[lr + e]);
+              accC[lr + e] = fmaf(gy, hist[lr + e], accC[lr + e]);
+              // keep the updates here: sunk to the end of the pass they
+              // would hold every row's operands in registers
+              asm volatile("" : "+v"(accB[lr + e]), "+v"(accC[lr + e]));
+              gc[q] = pf[e] * xb;
               v[j] = tf;
               v[kGnRG + j] = tw;
             }
@@ -1931,13 +1762,12 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
           // lanes holding dfl sums (the lower half of the group) take the
           // matching dws sums from the upper half and write the outputs over
           // the consumed f, i, u of their rows
-          constexpr int KF = 2 * kGnRG >= LG ? 2 * kGnRG / LG : 1;
-          constexpr int SPREAD = 2 * kGnRG >= LG ? 1 : LG / (2 * kGnRG);
+          constexpr int KF = 2 * kGnRG / LG;
           float vw[KF];
 #pragma unroll
-          for (int j = 0; j < KF; ++j) vw[j] = from_upper<LG / 2>(v[j]);
-          if (nl < LG / 2 && nl % SPREAD == 0) {
-            const int e0 = (nl / SPREAD) * KF;
+          for (int j = 0; j < KF; ++j) vw[j] = __shfl_xor(v[j], LG / 2, 64);
+          if (nl < LG / 2) {
+            const int e0 = nl * KF;
 #pragma unroll
             for (int j = 0; j < KF; ++j) {
               const int r = hr0 + grp * kGnRG + e0 + j;
@@ -1953,26 +1783,21 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
       // wave, then over the waves in wave order
       if constexpr (G > 1) {
 #pragma unroll
-        for (int r = 0; r < kGnH; ++r)
+        for (int r = 0; r < kGnH; ++r) {
 #pragma unroll
-          for (int s2 = 0; s2 < S; ++s2) {
-#pragma unroll
-            for (int m = 32; m >= LG; m >>= 1) {
-              accB[r][s2] += __shfl_xor(accB[r][s2], m, 64);
-              accC[r][s2] += __shfl_xor(accC[r][s2], m, 64);
-            }
+          for (int m = 32; m >= LG; m >>= 1) {
+            accB[r] += __shfl_xor(accB[r], m, 64);
+            accC[r] += __shfl_xor(accC[r], m, 64);
           }
+        }
       }
       for (int w = 0; w < W; ++w) {
         if (wv == w && gl == 0) {
 #pragma unroll
-          for (int r = 0; r < kGnH; ++r)
-#pragma unroll
-            for (int s2 = 0; s2 < S; ++s2) {
-              const int n = nl + 64 * s2;
-              s_pB[hr0 + r][n] = (w == 0 ? 0.f : s_pB[hr0 + r][n]) + accB[r][s2];
-              s_pC[hr0 + r][n] = (w == 0 ? 0.f : s_pC[hr0 + r][n]) + accC[r][s2];
-            }
+          for (int r = 0; r < kGnH; ++r) {
+            s_pB[hr0 + r][nl] = (w == 0 ? 0.f : s_pB[hr0 + r][nl]) + accB[r];
+            s_pC[hr0 + r][nl] = (w == 0 ? 0.f : s_pC[hr0 + r][nl]) + accC[r];
+          }
         }
         __syncthreads();
       }
@@ -2026,11 +1851,7 @@ __global__ __launch_bounds__(64 * W) void gn_bwd_kernel(const ScanArgs a, int x_
     const int64_t d = dbase + (int64_t)pass * G + gl;
     if (d >= D) continue;
     if (a.dh0 && seg == 0) {
-#pragma unroll
-      for (int s2 = 0; s2 < S; ++s2) {
-        const int n = nl + 64 * s2;
-        if (n < N) a.dh0[((int64_t)b * D + d) * N + n] = gc[q][s2];
-      }
+      if (nl < N) a.dh0[((int64_t)b * D + d) * N + nl] = gc[q];
     }
   }
   // dD = sum dy * u over this segment's rows, in wave order
@@ -2220,13 +2041,9 @@ constexpr int kGnBwdDT = 32, kGnBwdW = 4;
 size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 int np_of(int64_t N);
-// The chunked matrix-core kernels serve 9 <= N <= 128 in the directions that
-// have them.
-constexpr bool kMcBwd = true;
-bool use_mc(int64_t N, bool bwd) { return mc_ok(N) && (!bwd || kMcBwd); }
 // Rows per checkpoint interval of the general-N forward: the chunked
 // backward reads the state entering every kMcQ-row sub-block.
-int64_t gn_ck_rows(int64_t N) { return use_mc(N, true) ? kMcQ : kGnCK; }
+int64_t gn_ck_rows(int64_t N) { return mc_ok(N) ? kMcQ : kGnCK; }
 // The checkpoint interval the flags ask for (NAJU_CKPT_ROWS; 0 = the
 // default: the backward's chunk at N = 1, gn_ck_rows at N > 1), or -1 when
 // the shape does not serve it: longer intervals than the default only on the
@@ -2295,7 +2112,7 @@ Layout make_layout(int64_t batch, int64_t T, int64_t D, int64_t N, int x_dt, int
   l.ck_rows = ck_rows;
   (void)x_dt;
   (void)g_dt;
-  const bool mc = use_mc(N, bwd);
+  const bool mc = mc_ok(N);
   if (N == 1) {
     l.V = n1_vec_width(bwd);
     l.CH = 64 * l.V;
@@ -2322,7 +2139,7 @@ Layout make_layout(int64_t batch, int64_t T, int64_t D, int64_t N, int x_dt, int
       l.seg_sc = mc_seg_sc(l.n_tiles, l.K, bwd, unit);
     } else {
       // forward (lanes over channels): about kGcTargetWaves waves; backward
-      // (8-wave workgroups over 64 channels): about kGnTargetWgs workgroups
+      // (4-wave workgroups over 32 channels): about kGnTargetWgs workgroups
       const int64_t per_seg = bwd ? l.n_tiles : batch * ((D + 63) / 64);
       const int64_t target = bwd ? kGnTargetWgs : kGcTargetWaves;
       int64_t want = (target + per_seg - 1) / per_seg;
@@ -2547,10 +2364,9 @@ ScanArgs mc_half_args(const ScanArgs& a, int h, int bc_dt) {
 // B / C (or dB / dC) with rows ld elements apart: ld = N always; another
 // ld only on the matrix-core path (9 <= N <= 64), a multiple of 4 with both
 // pointers aligned to four elements (the staging loads of the kernels).
-int check_bc_ld(const void* p, const void* q, int64_t N, int dt, int64_t ld, bool bwd) {
+int check_bc_ld(const void* p, const void* q, int64_t N, int dt, int64_t ld) {
   if (ld == N) return NAJU_OK;
   if (ld < N) return fail(NAJU_ERR_INVALID, "B / C row stride (%lld) must be >= N (%lld)", (long long)ld, (long long)N);
-  (void)bwd;
   if (!mc_ext_ok(N))
     return fail(NAJU_ERR_UNSUPPORTED, "a B / C row stride other than N is served at 9 <= N <= 64 only");
   // the kernels address a sub-block's rows with 32-bit offsets
@@ -2572,7 +2388,7 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
   g_err[0] = 0;
   int rc = check_common(batch, T, D, N, x_dtype, gate_dtype, bc_dtype);
   if (rc) return rc;
-  if ((rc = check_bc_ld(B, C, N, bc_dtype, ldbc, false))) return rc;
+  if ((rc = check_bc_ld(B, C, N, bc_dtype, ldbc))) return rc;
   if (flags & ~(NAJU_FLAG_OUT_F32 | NAJU_FLAG_DETERMINISTIC | NAJU_CKPT_MASK))
     return fail(NAJU_ERR_INVALID, "unknown flag bits 0x%x", flags);
   const int ck_rows = ckpt_rows(flags, N);
@@ -2634,7 +2450,7 @@ int scan_fwd_impl(const void* u, const void* f_logit, const void* i_logit, const
     a.segF = (float*)(ws + l.off_segF);
     a.segZ = (float*)(ws + l.off_segZ);
     a.seg0 = (float*)(ws + l.off_seg0);
-    if (use_mc(N, false)) {
+    if (mc_ok(N)) {
       // chunked matrix-core forward: segment maps, their carry, the scan
       a.n_dtiles = l.n_dtiles;
       a.n_tiles = l.n_tiles;
@@ -2814,8 +2630,8 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
   g_err[0] = 0;
   int rc = check_common(batch, T, D, N, x_dtype, gate_dtype, bc_dtype);
   if (rc) return rc;
-  if ((rc = check_bc_ld(B, C, N, bc_dtype, ldbc, true))) return rc;
-  if ((rc = check_bc_ld(dB, dC, N, (flags & NAJU_FLAG_OUT_F32) ? (int)NAJU_DTYPE_F32 : bc_dtype, lddbc, true)))
+  if ((rc = check_bc_ld(B, C, N, bc_dtype, ldbc))) return rc;
+  if ((rc = check_bc_ld(dB, dC, N, (flags & NAJU_FLAG_OUT_F32) ? (int)NAJU_DTYPE_F32 : bc_dtype, lddbc)))
     return rc;
   if (lddbc != N && batch * T > 0 && D == 0)
     return fail(NAJU_ERR_UNSUPPORTED, "strided dB / dC need D > 0");
@@ -2902,7 +2718,7 @@ static int scan_bwd_impl(const void* u, const void* f_logit, const void* i_logit
     a.segZ = (float*)(ws + l.off_segZ);
     a.seg0 = (float*)(ws + l.off_seg0);
     if ((int64_t)l.n_tiles * l.nseg > 0x7fffffff) return fail(NAJU_ERR_UNSUPPORTED, "problem too large");
-    if (use_mc(N, true)) {
+    if (mc_ok(N)) {
       // chunked matrix-core backward: adjoint segment maps, their carry, the
       // backward itself
       hipError_t e = hipSuccess;

@@ -1,4 +1,5 @@
-// naju_scan_map.hip -- time-segment maps of the chunked scan (9 <= N <= 64).
+// naju_scan_map.hip -- time-segment maps of the chunked scan (9 <= N <= 128,
+// above 64 in two launches over halves of the entries).
 //
 // When T is split into segments, the state (adjoint carry) entering a segment
 // comes from composing the maps of the segments before (after) it, s -> F s + Z
@@ -20,7 +21,7 @@
 // never leave the lane's registers. The decays of a lane's 8 rows are a
 // product chain, those of the four lane groups two lane swaps. B (or C) of the
 // block goes through the wave's own LDS as [n][row], whose 8 rows per lane are
-// the A operand in one 16-byte read (bf16). There is no barrier in the walk;
+// the A operand in two 8-byte reads (bf16; 16-byte ones for float32). There is no barrier in the walk;
 // the W waves of a workgroup take consecutive runs of a segment's rows and add
 // their maps in wave order at the end.
 //
@@ -83,9 +84,9 @@ struct RawV {
 
 // Whether the A operand goes through LDS as bf16 (exact) or as float32.
 template <typename TB>
-constexpr bool kMap16 =  __is_same(TB, bf16_t);
-// LDS row pitch of the [n][row] tile: 16-byte reads of 16 rows n without bank
-// conflicts (80 bytes for bf16, 144 for float32).
+constexpr bool kMap16 = __is_same(TB, bf16_t);
+// LDS row pitch of the [n][row] tile in elements: 88 bytes for bf16 (so rows
+// are 8-byte aligned), 144 for float32.
 template <typename TB>
 constexpr int kMapPitch = kMap16<TB> ? 44 : 36;
 // Bytes of a wave's LDS: the tile, or its part of the final sum.

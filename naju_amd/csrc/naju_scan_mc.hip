@@ -617,19 +617,20 @@ __global__ __launch_bounds__(64 * kMcW) __attribute__((amdgpu_waves_per_eu(NP <=
 //   ghat'  = Pall ghat + C^T (Pf dy)   (the carry leaving the first row)
 // (naju/cuda/naju_cuda.cu:104-141 restated per sub-block.) C X, B ghat,
 // G = C B^T, the dB / dC products and the carry update run on the matrix
-// cores; the per-channel sums over pairs of rows on the vector units.
+// cores, and so do the per-channel sums over pairs of rows where the decays can
+// be taken as ratios; as exact products they run on the vector units.
 //
-// Layouts. "D layout" as in the forward: lane (j, g) value r holds row
-// 4r + g of channel j, or state entry n = 16m + 4g + r of channel j. "T
-// layout": lane (j, g) value r holds entry n = 16m + j of channel 4g + r.
-// ghat is kept in both (the two carry updates read the same operands with
-// the A and B roles swapped); X is read from the checkpoint in both.
+// Layout ("D layout", as in the forward): lane (j, g) value r holds row 4r + g
+// of channel j, or state entry n = 16m + 4g + r of channel j.
 //
 // LDS per workgroup (NP = 64): B / C staged as Bn, C [t][n] and Bt, Ct
-// [n][p(t)] (19 KB), per wave the gate tiles f, w, dy, i [channel][row]
-// (5 KB) and a pool of seven [16][TP] tiles (8.75 KB) that holds G, G^T,
-// gathers, the rectangle sums' partials, (dy Pf) / (w Pe), H / H^T and
-// finally the wave's dB / dC, which the workgroup adds in wave order.
+// [n][p(t)] (19 KB as float32, 21 KB as two buffers of bf16), per wave the gate
+// tiles f, dy, w, i [channel][row] (5 KB; later the outputs, and dy Pf and
+// w Pe) and a pool of nine [16][TP] tiles (11 KB) that holds G, a and b or the
+// gathers of the exact path, the rectangle sums' partials, H / H^T and X and
+// ghat as [channel][n]. At NP = 64 the workgroup's dB / dC tiles are products
+// over the operands of all waves; below, each wave's dB / dC go through its
+// pool and are added in wave order.
 // With bf16 B and C every product that takes them is on the 16-bit matrix
 // cores, so their tiles hold bf16 as loaded: no conversion, half the LDS bytes
 // (the LM layer's backward, 8 x 2048 x 1536: 435 -> 419 us).

@@ -155,10 +155,9 @@ def test_full_size_c2_n64_channel_slice(gpu):
 
 @pytest.mark.parametrize("N,D", [(48, 1536), (32, 3072), (16, 6144)])
 def test_wide_grid_forward_general_n(gpu, N, D):
-    """Batch x channel grids that fill the GPU on their own take the forward
-    with four states per lane and no time segments (the C5 layer is one:
-    8 x 1536 channels at N = 64): ragged T, N below its power-of-two tile,
-    h0, and the mixer's dtypes (bf16 u, B, C; f32 gates)."""
+    """Wide batch x channel grids (the LM's layer is one: 8 x 1536 channels at
+    N = 64): ragged T, N below its tile of entries, h0, and the mixer's dtypes
+    (bf16 u, B, C; f32 gates)."""
     ins = rand_inputs(8, 70, D, N, seed=N, dtype=torch.bfloat16, gate_dtype=torch.float32,
                       bc_dtype=torch.bfloat16, h0_std=0.3)
     y, g = run_hip(ins, gpu)
