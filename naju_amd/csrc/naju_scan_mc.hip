@@ -855,9 +855,9 @@ __device__ __forceinline__ void store_row4(void* p, uint32_t o, const float (*tl
 // half's own, and what is summed over the entries, dws and
 // f xbar . x_{t-1}, the first
 // (HALF = 1) leaves in a.half and the second (HALF = 2) adds before it forms
-// du, dfl and dil. (bf16 4 x 2048 x 1024, N = 128: 161 + 172 us for the two
+// du, dfl and dil. (bf16 4 x 2048 x 1024, N = 128: 148 + 159 us for the two
 // halves against 744 us on the vector units; the forward, whole at NP = 128,
-// 104 us against 522.)
+// 107 us against 522.)
 template <int NP, int HALF, typename TU, typename TG, typename TB>
 __global__ __launch_bounds__(64 * kMcWB) void mc_bwd_kernel(const ScanArgs a, int du_dt, int dg_dt) {
   constexpr int MT = NP / 16;
