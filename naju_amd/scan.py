@@ -143,7 +143,8 @@ def workspace_status(device=None):
     1 or 2 after a failed call (then cleared, so the workspace is usable
     again). Synchronises the stream. Where calls captured on this stream have
     a workspace of their own, its word is read too."""
-    dev = torch.device("cuda", torch.cuda.current_device() if device is None else torch.device(device).index)
+    index = None if device is None else torch.device(device).index
+    dev = torch.device("cuda", torch.cuda.current_device() if index is None else index)
     stream = _stream_handle(dev)
     key = (dev.index, stream)
     found = 0

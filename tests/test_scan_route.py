@@ -54,3 +54,12 @@ def test_sizes_are_those_of_the_library():
     for k in range(300):  # bounded
         scan._sizes(1, k + 1, 8, 1, (0, 0, 0), 0)
     assert len(scan._SIZES) <= 256
+
+
+@pytest.mark.parametrize("device", [None, "cuda", torch.device("cuda"), "cuda:1", 1])
+def test_workspace_status_takes_a_device_without_an_index(monkeypatch, device):
+    """"cuda" names the current device, as it does everywhere in torch."""
+    asked = []
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(scan, "_stream_handle", lambda dev: asked.append(dev.index) or 0)
+    assert scan.workspace_status(device) == 0 and asked == [1]
